@@ -2,7 +2,7 @@
 // megakernel, so both paths run the same arithmetic in the same order.
 //
 // Split-KV: the attended positions 0..L-1 are cut into chunks of
-// attn_chunk_len(L, parts, kAttnGrain) positions (a multiple of 16, at most
+// decode_chunk_len(L) positions (a multiple of 16, at most
 // kAttnMaxChunks chunks). A chunk of one KV group is one workgroup's work,
 // computed in one of two ways fixed by the chunk length, so every path
 // agrees:
@@ -140,7 +140,7 @@ __device__ __forceinline__ void attn_block_valu(K4 k4, Q4 q4, V v, PB &pb, int b
 }
 
 // A chunk of at most one block (chunk length up to kAttnPass: contexts of
-// up to 64 * parts positions) is computed on the vector ALUs, one query head
+// up to 1,024 positions) is computed on the vector ALUs, one query head
 // per wave (attn_block_valu); longer chunks go through the MFMA tiles below.
 // With one block per chunk the tiles' cross-wave merge would be all
 // overhead, and a wave per head keeps the K/V reads to one block.

@@ -15,17 +15,15 @@ constexpr int kMaxGroup = 16;          // query heads per KV head
 
 // Split-KV attention geometry (qd_attention.hpp): chunks are whole grains
 // of positions, at most kAttnMaxChunks per head; a partial record is (m, l,
-// acc[64]). The batch-1 decode paths cut chunks in grains of one attention
-// tile (kAttnGrain, 16 positions); the batched kernel in passes of 64 (16
-// positions per wave of its four-wave unit).
+// acc[64]). The batched kernel cuts chunks in passes of 64 (16 positions per
+// wave of its four-wave unit); the batch-1 decode paths by decode_chunk_len.
 constexpr int kAttnPass = 64;
 constexpr int kAttnGrain = 16;
 constexpr int kAttnMaxChunks = 16;
 constexpr int kPartStride = kHeadDim + 2;
 
 // Chunks of a context of `length` positions split `parts` ways (parts <=
-// kAttnMaxChunks; the decode engine uses its resident plan's attention CUs
-// per KV group, so that each takes one chunk): whole grains per chunk.
+// kAttnMaxChunks): whole grains per chunk.
 __host__ __device__ inline int attn_chunk_len(int length, int parts = kAttnMaxChunks, int grain = kAttnPass) {
   const int grains = (length + grain - 1) / grain;
   const int per_chunk = (grains + parts - 1) / parts;
@@ -35,6 +33,36 @@ __host__ __device__ inline int attn_chunk_len(int length, int parts = kAttnMaxCh
 __host__ __device__ inline int attn_chunks(int length, int parts = kAttnMaxChunks, int grain = kAttnPass) {
   const int cl = attn_chunk_len(length, parts, grain);
   return (length + cl - 1) / cl;
+}
+
+// Chunk length of the batch-1 decode paths, a function of the context alone so
+// that the stream kernels and any resident launch split it alike: one block
+// of kAttnPass positions (a chunk of one block costs the same however few
+// positions it holds) until kAttnMaxChunks blocks are full; then, in the form
+// whose waves take 32-position tiles, at least two blocks (at context 1040, 9
+// chunks of 128: 449 us per token against 456 for 14 chunks of 80), and the
+// fewest grains of 16 that kAttnMaxChunks chunks need beyond 2,048 positions.
+__host__ __device__ inline int decode_chunk_len(int length) {
+  const int cl = attn_chunk_len(length, kAttnMaxChunks, kAttnGrain);
+  return cl <= kAttnPass ? kAttnPass : cl < 2 * kAttnPass ? 2 * kAttnPass : cl;
+}
+
+__host__ __device__ inline int decode_chunks(int length) {
+  const int cl = decode_chunk_len(length);
+  return (length + cl - 1) / cl;
+}
+
+// The most chunks any context first .. last has (the count drops where the
+// chunk length grows, and grows with the grains in between).
+inline int decode_chunks_most(int first, int last) {
+  int most = 1;
+  for (int length = first;;) {
+    const int chunks = decode_chunks(length);
+    if (chunks > most) most = chunks;
+    if (length >= last) return most;
+    length = (length / kAttnGrain + 1) * kAttnGrain;
+    if (length > last) length = last;
+  }
 }
 
 enum Mode : uint32_t { kModeStep = 0, kModeGenerate = 1 };

@@ -168,11 +168,6 @@ struct qd_engine {
   uint32_t *resident_error = nullptr;       // [1 + kXcds]
   uint32_t spin_limit = qd::kResidentSpinLimit;
   int roles_grid = 0;                       // 0: resident path unavailable
-  // Attention chunk geometry of both paths, attn_chunks(length, attn_parts, kAttnGrain):
-  // the resident plan's attention CUs per KV group at the engine's capacity
-  // (fixed at create, so the stream kernels split a context as the resident
-  // kernel does whether or not it runs), else kAttnMaxChunks.
-  int attn_parts = qd::kAttnMaxChunks;
   std::string resident_off_reason;
   // Prompt workspace (allocated on the first prefill): rows of the hidden
   // states, RMSNorm output, packed QKV, attention output and SwiGLU
@@ -338,7 +333,6 @@ struct qd_engine {
     a.k_cache = kv_slice(k_cache, seq, layer);
     a.v_cache = kv_slice(v_cache, seq, layer);
     a.part = part;
-    a.attn_parts = attn_parts;
     a.weights_dtype = wdtype;
     a.capacity = static_cast<int>(CAP);
     a.nq = static_cast<int>(NQ);
@@ -380,8 +374,8 @@ struct qd_engine {
   // The slot's qd_step launch sequence as an instantiated HIP graph,
   // captured on first use. Every kernel of it reads the position and the
   // token from the slot's device state and takes only fixed buffers and a
-  // fixed grid as arguments (the attention split is the engine's, fixed at
-  // creation), so one capture serves every later step of the slot. The
+  // fixed grid as arguments (the attention split follows from the position,
+  // within a grid of kAttnMaxChunks), so one capture serves every later step of the slot. The
   // graph holds kernel nodes only (no memset or copy nodes).
   hipGraphExec_t step_graph(uint32_t seq) {
     if (step_graphs.empty()) step_graphs.assign(B, nullptr);
@@ -409,7 +403,7 @@ struct qd_engine {
   double kernel_bytes(int kernel, double length) const {
     const double f = 4.0;
     const double mf = static_cast<double>(mat_elem());  // bytes per decoder-matrix element
-    const double chunks = qd::attn_chunks(static_cast<int>(length), attn_parts, qd::kAttnGrain);
+    const double chunks = qd::decode_chunks(static_cast<int>(length));
     switch (kernel) {
       case qd::kKEmbed: return 2 * H * f;
       case qd::kKQkvRope:
@@ -651,11 +645,11 @@ struct qd_engine {
     }
   }
 
-  // Role plan of a resident launch whose longest context is `reach`; false
-  // when the resident path is off or the plan does not fit the grid.
-  bool resident_plan(uint32_t reach, qd::RolePlan *plan) const {
-    return roles_grid > 0 &&
-           qd::plan_roles(roles_grid, int(H), int(I), int(NQ), int(NKV), int(reach), plan);
+  // Role plan of a resident launch of `tokens` tokens from position `start`;
+  // false when the resident path is off or the plan does not fit the grid.
+  bool resident_plan(uint32_t start, uint32_t tokens, qd::RolePlan *plan) const {
+    return roles_grid > 0 && qd::plan_roles(roles_grid, int(H), int(I), int(NQ), int(NKV), int(start) + 1,
+                                            int(start + tokens), plan);
   }
 
   // Launches the resident megakernel (stream ordered; no synchronisation)
@@ -702,14 +696,13 @@ struct qd_engine {
     for (int r = 0; r < qd::kRoleCount; ++r) ra.role_end[r] = plan.end[r];
     for (int r = 0; r < 3; ++r) ra.group_cus[r] = plan.group_cus[r];
     ra.xcd_place = plan.xcd_place;
-    ra.attn_parts = attn_parts;
     // The first token attends to the fewest positions and the last to the
     // most; a chunk never shrinks as the context grows.
     {
       const int first = static_cast<int>(positions[seq]) + 1;
       const int last = static_cast<int>(std::min<uint64_t>(uint64_t(positions[seq]) + max_tokens, CAP));
-      ra.attn_mode = qd::attn_chunk_len(first, attn_parts, qd::kAttnGrain) > qd::kAttnPass ? 1
-                     : qd::attn_chunk_len(last, attn_parts, qd::kAttnGrain) <= qd::kAttnPass ? 2
+      ra.attn_mode = qd::decode_chunk_len(first) > qd::kAttnPass ? 1
+                     : qd::decode_chunk_len(last) <= qd::kAttnPass ? 2
                                                                                              : 0;
     }
     ra.weights_dtype = wdtype;
@@ -967,19 +960,13 @@ qd_status qd_engine_create(const qd_config *config, qd_engine **out) {
     // force the give-up path with it).
     const int cus = qd::device_cu_count(c.device);
     e->cu_count = std::max(cus, 0);
-    {
-      qd::RolePlan cap_plan{};
-      if (cus >= 64 && cus <= qd::kMaxRoleGrid &&
-          qd::plan_roles(cus, int(e->H), int(e->I), int(e->NQ), int(e->NKV), int(e->CAP), &cap_plan))
-        e->attn_parts = std::min(qd::kAttnMaxChunks, cap_plan.group_cus[1]);
-    }
     const char *env = std::getenv("QD_RESIDENT");
     qd::RolePlan plan{};
     if (env && std::strcmp(env, "0") == 0) {
       e->resident_off_reason = "QD_RESIDENT=0";
     } else if (cus < 64 || cus > qd::kMaxRoleGrid || qd::roles_max_grid(c.device, e->wdtype) < cus) {
       e->resident_off_reason = "device cannot co-schedule one role workgroup per CU";
-    } else if (!qd::plan_roles(cus, int(e->H), int(e->I), int(e->NQ), int(e->NKV), 1, &plan)) {
+    } else if (!qd::plan_roles(cus, int(e->H), int(e->I), int(e->NQ), int(e->NKV), 1, 1, &plan)) {
       e->resident_off_reason = "no role plan for this model shape";
     } else {
       e->roles_grid = cus;
@@ -1453,7 +1440,7 @@ qd_status step_common(qd_engine *e, uint32_t seq, uint32_t token, float *logits_
     // (one cooperative launch instead of the stream kernels' ~150); the graph
     // replays the stream kernels. Both compute the same values bit for bit.
     qd::RolePlan plan{};
-    bool resident = !graph && e->resident_fits(1) && e->resident_plan(e->positions[seq] + 1, &plan);
+    bool resident = !graph && e->resident_fits(1) && e->resident_plan(e->positions[seq], 1, &plan);
     if (resident) {
       const hipError_t err = e->launch_resident(plan, seq, token, 1, UINT32_MAX, dev_logits, 0, nullptr);
       if (err != hipSuccess) {
@@ -1814,7 +1801,7 @@ qd_status qd_generate_resident(qd_engine *e, uint32_t seq, uint32_t first_token,
       use_hist = 1;
     }
     qd::RolePlan plan{};
-    bool resident = e->resident_fits(max_tokens) && e->resident_plan(e->positions[seq] + max_tokens, &plan);
+    bool resident = e->resident_fits(max_tokens) && e->resident_plan(e->positions[seq], max_tokens, &plan);
     check(hipEventRecord(e->ev_begin, e->stream), "hipEventRecord");
     if (resident) {
       // The kernel takes its start from the launch arguments and writes the
@@ -1941,7 +1928,7 @@ void profiled_resident_launch(qd_engine *e, uint32_t seq, uint32_t first_token, 
     fail(QD_ERROR_INVALID_ARGUMENT, "profiling %u tokens overflows capacity", tokens);
   if (!e->resident_fits(tokens)) fail(QD_ERROR_INVALID_ARGUMENT, "too many tokens for one resident launch");
   qd::RolePlan plan{};
-  if (!e->resident_plan(e->positions[seq] + tokens, &plan))
+  if (!e->resident_plan(e->positions[seq], tokens, &plan))
     fail(QD_ERROR_NOT_SUPPORTED, "no resident role plan reaches context %zu", size_t(e->positions[seq]) + tokens);
   e->set_device();
   const size_t trace_elems =

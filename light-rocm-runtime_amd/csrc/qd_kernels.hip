@@ -111,15 +111,15 @@ constexpr int kAttnThreads = kAttnSlots * kWave;
 __global__ __launch_bounds__(kAttnThreads) void attn_partial_kernel(
     const float *__restrict__ q, const float *__restrict__ k_cache,
     const float *__restrict__ v_cache, const SeqState *__restrict__ st,
-    int nq, int nkv, float *__restrict__ part, int capacity, int parts) {
+    int nq, int nkv, float *__restrict__ part, int capacity) {
   __shared__ float ps[kAttnSlots * kAttnPsFloats];
   __shared__ float stage_lds[kAttnStageFloats];
   if (st->stopped || st->position >= static_cast<uint32_t>(capacity)) return;
   const int position = static_cast<int>(st->position);
   const int length = position + 1;
   const int chunk = blockIdx.x;
-  if (chunk >= attn_chunks(length, parts, kAttnGrain)) return;
-  const int chunk_len = attn_chunk_len(length, parts, kAttnGrain);
+  if (chunk >= decode_chunks(length)) return;
+  const int chunk_len = decode_chunk_len(length);
   const int g = blockIdx.y;
   const int group = nq / nkv;
   const int kv_dim = nkv * kHeadDim;
@@ -183,9 +183,9 @@ __global__ __launch_bounds__(kAttnThreads) void attn_partial_kernel(
 // Merges each head's partials into attn[h*64 + d].
 __global__ __launch_bounds__(kHeadDim) void attn_combine_kernel(
     const float *__restrict__ part, const SeqState *__restrict__ st, int nq,
-    float *__restrict__ attn, int capacity, int parts) {
+    float *__restrict__ attn, int capacity) {
   if (st->stopped || st->position >= static_cast<uint32_t>(capacity)) return;
-  const int chunks = attn_chunks(static_cast<int>(st->position) + 1, parts, kAttnGrain);
+  const int chunks = decode_chunks(static_cast<int>(st->position) + 1);
   const int h = blockIdx.x;
   const int d = threadIdx.x;
   attn[h * kHeadDim + d] = attn_merge(
@@ -576,15 +576,14 @@ hipError_t launch_layer_as(hipStream_t s, const LayerLaunch &p, Marker *m) {
   }
   {
     Scope scope(m, kKAttnPartial);
-    if (p.attn_parts < 1 || p.attn_parts > kAttnMaxChunks) return hipErrorInvalidValue;
     if (p.nq / p.nkv > kAttnMaxGroup) return hipErrorInvalidValue;
-    attn_partial_kernel<<<dim3(p.attn_parts, p.nkv), kAttnThreads, 0, s>>>(
-        p.q, p.k_cache, p.v_cache, p.st, p.nq, p.nkv, p.part, p.capacity, p.attn_parts);
+    attn_partial_kernel<<<dim3(kAttnMaxChunks, p.nkv), kAttnThreads, 0, s>>>(
+        p.q, p.k_cache, p.v_cache, p.st, p.nq, p.nkv, p.part, p.capacity);
   }
   {
     Scope scope(m, kKAttnCombine);
     attn_combine_kernel<<<p.nq, kHeadDim, 0, s>>>(p.part, p.st, p.nq, p.attn,
-                                                  p.capacity, p.attn_parts);
+                                                  p.capacity);
   }
   {
     Scope scope(m, kKOproj);

@@ -83,7 +83,6 @@ struct ResidentArgs {
   uint32_t spin_limit;          // polls before a wait gives up
   int role_end[kRoleCount];     // RolePlan::end
   int group_cus[3];             // RolePlan::group_cus
-  int attn_parts;               // chunk geometry: attn_chunks(length, attn_parts, kAttnGrain)
   int xcd_place;                // RolePlan::xcd_place
   int weights_dtype;            // kWeights*: storage of the layers' matrices (picks the instance)
   int attn_mode;                // attention role instance: 0 both chunk forms, 1 every chunk
@@ -115,10 +114,10 @@ constexpr size_t roles_slot_floats(int hidden, int inter, int heads, int kv_head
 
 int device_cu_count(int device);
 
-// Role split of `grid` CUs for generations reaching context `max_length`;
-// false when the model shape has no role kernel or the grid cannot hold one
+// Role split of `grid` CUs for a launch whose tokens attend over min_length ..
+// max_length positions; false when the model shape has no role kernel or the grid cannot hold one
 // layer's weights on chip.
-bool plan_roles(int grid, int hidden, int inter, int heads, int kv_heads, int max_length,
+bool plan_roles(int grid, int hidden, int inter, int heads, int kv_heads, int min_length, int max_length,
                 RolePlan *plan);
 hipError_t launch_roles(hipStream_t s, const ResidentArgs &args, int grid);
 // Prepares a resident launch in one dispatch: error[0 .. kXcds] zero, the

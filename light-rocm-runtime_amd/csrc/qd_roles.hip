@@ -1460,7 +1460,7 @@ struct Roles {
     float vw2[kAttnTile];
     auto pre_lds = [&](int l, int position) {
       const int length = position + 1;
-      const int chunks = attn_chunks(length, a.attn_parts, kAttnGrain), cl = attn_chunk_len(length, a.attn_parts, kAttnGrain);
+      const int chunks = decode_chunks(length), cl = decode_chunk_len(length);
       if (rr >= chunks || position >= a.capacity) return;
       const int begin = rr * cl, end = min(length, begin + cl);
       attn_dma(l, g, begin, min(end, begin + kAttnCap), ar);
@@ -1480,7 +1480,7 @@ struct Roles {
     auto pre_regs = [](int) {};
     loop(kRoleAttn, false, [&](uint32_t t, int l, int position) {
       const int length = position + 1;
-      const int chunks = attn_chunks(length, a.attn_parts, kAttnGrain), cl = attn_chunk_len(length, a.attn_parts, kAttnGrain);
+      const int chunks = decode_chunks(length), cl = decode_chunk_len(length);
       const Slots in = s_qkv(l, t), out = s_part(l, t);
       // Record (h, c) is kRoleRecStride floats at (h * kAttnMaxChunks + c) *
       // kRoleRecStride: whole float4s.
@@ -1492,7 +1492,7 @@ struct Roles {
         // 1025) and regrows later, which leaves older records in slots beyond
         // it.
         const Slots next = s_part(l, t + 1);
-        const int chunks_next = attn_chunks(length + 1, a.attn_parts, kAttnGrain);
+        const int chunks_next = decode_chunks(length + 1);
         for (int c = rr; c < chunks_next; c += na) {
           for (int e = threadIdx.x; e < GROUP * kRec4; e += kT)
             next.clear4(((g * GROUP + e / kRec4) * kAttnMaxChunks + c) * kRec4 + e % kRec4);
@@ -1682,7 +1682,7 @@ struct Roles {
     OutMap om;  // rows [2 u0, 2 u0 + 2 n), staged from element 2 u0 rounded down to 4
     om.take(2 * u0, 2 * ro.n, (2 * u0) & ~3, threadIdx.x, 0);
     loop(kRoleO, false, [&](uint32_t t, int l, int position) {
-      const int C = attn_chunks(position + 1, a.attn_parts, kAttnGrain);
+      const int C = decode_chunks(position + 1);
       const Slots out = s_h1(l, t, g);
       if (om.q >= 0) clear_quad(s_h1(l, t + 1, g), om);
       // Group 0 adds the residual: rows [2 u0, 2 u0 + 2 n) of the layer
@@ -2073,10 +2073,10 @@ __global__ __launch_bounds__(256) void roles_prepare_kernel(uint32_t *error, uin
 
 }  // namespace
 
-bool plan_roles(int grid, int hidden, int inter, int heads, int kv_heads, int max_length,
-                RolePlan *plan) {
+bool plan_roles(int grid, int hidden, int inter, int heads, int kv_heads, int min_length,
+                int max_length, RolePlan *plan) {
   if (hidden != 896 || inter != 4864 || heads != 14 || kv_heads != 2) return false;
-  if (grid > kMaxRoleGrid || max_length < 1) return false;
+  if (grid > kMaxRoleGrid || min_length < 1 || max_length < min_length) return false;
   // Units per role, their capacity per CU (LDS + register slots) and bytes.
   // O: each of the KV groups covers every row pair (Roles::run_o).
   const int units[4] = {Qwen::QkvUnits, kv_heads * Qwen::OUnits, inter, hidden};
@@ -2097,13 +2097,11 @@ bool plan_roles(int grid, int hidden, int inter, int heads, int kv_heads, int ma
   };
   int floor_weights = 0;
   for (int r = 0; r < 4; ++r) floor_weights += need_of(r);
-  // One attention CU per (KV head, chunk) unit of the longest context, or
-  // as many as the weight roles leave (an attention CU then takes several
-  // units, the later ones staged after its query arrives). A long context
-  // gets a chunk per window of kAttnCap positions (up to kAttnMaxChunks),
-  // so each chunk's tiles run as one round on the CU's waves.
-  const int chunks = std::max(attn_chunks(max_length),
-                              std::min(kAttnMaxChunks, (max_length + kAttnCap - 1) / kAttnCap));
+  // One attention CU per (KV head, chunk) of the launch's contexts, or as
+  // many as the weight roles leave (an attention CU then takes several chunks,
+  // the later ones staged after its query arrives: at context 512 with 12
+  // chunks on 9 CUs a token took 494 us instead of 411).
+  const int chunks = decode_chunks_most(min_length, max_length);
   int n_attn = std::min(kv_heads * chunks, grid - floor_weights);
   n_attn -= n_attn % kv_heads;  // whole KV groups
   if (n_attn < kv_heads) return false;
