@@ -31,16 +31,6 @@
 #include "qd_resident.hpp"
 #include "qd_rng.hpp"
 
-// Stream-K workgroups per CU of the prompt's QKV and down GEMMs (0:
-// split-K). The O GEMM keeps split-K 2: its 224 workgroups already give
-// every CU one equal share.
-#ifndef QD_PREFILL_SK_QKV
-#define QD_PREFILL_SK_QKV 1
-#endif
-#ifndef QD_PREFILL_SK_DOWN
-#define QD_PREFILL_SK_DOWN 2
-#endif
-
 namespace {
 
 constexpr uint32_t kAbiVersion = 4;
@@ -169,29 +159,14 @@ struct qd_engine {
   uint32_t spin_limit = qd::kResidentSpinLimit;
   int roles_grid = 0;                       // 0: resident path unavailable
   std::string resident_off_reason;
-  // Prompt workspace (allocated on the first prefill): rows of the hidden
-  // states, RMSNorm output, packed QKV, attention output and SwiGLU
-  // activation, plus the chunk's token ids.
-  static constexpr size_t kPrefillRows = 512;
-  float *pf_h = nullptr, *pf_xn = nullptr, *pf_qkv = nullptr, *pf_attn = nullptr,
-        *pf_act = nullptr, *pf_split = nullptr;
-  // Split-K factors of the narrow GEMMs (QKV, O, down) so they fill the CUs,
-  // used when stream-K is off (sk_target 0).
-  static constexpr int kSplitQkv = 2, kSplitO = 2, kSplitDown = 4;
-  // Stream-K for the QKV and down GEMMs: up to per_cu workgroups per CU
-  // (QD_PREFILL_SK_QKV / QD_PREFILL_SK_DOWN), each taking at least
-  // kSkMinSlices K slices of 32, so every CU gets an equal share of the
-  // (tile, slice) work; pf_split_floats is the partial workspace that any
-  // prompt chunk of up to kPrefillRows rows needs.
-  static constexpr int kSkMinSlices = 8;
-  int cu_count = 0;
-  size_t pf_split_floats = 0;
-  int sk_groups(int m, int n, int k, int per_cu) const {
-    if (per_cu <= 0 || cu_count <= 0) return 0;
-    const long long total = static_cast<long long>((m + 63) / 64) * ((n + 63) / 64) * (k / 32);
-    return static_cast<int>(
-        std::min<long long>(static_cast<long long>(per_cu) * cu_count, std::max<long long>(1, total / kSkMinSlices)));
-  }
+  // Prompt workspace (allocated on the first prefill) for chunks of up to
+  // kPrefillRows positions: rows of the hidden states and the rotated queries,
+  // the GEMMs' left operands in parts (RMSNorm output, attention output,
+  // SwiGLU activation), their partial products and the chunk's token ids.
+  // Longer chunks read each weight for more rows (the 128-row GEMM tiles).
+  static constexpr size_t kPrefillRows = 2048;
+  float *pf_h = nullptr, *pf_q = nullptr, *pf_split = nullptr;
+  qd::PartRows pf_xn{}, pf_attn{}, pf_act{};
   uint32_t *pf_tokens = nullptr;
   // Batched-step workspace (allocated on the first batched step): rows of
   // up to kBatchRows sequences, attention and split-K partials, arrival
@@ -527,12 +502,12 @@ struct qd_engine {
 
   // Kernels of the prompt path, for per-kernel event timing.
   enum PrefillKernel : int {
-    kPEmbed = 0, kPNorm, kPGemmQkv, kPAttn, kPGemmO, kPGemmGateUp, kPGemmDown,
+    kPEmbed = 0, kPGemmQkv, kPAttn, kPGemmO, kPGemmGateUp, kPGemmDown,
     kPTail, kPrefillKernels
   };
   static const char *prefill_kernel_name(int id) {
     static const char *const names[kPrefillKernels] = {
-        "embed_rows_kernel",    "rmsnorm_rows_kernel",      "gemm_nt_kernel:qkv+rope",
+        "embed_norm_kernel",    "gemm_nt_kernel:qkv+rope",
         "attention_prefill_kernel", "gemm_nt_kernel:o+norm",
         "gemm_nt_kernel:gateup+swiglu", "gemm_nt_kernel:down+norm",
         "lmhead_kernel+argmax"};
@@ -544,16 +519,16 @@ struct qd_engine {
   // that accumulate read and write C.
   std::pair<double, double> prefill_cost(int kernel, double n, double pos0) const {
     const double f = 4.0;
+    const double mf = static_cast<double>(mat_elem());
     switch (kernel) {
-      case kPEmbed: return {2 * n * H * f, 0};
-      case kPNorm: return {(2 * n * H + H) * f, 0};
-      case kPGemmQkv: return {(QKV * H + QKV + n * (H + QKV + 2 * QD + 4 * KVD)) * f, 2 * n * QKV * H};
+      case kPEmbed: return {(3 * n * H + H) * f, 0};
+      case kPGemmQkv: return {QKV * H * mf + (QKV + n * (H + QKV + 2 * QD + 4 * KVD)) * f, 2 * n * QKV * H};
       case kPAttn:
         return {(2 * (pos0 + n) * KVD + 2 * n * QD) * f,
                 4 * NQ * qd::kHeadDim * (n * pos0 + n * (n + 1) / 2)};
-      case kPGemmO: return {(H * QD + H + n * (QD + 3 * H)) * f, 2 * n * H * QD};
-      case kPGemmGateUp: return {(2 * I * H + n * (H + I)) * f, 4 * n * I * H};
-      case kPGemmDown: return {(H * I + H + n * (I + 3 * H)) * f, 2 * n * H * I};
+      case kPGemmO: return {H * QD * mf + (H + n * (QD + 3 * H)) * f, 2 * n * H * QD};
+      case kPGemmGateUp: return {2 * I * H * mf + n * (H + I) * f, 4 * n * I * H};
+      case kPGemmDown: return {H * I * mf + (H + n * (I + 3 * H)) * f, 2 * n * H * I};
       case kPTail: return {(V * H + H + V) * f, 2 * V * H};
     }
     return {0, 0};
@@ -566,81 +541,59 @@ struct qd_engine {
   void prefill_chunk(uint32_t seq, const uint32_t *tokens, int n, int pos0, qd::Marker *m = nullptr) {
     if (!pf_h) {
       pf_h = alloc<float>(kPrefillRows * H);
-      pf_xn = alloc<float>(kPrefillRows * H);
-      pf_qkv = alloc<float>(kPrefillRows * QKV);
-      pf_attn = alloc<float>(kPrefillRows * QD);
-      pf_act = alloc<float>(kPrefillRows * I);
+      pf_q = alloc<float>(kPrefillRows * QD);
+      auto parts = [&](size_t width) {
+        return qd::PartRows{alloc<uint16_t>(3 * kPrefillRows * width), kPrefillRows * width};
+      };
+      pf_xn = parts(H);
+      pf_attn = parts(QD);
+      pf_act = parts(I);
       pf_tokens = alloc<uint32_t>(kPrefillRows);
-      pf_split_floats = kPrefillRows * std::max({kSplitQkv * QKV, kSplitO * H, kSplitDown * H});
-      const int shapes[2][3] = {{int(QKV), int(H), QD_PREFILL_SK_QKV}, {int(H), int(I), QD_PREFILL_SK_DOWN}};
+      size_t split = 0;
       for (int rows = 1; rows <= int(kPrefillRows); ++rows)
-        for (const auto &sh : shapes) {
-          const int g = sk_groups(rows, sh[0], sh[1], sh[2]);
-          if (g > 0)
-            pf_split_floats = std::max(pf_split_floats, size_t(qd::gemm_streamk_slots(rows, sh[0], sh[1], g)) *
-                                                            size_t(rows) * size_t(sh[0]));
-        }
-      pf_split = alloc<float>(pf_split_floats);
+        for (const auto &[cols, k] : {std::pair<size_t, size_t>{QKV, H}, {H, QD}, {H, I}})
+          split = std::max(split, size_t(qd::gemm_splits(rows, int(cols), int(k))) * size_t(rows) * cols);
+      pf_split = alloc<float>(split);
     }
     check(hipMemcpyAsync(pf_tokens, tokens, size_t(n) * 4, hipMemcpyHostToDevice, stream), "H2D");
     const int h = int(H), in = int(I), qkv = int(QKV), qd = int(QD);
-    const int nq = int(NQ), nkv = int(NKV);
     auto span = [&](int id, const char *what, auto &&launch) {
       if (m) m->before(id);
       check(launch(), what);
       if (m) m->after(id);
     };
-    span(kPEmbed, "embed rows",
-         [&] { return qd::launch_embed_rows(stream, embed, pf_tokens, n, h, pf_h); });
+    // Partials of one projection, then the row kernel that finishes its rows.
+    auto project = [&](const qd::PartRows &a, const float *w, int cols, int k, auto &&finish) {
+      const int splits = qd::gemm_splits(n, cols, k);
+      const hipError_t err = qd::launch_gemm_partials(stream, wdtype, a, n, w, cols, k, pf_split, splits);
+      return err != hipSuccess ? err : finish(splits);
+    };
+    span(kPEmbed, "embed rows + norm", [&] {
+      return qd::launch_embed_norm(stream, embed, pf_tokens, n, layers[0].attn_norm, cfg.rms_eps, pf_h, pf_xn);
+    });
     for (size_t l = 0; l < L; ++l) {
       const qd::LayerPtrs &w = layers[l];
       float *kc = kv_slice(k_cache, seq, l), *vc = kv_slice(v_cache, seq, l);
-      // The attention norm of layer 0 runs on its own; every other norm and
-      // the RoPE run in the reduction of the split-K GEMM before them.
-      if (l == 0)
-        span(kPNorm, "norm",
-             [&] { return qd::launch_rmsnorm_rows(stream, pf_h, w.attn_norm, cfg.rms_eps, n, pf_xn); });
       span(kPGemmQkv, "qkv gemm + rope", [&] {
-        qd::RowEpilogue rope;
-        rope.kind = qd::kRowRope;
-        rope.pos0 = pos0;
-        rope.nq = nq;
-        rope.nkv = nkv;
-        rope.rope_cos = rope_cos;
-        rope.rope_sin = rope_sin;
-        rope.k_cache = kc;
-        rope.v_cache = vc;
-        return qd::launch_gemm_nt(stream, pf_xn, h, w.wqkv, h, pf_qkv, qkv, n, qkv, h, qd::kGemmBias,
-                                  w.bqkv, kSplitQkv, pf_split, &rope, sk_groups(n, qkv, h, QD_PREFILL_SK_QKV),
-                                  pf_split_floats);
+        return project(pf_xn, w.wqkv, qkv, h, [&](int splits) {
+          return qd::launch_qkv_rope(stream, pf_split, splits, n, w.bqkv, pos0, rope_cos, rope_sin, pf_q, kc, vc);
+        });
       });
       span(kPAttn, "attention", [&] {
-        return qd::launch_attention_prefill(stream, pf_qkv, n, pos0, nq, nkv, kc, vc, pf_attn);
+        return qd::launch_attention_prefill(stream, pf_q, n, pos0, int(NQ), int(NKV), kc, vc, pf_attn);
       });
       span(kPGemmO, "o gemm + norm", [&] {
-        qd::RowEpilogue norm;
-        norm.kind = qd::kRowNorm;
-        norm.gain = w.mlp_norm;
-        norm.eps = cfg.rms_eps;
-        norm.y = pf_xn;
-        return qd::launch_gemm_nt(stream, pf_attn, qd, w.wo, qd, pf_h, h, n, h, qd,
-                                  qd::kGemmAccumulate, nullptr, kSplitO, pf_split, &norm);
+        return project(pf_attn, w.wo, h, qd, [&](int splits) {
+          return qd::launch_residual_norm(stream, pf_split, splits, n, pf_h, w.mlp_norm, cfg.rms_eps, pf_xn);
+        });
       });
-      span(kPGemmGateUp, "gate/up gemm + swiglu", [&] {
-        return qd::launch_gemm_swiglu(stream, pf_xn, h, w.wg, w.wu, h, pf_act, in, n, in, h);
-      });
-      span(kPGemmDown, "down gemm", [&] {
-        qd::RowEpilogue norm;
-        if (l + 1 < L) {
-          norm.kind = qd::kRowNorm;
-          norm.gain = layers[l + 1].attn_norm;
-          norm.eps = cfg.rms_eps;
-          norm.y = pf_xn;
-        }
-        return qd::launch_gemm_nt(stream, pf_act, in, w.wd, in, pf_h, h, n, h, in,
-                                  qd::kGemmAccumulate, nullptr, kSplitDown, pf_split,
-                                  l + 1 < L ? &norm : nullptr, sk_groups(n, h, in, QD_PREFILL_SK_DOWN),
-                                  pf_split_floats);
+      span(kPGemmGateUp, "gate/up gemm + swiglu",
+           [&] { return qd::launch_gemm_swiglu(stream, wdtype, pf_xn, n, w.wg, w.wu, in, h, pf_act); });
+      span(kPGemmDown, "down gemm + norm", [&] {
+        return project(pf_act, w.wd, h, in, [&](int splits) {
+          return qd::launch_residual_norm(stream, pf_split, splits, n, pf_h,
+                                          l + 1 < L ? layers[l + 1].attn_norm : nullptr, cfg.rms_eps, pf_xn);
+        });
       });
     }
   }
@@ -959,7 +912,6 @@ qd_status qd_engine_create(const qd_config *config, qd_engine **out) {
     // lowers the polls a hand-off wait makes before it gives up (tests
     // force the give-up path with it).
     const int cus = qd::device_cu_count(c.device);
-    e->cu_count = std::max(cus, 0);
     const char *env = std::getenv("QD_RESIDENT");
     qd::RolePlan plan{};
     if (env && std::strcmp(env, "0") == 0) {
@@ -1575,24 +1527,6 @@ void check_prefill(qd_engine *e, uint32_t seq, const uint32_t *tokens, uint32_t 
 // on the last position, which advances the slot to pos0 + n. m (nullable)
 // times every launch.
 void run_prefill(qd_engine *e, uint32_t seq, const uint32_t *tokens, uint32_t n, EventMarker *m) {
-  if (e->narrow()) {
-    // BF16 or FP16 decoder weights: the prompt runs position by position through the
-    // stream-ordered step kernels (the prompt GEMMs read FP32 matrices),
-    // writing every position's K/V row; then the tail on the last position.
-    for (uint32_t i = 0; i < n; ++i) {
-      check(qd::launch_set_state(e->stream, e->states + seq, e->positions[seq], tokens[i]), "state launch");
-      check(qd::launch_embed(e->stream, e->embed, e->states + seq, e->hidden + size_t(seq) * e->H,
-                             static_cast<int>(e->H), static_cast<int>(e->V)),
-            "embed launch");
-      for (size_t l = 0; l < e->L; ++l) check(qd::launch_layer(e->stream, e->layer_args(seq, l)), "layer launch");
-      if (i + 1 < n) e->positions[seq] += 1;
-    }
-    e->push_state(seq, tokens[n - 1], qd::kModeStep, UINT32_MAX, 0);
-    check(qd::launch_tail(e->stream, e->tail_args(seq, e->logits + seq * e->V, 0, nullptr), nullptr),
-          "tail launch");
-    e->positions[seq] += 1;
-    return;
-  }
   for (uint32_t done = 0; done < n;) {
     const uint32_t rows = std::min<uint32_t>(n - done, uint32_t(qd_engine::kPrefillRows));
     if (m) {
