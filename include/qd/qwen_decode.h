@@ -78,8 +78,8 @@ typedef struct qd_config {
                            * exactly and computes in FP32 in the FP32 order, so
                            * such an engine equals an FP32 engine loaded with the
                            * rounded weights bit for bit. It runs the resident
-                         * kernel and the prompt GEMMs; it has no batched step
-                         * (QD_ERROR_NOT_SUPPORTED). */
+                           * kernel and the prompt GEMMs; it has no batched step
+                           * (QD_ERROR_NOT_SUPPORTED). */
 } qd_config;
 
 /* Storage types of qd_config.decoder_dtype. */

@@ -162,10 +162,11 @@ struct qd_engine {
   // Prompt workspace (allocated on the first prefill) for chunks of up to
   // kPrefillRows positions: rows of the hidden states and the rotated queries,
   // the GEMMs' left operands in parts (RMSNorm output, attention output,
-  // SwiGLU activation), their partial products and the chunk's token ids.
+  // SwiGLU activation), their partial products, the attention's partial
+  // records and the chunk's token ids.
   // Longer chunks read each weight for more rows (the 128-row GEMM tiles).
   static constexpr size_t kPrefillRows = 2048;
-  float *pf_h = nullptr, *pf_q = nullptr, *pf_split = nullptr;
+  float *pf_h = nullptr, *pf_q = nullptr, *pf_split = nullptr, *pf_rec = nullptr;
   qd::PartRows pf_xn{}, pf_attn{}, pf_act{};
   uint32_t *pf_tokens = nullptr;
   // Batched-step workspace (allocated on the first batched step): rows of
@@ -554,6 +555,7 @@ struct qd_engine {
         for (const auto &[cols, k] : {std::pair<size_t, size_t>{QKV, H}, {H, QD}, {H, I}})
           split = std::max(split, size_t(qd::gemm_splits(rows, int(cols), int(k))) * size_t(rows) * cols);
       pf_split = alloc<float>(split);
+      pf_rec = alloc<float>(size_t(qd::kAttnRecRows) * qd::kAttnRecFloats);
     }
     check(hipMemcpyAsync(pf_tokens, tokens, size_t(n) * 4, hipMemcpyHostToDevice, stream), "H2D");
     const int h = int(H), in = int(I), qkv = int(QKV), qd = int(QD);
@@ -580,7 +582,7 @@ struct qd_engine {
         });
       });
       span(kPAttn, "attention", [&] {
-        return qd::launch_attention_prefill(stream, pf_q, n, pos0, int(NQ), int(NKV), kc, vc, pf_attn);
+        return qd::launch_attention_prefill(stream, pf_q, n, pos0, kc, vc, pf_rec, pf_attn);
       });
       span(kPGemmO, "o gemm + norm", [&] {
         return project(pf_attn, w.wo, h, qd, [&](int splits) {

@@ -42,6 +42,25 @@ __device__ __forceinline__ uint32_t pack_bf16(float x, float y) {
 __device__ __forceinline__ float bf16_lo(uint32_t p) { return __uint_as_float(p << 16); }
 __device__ __forceinline__ float bf16_hi(uint32_t p) { return __uint_as_float(p & 0xFFFF0000u); }
 
+// Two floats' three parts, packed (any value: an infinity or one that rounds
+// to it leaves NaN in the later parts).
+__device__ __forceinline__ void split_pair(float x, float y, uint32_t &h, uint32_t &m, uint32_t &l) {
+  h = pack_bf16(x, y);
+  const float r0 = x - bf16_lo(h), r1 = y - bf16_hi(h);
+  m = pack_bf16(r0, r1);
+  l = pack_bf16(r0 - bf16_lo(m), r1 - bf16_hi(m));
+}
+
+// Eight floats as three matrix operands.
+__device__ __forceinline__ void split_eight(const float (&x)[8], bf8v (&out)[3]) {
+  uint32_t h[4], m[4], l[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) split_pair(x[2 * i], x[2 * i + 1], h[i], m[i], l[i]);
+  out[0] = __builtin_bit_cast(bf8v, u4v{h[0], h[1], h[2], h[3]});
+  out[1] = __builtin_bit_cast(bf8v, u4v{m[0], m[1], m[2], m[3]});
+  out[2] = __builtin_bit_cast(bf8v, u4v{l[0], l[1], l[2], l[3]});
+}
+
 // The three parts of an operand stored for the GEMM. Unlike the weights'
 // split in registers, a value that is not finite keeps itself as its first
 // part (the others 0), and one that would round to infinity is truncated, so
@@ -78,17 +97,7 @@ struct WeightOp<float> {
   __device__ static void operand(const u4v *row, int sw, int octet, bf8v (&out)[3]) {
     const f4v a = __builtin_bit_cast(f4v, row[(2 * octet) ^ sw]), b = __builtin_bit_cast(f4v, row[(2 * octet + 1) ^ sw]);
     const float x[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
-    u4v h, m, l;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      h[i] = pack_bf16(x[2 * i], x[2 * i + 1]);
-      const float r0 = x[2 * i] - bf16_lo(h[i]), r1 = x[2 * i + 1] - bf16_hi(h[i]);
-      m[i] = pack_bf16(r0, r1);
-      l[i] = pack_bf16(r0 - bf16_lo(m[i]), r1 - bf16_hi(m[i]));
-    }
-    out[0] = __builtin_bit_cast(bf8v, h);
-    out[1] = __builtin_bit_cast(bf8v, m);
-    out[2] = __builtin_bit_cast(bf8v, l);
+    split_eight(x, out);
   }
 };
 __device__ __forceinline__ int narrow_swizzle(int row) { return (row >> 2) & 3; }

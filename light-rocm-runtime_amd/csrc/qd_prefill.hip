@@ -16,6 +16,7 @@
 #include <algorithm>
 #include <cstdint>
 
+#include "qd_attention.hpp"
 #include "qd_device.hpp"
 #include "qd_device_math.hpp"
 #include "qd_gemm.hpp"
@@ -161,218 +162,314 @@ __global__ __launch_bounds__(kBlock) void qkv_rope_kernel(const float *__restric
 }
 
 // ---- causal GQA flash attention ---------------------------------------------------
-// One query block = (query head h, 16 prompt rows); a workgroup's four waves take
-// the key blocks (32 positions) round-robin, each keeping an online softmax
-// and an output accumulator for the 16 queries, merged in LDS at the end.
-// Per key block a wave computes S = Q . K^T (two 16 x 16 tiles over 64
-// dims) and O += P . V (four 16 x 16 tiles over 32 keys) with
-// v_mfma_f32_16x16x4f32, whose lane l supplies A[l % 16][l / 16] and
-// B[l / 16][l % 16] and holds D[(l / 16) * 4 + r][l % 16] in register r.
-constexpr int kQBlock = 16;
-constexpr int kKBlock = 32;
-constexpr int kKRow = kHeadDim + 4;   // LDS K row stride (conflict-free B reads)
-constexpr int kVRow = kHeadDim + 16;  // LDS V row stride
-constexpr int kPRow = kKBlock + 4;    // LDS P row stride
+// A workgroup takes 16 prompt rows of one KV group: a wave per query head of
+// the group, which share each block of 64 keys, split once into BF16 parts in
+// LDS. Both products run on v_mfma_f32_16x16x32_bf16 with the six products of
+// qd_gemm.hpp, the leading one in its own accumulator:
+//   S^T[key][row] = K . Q^T      A = K (lane: key l % 16, 8 dims from 8 (l / 16)),
+//                                B = Q (row l % 16, the same dims)
+//   O^T[dim][row] += V^T . P^T   A = V^T (dim l % 16), B = P (row l % 16)
+// D holds element (4 (l / 16) + r, l % 16) in register r of lane l, so a lane
+// keeps one prompt row throughout: its running maximum and rescale factor are
+// its own, only the block maximum crosses lanes, and the probabilities of two
+// 16-key tiles (keys 4 (l / 16) + r of each) are the B operand of the second
+// product as they stand; V^T is laid out in LDS in that key order.
+// What bounds it is the work per CU, not memory: a chunk of 512 rows is 64
+// (row block, KV group) pairs, so each pair's key blocks are dealt to
+// workgroups of `per_split` blocks whose partials a second kernel merges.
+// Scores are in base-2 units, the query scaled by log2(e) / 8 (one v_exp_f32
+// per exponential).
+constexpr int kQRows = 16, kKeyBlock = 64, kGroupHeads = 7;
+constexpr int kAttnWaves = kGroupHeads, kAttnThreads = kAttnWaves * kWave;
+constexpr int kRec = kHeadDim + 4;        // partial record: m, l, two pad words, acc[64]
+constexpr int kKv = 2 * kHeadDim;         // floats of a cache row
+constexpr int kRowBytes = 2 * kHeadDim;   // an LDS row: 64 BF16 parts
+constexpr int kKvPlane = kKeyBlock * kRowBytes;
+static_assert(kHeadDim == kKeyBlock, "K and V^T rows are both 64 parts");
 
-struct PrefillAttnLds {
-  float k[kWavesPerBlock][kKBlock][kKRow];
-  float v[kWavesPerBlock][kKBlock][kVRow];
-  float p[kWavesPerBlock][kQBlock][kPRow];
-  float ml[kWavesPerBlock][kQBlock][2];
-  float o[kWavesPerBlock][kQBlock][kHeadDim + 1];
+// 16-byte slot s of LDS row `row` (a key's dims or a dim's keys), so that the
+// rows of sixteen consecutive lanes at one slot fall on distinct banks.
+__device__ __forceinline__ int kv_slot(int row, int s) { return row * kRowBytes + 16 * (s ^ ((row >> 1) & 7)); }
+
+// Maximum / sum over the four lanes l % 16 + 16 i, in each of them.
+__device__ __forceinline__ void half_swap(float v, float &a, float &b) {
+  a = b = v;
+  asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1" : "+v"(a), "+v"(b));
+}
+__device__ __forceinline__ float quads_max(float v) {
+  float a, b;
+  half_swap(row_pair_max(v), a, b);
+  return fmaxf(a, b);
+}
+__device__ __forceinline__ float quads_sum(float v) {
+  float a, b;
+  half_swap(row_pair_sum(v), a, b);
+  return a + b;
+}
+
+__device__ __forceinline__ f4v mfma16(gemm::bf8v a, gemm::bf8v b, f4v c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+}
+struct AttnArgs {
+  const float *q;  // [rows][896]
+  const float *k_cache, *v_cache;
+  int rows, pos0, per_split, splits;
+  float *rec;  // [rows][14][splits][kRec], splits > 1
+  PartRows out;
 };
 
-// Query block qb of head h (the causal extent of a block grows with qb).
-__device__ __forceinline__ void attention_prefill_block(
-    PrefillAttnLds &sh, int qb, const float *__restrict__ q, int rows, int pos0, int nq, int nkv,
-    const float *__restrict__ k_cache, const float *__restrict__ v_cache, PartRows out) {
-  const int h = blockIdx.y;
-  const int r0 = qb * kQBlock;
-  const int g = h / (nq / nkv);
-  const int qd = nq * kHeadDim, kvd = nkv * kHeadDim;
-  const int w = wave_id();
-  const int lane = lane_id();
-  const int lr = lane & 15, lg = lane >> 4;
-  // Scores in base-2 units, s log2(e) / sqrt(64), so each softmax
-  // exponential is one v_exp_f32 (2^x): e^(s / 8 - m) = 2^(s log2(e) / 8 - m').
-  const float scale = 0.18033688011112042f;  // log2(e) / sqrt(64)
-  const int last_row = min(rows, r0 + kQBlock) - 1;
-  const int keys = pos0 + last_row + 1;  // causal extent of the block
-  const int kblocks = (keys + kKBlock - 1) / kKBlock;
-
-  // Query operand: lane supplies Q[row lr][dim 16 lg + s] at k-step s < 16
-  // (the K operand takes the same dims), so each lane's 16 dims are
-  // contiguous: four float4 reads.
-  float qa[kHeadDim / 4];
-  {
-    const int qrow = min(r0 + lr, rows - 1);
-    const float4 *q4 = reinterpret_cast<const float4 *>(q + static_cast<size_t>(qrow) * qd + h * kHeadDim + 16 * lg);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const float4 v = q4[j];
-      qa[4 * j] = v.x;
-      qa[4 * j + 1] = v.y;
-      qa[4 * j + 2] = v.z;
-      qa[4 * j + 3] = v.w;
-    }
-  }
-  // Running state of the lane's four query rows lg * 4 + r.
-  float m[4], l[4];
-  f4v o[4];
-#pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    m[r] = -INFINITY;
-    l[r] = 0.f;
-    o[r] = f4v{0.f, 0.f, 0.f, 0.f};
-  }
-  float (*ks)[kKRow] = sh.k[w];
-  float (*vs)[kVRow] = sh.v[w];
-  float (*ps)[kPRow] = sh.p[w];
-  // The block's K and V rows in registers: lane covers rows lane / 16 +
-  // 4 i, float4 column lane % 16 (zeros past the causal extent). The wave's
-  // next block is loaded while the current one is computed.
-  float4 kr[kKBlock / 4], vr[kKBlock / 4];
-  auto load_block = [&](int kb) {
-#pragma unroll
-    for (int i = 0; i < kKBlock / 4; ++i) {
-      const int j = kb * kKBlock + lg + 4 * i;
-      kr[i] = vr[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-      if (j < keys) {
-        kr[i] = *reinterpret_cast<const float4 *>(k_cache + static_cast<size_t>(j) * kvd + g * kHeadDim + 4 * lr);
-        vr[i] = *reinterpret_cast<const float4 *>(v_cache + static_cast<size_t>(j) * kvd + g * kHeadDim + 4 * lr);
-      }
-    }
-  };
-  if (w < kblocks) load_block(w);
-  for (int kb = w; kb < kblocks; kb += kWavesPerBlock) {
-    const int k0 = kb * kKBlock;
-    // Stage the block's rows in the wave's LDS, then start the next block's
-    // loads.
-#pragma unroll
-    for (int i = 0; i < kKBlock / 4; ++i) {
-      const int row = lg + 4 * i;
-      const float4 kv = kr[i], vv = vr[i];
-      *reinterpret_cast<float4 *>(&ks[row][4 * lr]) = kv;
-      *reinterpret_cast<float4 *>(&vs[row][4 * lr]) = vv;
-    }
-    if (kb + kWavesPerBlock < kblocks) load_block(kb + kWavesPerBlock);
-    // S tiles: keys k0 + 16 tt + lr. Every B operand is read from LDS before
-    // the first MFMA (one wait instead of one per step), and the two tiles'
-    // chains run interleaved; each chain keeps its order over st.
-    float kop[2][kHeadDim / 4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-#pragma unroll
-      for (int tt = 0; tt < 2; ++tt) {
-        const float4 v = *reinterpret_cast<const float4 *>(&ks[16 * tt + lr][16 * lg + 4 * j]);
-        kop[tt][4 * j] = v.x;
-        kop[tt][4 * j + 1] = v.y;
-        kop[tt][4 * j + 2] = v.z;
-        kop[tt][4 * j + 3] = v.w;
-      }
-    }
-    __builtin_amdgcn_sched_barrier(0);
-    f4v s[2] = {f4v{0.f, 0.f, 0.f, 0.f}, f4v{0.f, 0.f, 0.f, 0.f}};
-#pragma unroll
-    for (int st = 0; st < kHeadDim / 4; ++st) {
-      s[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(qa[st], kop[0][st], s[0], 0, 0, 0);
-      s[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(qa[st], kop[1][st], s[1], 0, 0, 0);
-    }
-    // Online softmax per query row (row = lg * 4 + r, spread over the 16
-    // lanes of DPP row lg and the two tiles).
-    float corr[4];
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int qpos = pos0 + min(r0 + lg * 4 + r, rows - 1);
-      float sv[2];
-#pragma unroll
-      for (int tt = 0; tt < 2; ++tt) {
-        const int key = k0 + 16 * tt + lr;
-        sv[tt] = key <= qpos ? s[tt][r] * scale : -INFINITY;
-      }
-      const float m_new = fmaxf(m[r], row16_max(fmaxf(sv[0], sv[1])));
-      float p0 = 0.f, p1 = 0.f;
-      corr[r] = 1.f;
-      if (m_new != -INFINITY) {
-        p0 = __builtin_amdgcn_exp2f(sv[0] - m_new);
-        p1 = __builtin_amdgcn_exp2f(sv[1] - m_new);
-        corr[r] = __builtin_amdgcn_exp2f(m[r] - m_new);
-      }
-      l[r] = fmaf(l[r], corr[r], row16_sum(p0 + p1));
-      m[r] = m_new;
-      ps[lg * 4 + r][lr] = p0;
-      ps[lg * 4 + r][16 + lr] = p1;
-    }
-#pragma unroll
-    for (int dt = 0; dt < 4; ++dt)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) o[dt][r] *= corr[r];
-    // O += P . V: A = P[row lr][key 4 st + lg], B = V[key 4 st + lg][dim 16 dt + lr],
-    // the operands read from LDS first as for S (this key order keeps the V
-    // reads of the four lane groups on different banks).
-    float pa[kKBlock / 4], vb[kKBlock / 4][4];
-#pragma unroll
-    for (int st = 0; st < kKBlock / 4; ++st) {
-      pa[st] = ps[lr][4 * st + lg];
-#pragma unroll
-      for (int dt = 0; dt < 4; ++dt) vb[st][dt] = vs[4 * st + lg][16 * dt + lr];
-    }
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int st = 0; st < kKBlock / 4; ++st)
-#pragma unroll
-      for (int dt = 0; dt < 4; ++dt)
-        o[dt] = __builtin_amdgcn_mfma_f32_16x16x4f32(pa[st], vb[st][dt], o[dt], 0, 0, 0);
-  }
-  // Merge the four waves' partials.
-#pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const int q = lg * 4 + r;
-    if (lr == 0) {
-      sh.ml[w][q][0] = m[r];
-      sh.ml[w][q][1] = l[r];
-    }
-#pragma unroll
-    for (int dt = 0; dt < 4; ++dt) sh.o[w][q][16 * dt + lr] = o[dt][r];
-  }
-  __syncthreads();
-  {
-    const int q = threadIdx.x >> 4;        // 16 queries
-    const int d0 = (threadIdx.x & 15) * 4;  // 4 dims each
-    const int row = r0 + q;
-    if (row < rows) {
-      float mx = -INFINITY;
-#pragma unroll
-      for (int v = 0; v < kWavesPerBlock; ++v) mx = fmaxf(mx, sh.ml[v][q][0]);
-      float den = 0.f, acc[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int v = 0; v < kWavesPerBlock; ++v) {
-        const float mv = sh.ml[v][q][0];
-        const float f = mv == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mv - mx);
-        den = fmaf(f, sh.ml[v][q][1], den);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) acc[e] = fmaf(f, sh.o[v][q][d0 + e], acc[e]);
-      }
-      put_parts(out.at(row, qd) + h * kHeadDim, out.plane, d0 / 4,
-                make_float4(acc[0] / den, acc[1] / den, acc[2] / den, acc[3] / den));
-    }
+// One head's attention of one prompt row over keys [k0, k1) in FP32, lane =
+// dim, a key at a time: for a wave whose split products were not finite (an
+// operand was not, or rounds to infinity in BF16).
+__device__ void attention_row_fp32(const AttnArgs &g, int row, int head, int kv, int k0, int k1, float &m, float &l,
+                                   float &acc) {
+  const int d = lane_id();
+  const float q = g.q[static_cast<size_t>(row) * kH + head * kHeadDim + d];
+  m = -INFINITY;
+  l = acc = 0.f;
+  for (int key = k0; key < k1; ++key) {
+    const size_t at = static_cast<size_t>(key) * kKv + kv * kHeadDim + d;
+    const float score = wave_sum(q * g.k_cache[at]) * kScoreScaleLog2;
+    if (score != -INFINITY) attn_fold(score, 1.f, g.v_cache[at], m, l, acc);
   }
 }
 
-// Workgroup (pair p, head h) takes query blocks p and nqb - 1 - p: the pair's
-// key blocks add up to about the same count for every p, so the launch is
-// one balanced round of workgroups instead of a long causal tail.
-__global__ __launch_bounds__(kBlock) void attention_prefill_kernel(
-    const float *__restrict__ q, int rows, int pos0, int nq, int nkv,
-    const float *__restrict__ k_cache, const float *__restrict__ v_cache, PartRows out) {
-  __shared__ __attribute__((aligned(16))) PrefillAttnLds sh;
-  const int nqb = (rows + kQBlock - 1) / kQBlock;
-  const int p = blockIdx.x;
-  attention_prefill_block(sh, p, q, rows, pos0, nq, nkv, k_cache, v_cache, out);
-  const int p2 = nqb - 1 - p;
-  if (p2 <= p) return;
-  __syncthreads();  // the first block's merge has read the LDS
-  attention_prefill_block(sh, p2, q, rows, pos0, nq, nkv, k_cache, v_cache, out);
+__global__ __launch_bounds__(kAttnThreads, 4) void attention_prefill_kernel(AttnArgs g) {
+  __shared__ __attribute__((aligned(16))) unsigned char kp[3 * kKvPlane], vp[3 * kKvPlane];
+  const int r0 = blockIdx.x * kQRows, kv = blockIdx.y, z = blockIdx.z;
+  const int keys = g.pos0 + min(g.rows, r0 + kQRows);  // causal extent of the row block
+  const int k_begin = z * g.per_split * kKeyBlock;
+  const int k_end = min(keys, k_begin + g.per_split * kKeyBlock);
+  if (k_begin >= k_end) return;
+  const int lane = lane_id(), head = kv * kGroupHeads + wave_id();
+  const int lr = lane & 15, lg = lane >> 4;
+  const int row = min(r0 + lr, g.rows - 1), pos = g.pos0 + row;
+
+  // The block's K and V^T items of this thread, loaded one block ahead: item
+  // i < 1024 is float4 i % 16 of key i / 16; 1024 + i is keys 4 (i / 64) .. + 3
+  // of dim i % 64. Keys past the causal extent are zeros.
+  constexpr int kItems = 2 * kKeyBlock * kHeadDim / 4, kPer = (kItems + kAttnThreads - 1) / kAttnThreads;
+  float4 item[kPer];
+  auto load = [&](int k0) {
+#pragma unroll
+    for (int n = 0; n < kPer; ++n) {
+      const int i = threadIdx.x + n * kAttnThreads;
+      item[n] = make_float4(0.f, 0.f, 0.f, 0.f);
+      if (i < kItems / 2) {
+        const int key = k0 + i / 16;
+        if (key < keys)
+          item[n] = reinterpret_cast<const float4 *>(g.k_cache + static_cast<size_t>(key) * kKv + kv * kHeadDim)[i % 16];
+      } else if (i < kItems) {
+        const int key = k0 + 4 * ((i - kItems / 2) / 64);
+        const float *v = g.v_cache + static_cast<size_t>(key) * kKv + kv * kHeadDim + i % 64;
+        if (key < keys) item[n].x = v[0];
+        if (key + 1 < keys) item[n].y = v[kKv];
+        if (key + 2 < keys) item[n].z = v[2 * kKv];
+        if (key + 3 < keys) item[n].w = v[3 * kKv];
+      }
+    }
+  };
+  auto stage = [&] {
+#pragma unroll
+    for (int n = 0; n < kPer; ++n) {
+      const int i = threadIdx.x + n * kAttnThreads;
+      if (i >= kItems) break;
+      uint2 p[3];
+      gemm::split_pair(item[n].x, item[n].y, p[0].x, p[1].x, p[2].x);
+      gemm::split_pair(item[n].z, item[n].w, p[0].y, p[1].y, p[2].y);
+      unsigned char *dst;
+      if (i < kItems / 2) {
+        const int key = i / 16, d4 = i % 16;
+        dst = kp + kv_slot(key, d4 / 2) + 8 * (d4 & 1);
+      } else {
+        // Keys 32 t + 16 h + 4 c .. + 3 are half h of slot 4 t + c.
+        const int dim = i % 64, k4 = (i - kItems / 2) / 64;
+        dst = vp + kv_slot(dim, 4 * (k4 >> 3) + (k4 & 3)) + 8 * ((k4 >> 2) & 1);
+      }
+#pragma unroll
+      for (int u = 0; u < 3; ++u) *reinterpret_cast<uint2 *>(dst + u * kKvPlane) = p[u];
+    }
+  };
+  gemm::bf8v qp[2][3];  // the wave's query rows, dims 32 s + 8 (l / 16) .. + 7
+  {
+    const float4 *q = reinterpret_cast<const float4 *>(g.q + static_cast<size_t>(row) * kH + head * kHeadDim);
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      const float4 a = q[8 * s + 2 * lg], b = q[8 * s + 2 * lg + 1];
+      const float x[8] = {a.x * kScoreScaleLog2, a.y * kScoreScaleLog2, a.z * kScoreScaleLog2, a.w * kScoreScaleLog2,
+                          b.x * kScoreScaleLog2, b.y * kScoreScaleLog2, b.z * kScoreScaleLog2, b.w * kScoreScaleLog2};
+      gemm::split_eight(x, qp[s]);
+    }
+  }
+  float m = -INFINITY, l = 0.f;  // l: this lane's share of the row's sum
+  f4v lead[4], tail[4];
+#pragma unroll
+  for (int d = 0; d < 4; ++d) lead[d] = tail[d] = f4v{0.f, 0.f, 0.f, 0.f};
+
+  for (int k0 = k_begin; k0 < k_end; k0 += kKeyBlock) {
+    load(k0);
+    stage();
+    __syncthreads();
+    float p[4][4];
+    // A tile of 16 keys at a time: more operands in flight would cost the
+    // registers that let two workgroups share a CU.
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      f4v sl = {0.f, 0.f, 0.f, 0.f}, st = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        gemm::bf8v kx[3];
+#pragma unroll
+        for (int u = 0; u < 3; ++u)
+          kx[u] = *reinterpret_cast<const gemm::bf8v *>(kp + u * kKvPlane + kv_slot(16 * t + lr, 4 * s + lg));
+        sl = mfma16(kx[0], qp[s][0], sl);
+        st = mfma16(kx[0], qp[s][1], st);
+        st = mfma16(kx[1], qp[s][0], st);
+        st = mfma16(kx[1], qp[s][1], st);
+        st = mfma16(kx[0], qp[s][2], st);
+        st = mfma16(kx[2], qp[s][0], st);
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r) p[t][r] = sl[r] + st[r];
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if (k0 + kKeyBlock > g.pos0 + r0 + 1) {  // the block reaches past some row's position
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (k0 + 16 * t + 4 * lg + r > pos) p[t][r] = -INFINITY;
+    }
+    float mx = p[0][0];
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) mx = fmaxf(mx, p[t][r]);
+    mx = fmaxf(m, quads_max(mx));
+    const float ref = mx == -INFINITY ? 0.f : mx;  // no key of the row yet: every term is 2^-inf = 0
+    const float corr = exp2_fast(m - ref);
+    m = mx;
+    float sum = 0.f;
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        p[t][r] = exp2_fast(p[t][r] - ref);
+        sum += p[t][r];
+      }
+    l = fmaf(l, corr, sum);
+#pragma unroll
+    for (int d = 0; d < 4; ++d) {
+      lead[d] *= corr;
+      tail[d] *= corr;
+    }
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      gemm::bf8v px[3];
+      const float x[8] = {p[2 * t][0],     p[2 * t][1],     p[2 * t][2],     p[2 * t][3],
+                          p[2 * t + 1][0], p[2 * t + 1][1], p[2 * t + 1][2], p[2 * t + 1][3]};
+      gemm::split_eight(x, px);
+#pragma unroll
+      for (int d = 0; d < 4; ++d) {
+        gemm::bf8v vx[3];
+#pragma unroll
+        for (int u = 0; u < 3; ++u)
+          vx[u] = *reinterpret_cast<const gemm::bf8v *>(vp + u * kKvPlane + kv_slot(16 * d + lr, 4 * t + lg));
+        lead[d] = mfma16(vx[0], px[0], lead[d]);
+        tail[d] = mfma16(vx[0], px[1], tail[d]);
+        tail[d] = mfma16(vx[1], px[0], tail[d]);
+        tail[d] = mfma16(vx[1], px[1], tail[d]);
+        tail[d] = mfma16(vx[0], px[2], tail[d]);
+        tail[d] = mfma16(vx[2], px[0], tail[d]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    __syncthreads();  // the next block overwrites K and V
+  }
+  l = quads_sum(l);
+  float probe = l * 0.f;
+#pragma unroll
+  for (int d = 0; d < 4; ++d) {
+    lead[d] += tail[d];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) probe = fmaf(lead[d][r], 0.f, probe);
+  }
+  auto record = [&](int of_row) {
+    return g.rec + ((static_cast<size_t>(of_row) * 2 * kGroupHeads + head) * g.splits + z) * kRec;
+  };
+  if (__builtin_amdgcn_ballot_w64(!(probe == 0.f)) != 0) {
+    for (int i = 0; i < kQRows && r0 + i < g.rows; ++i) {
+      float fm, fl, fa;
+      attention_row_fp32(g, r0 + i, head, kv, k_begin, min(k_end, g.pos0 + r0 + i + 1), fm, fl, fa);
+      if (g.splits > 1) {
+        float *rec = record(r0 + i);
+        rec[4 + lane] = fa;
+        if (lane < 2) rec[lane] = lane == 0 ? fm : fl;
+      } else {
+        const gemm::Parts out = gemm::split_value(fa / fl);
+        uint16_t *dst = g.out.at(r0 + i, kH) + head * kHeadDim + lane;
+#pragma unroll
+        for (int u = 0; u < 3; ++u) dst[u * g.out.plane] = out.p[u];
+      }
+    }
+    return;
+  }
+  if (r0 + lr >= g.rows) return;
+  // Lane: dims 16 d + 4 (l / 16) .. + 3 of its row.
+  if (g.splits > 1) {
+    float *rec = record(row);
+#pragma unroll
+    for (int d = 0; d < 4; ++d)
+      *reinterpret_cast<float4 *>(rec + 4 + 16 * d + 4 * lg) = make_float4(lead[d][0], lead[d][1], lead[d][2], lead[d][3]);
+    if (lg == 0) *reinterpret_cast<float2 *>(rec) = make_float2(m, l);
+  } else {
+#pragma unroll
+    for (int d = 0; d < 4; ++d)
+      put_parts(g.out.at(row, kH) + head * kHeadDim, g.out.plane, 4 * d + lg,
+                make_float4(lead[d][0] / l, lead[d][1] / l, lead[d][2] / l, lead[d][3] / l));
+  }
+}
+
+// One prompt row: the partials of its heads over the row block's splits.
+__global__ __launch_bounds__(kBlock) void attention_merge_kernel(AttnArgs g) {
+  const int row = blockIdx.x;
+  const int keys = g.pos0 + min(g.rows, (row / kQRows + 1) * kQRows);
+  const int splits = (keys + g.per_split * kKeyBlock - 1) / (g.per_split * kKeyBlock);
+  const int head = threadIdx.x / (kHeadDim / 4), c = threadIdx.x % (kHeadDim / 4);
+  if (head >= 2 * kGroupHeads) return;
+  const float *rec = g.rec + (static_cast<size_t>(row) * 2 * kGroupHeads + head) * g.splits * kRec;
+  // Eight records requested before any is used (a read at a time took 1 us
+  // per split).
+  constexpr int kBatch = 8;
+  float m = -INFINITY, den = 0.f;
+  float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+  for (int z0 = 0; z0 < splits; z0 += kBatch) {
+    float2 ml[kBatch];
+    float4 a[kBatch];
+#pragma unroll
+    for (int j = 0; j < kBatch; ++j) {
+      const float *r = rec + min(z0 + j, splits - 1) * kRec;
+      ml[j] = *reinterpret_cast<const float2 *>(r);
+      a[j] = *reinterpret_cast<const float4 *>(r + 4 + 4 * c);
+    }
+    float mx = m;
+#pragma unroll
+    for (int j = 0; j < kBatch; ++j) mx = fmaxf(mx, ml[j].x);
+    const float ref = mx == -INFINITY ? 0.f : mx;
+    const float corr = exp2_fast(m - ref);
+    m = mx;
+    den *= corr;
+    acc = make_float4(acc.x * corr, acc.y * corr, acc.z * corr, acc.w * corr);
+#pragma unroll
+    for (int j = 0; j < kBatch; ++j) {
+      if (z0 + j >= splits || (ml[j].x == -INFINITY && ml[j].y == 0.f)) continue;  // no key of the row in the split
+      const float w = exp2_fast(ml[j].x - ref);
+      den = fmaf(w, ml[j].y, den);
+      acc = make_float4(fmaf(w, a[j].x, acc.x), fmaf(w, a[j].y, acc.y), fmaf(w, a[j].z, acc.z), fmaf(w, a[j].w, acc.w));
+    }
+  }
+  put_parts(g.out.at(row, kH) + head * kHeadDim, g.out.plane, c,
+            make_float4(acc.x / den, acc.y / den, acc.z / den, acc.w / den));
 }
 
 // ---- GEMM launches ------------------------------------------------------------------
@@ -507,11 +604,20 @@ hipError_t launch_qkv_rope(hipStream_t s, const float *partials, int splits, int
   return hipGetLastError();
 }
 
-hipError_t launch_attention_prefill(hipStream_t s, const float *q, int rows, int pos0, int nq, int nkv,
-                                    const float *k_cache, const float *v_cache, const PartRows &out) {
-  const int nqb = (rows + kQBlock - 1) / kQBlock;
-  const dim3 grid((nqb + 1) / 2, nq);
-  attention_prefill_kernel<<<grid, kBlock, 0, s>>>(q, rows, pos0, nq, nkv, k_cache, v_cache, out);
+// Key blocks per workgroup: one until about two workgroups per CU are busy,
+// and no more partials than kAttnRecRows rows of records hold.
+hipError_t launch_attention_prefill(hipStream_t s, const float *q, int rows, int pos0, const float *k_cache,
+                                    const float *v_cache, float *records, const PartRows &out) {
+  if (rows <= 0 || pos0 < 0) return hipErrorInvalidValue;
+  const int nqb = (rows + kQRows - 1) / kQRows;
+  long long units = 0;
+  for (int b = 0; b < nqb; ++b) units += (pos0 + std::min(rows, (b + 1) * kQRows) + kKeyBlock - 1) / kKeyBlock;
+  const int blocks = (pos0 + rows + kKeyBlock - 1) / kKeyBlock;
+  const int most = std::max(1, kAttnRecRows / rows);
+  const int per_split = std::max<int>((2 * units + 511) / 512, (blocks + most - 1) / most);
+  AttnArgs g{q, k_cache, v_cache, rows, pos0, per_split, (blocks + per_split - 1) / per_split, records, out};
+  attention_prefill_kernel<<<dim3(nqb, 2, g.splits), kAttnThreads, 0, s>>>(g);
+  if (g.splits > 1) attention_merge_kernel<<<rows, kBlock, 0, s>>>(g);
   return hipGetLastError();
 }
 

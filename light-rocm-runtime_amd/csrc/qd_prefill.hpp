@@ -55,8 +55,10 @@ hipError_t launch_qkv_rope(hipStream_t s, const float *partials, int splits, int
                            float *v_cache);
 
 // Causal GQA attention of rows rotated queries at positions pos0.. over cache
-// positions 0..pos0 + r.
-hipError_t launch_attention_prefill(hipStream_t s, const float *q, int rows, int pos0, int nq, int nkv,
-                                    const float *k_cache, const float *v_cache, const PartRows &out);
+// positions 0..pos0 + r (rows <= kAttnRecRows). records:
+// kAttnRecRows * kAttnRecFloats floats of workspace for partial results.
+constexpr int kAttnRecRows = 8192, kAttnRecFloats = 14 * (kHeadDim + 4);
+hipError_t launch_attention_prefill(hipStream_t s, const float *q, int rows, int pos0, const float *k_cache,
+                                    const float *v_cache, float *records, const PartRows &out);
 
 }  // namespace qd

@@ -124,3 +124,46 @@ def test_weights_beyond_bf16_range_give_fp32_results(value, tmp_path):
     assert np.isfinite(want).all() == np.isfinite(value)
     if np.isfinite(value):
         assert rel_err(k0, k1) <= RTOL and rel_err(got, want) <= RTOL
+
+
+@pytest.mark.parametrize("start,rows", [(1, 1), (15, 17), (47, 17), (63, 2), (64, 64), (100, 16), (1000, 37), (1500, 590)])
+def test_continued_prompts_match_oracle(pair, start, rows):
+    """Row blocks of 16 and key blocks of 64 at positions that are not their
+    multiples, with one and with several key splits per row block."""
+    eng, prompt, cache = pair
+    print(f"prefill {eng.config.decoder_dtype} {start} + {rows} rows", flush=True)
+    eng.kv_reset(0, 0)
+    eng.prefill(0, prompt[:start], want_logits=False)
+    eng.prefill(0, prompt[start:start + rows], want_logits=False)
+    k, v = eng.read_kv(0, LAYERS - 1, start, rows)
+    assert rel_err(k, cache.layer(LAYERS - 1, False)[start:start + rows]) <= RTOL
+    assert rel_err(v, cache.layer(LAYERS - 1, True)[start:start + rows]) <= RTOL
+
+
+@pytest.mark.parametrize("k_value,v_value", [(3.395e38, 1.0), (-np.inf, 1.0), (np.inf, 1.0), (1.0, 3.395e38), (1.0, np.inf)])
+def test_cache_rows_beyond_bf16_range_give_fp32_results(k_value, v_value):
+    """Cached K / V values that round to infinity in BF16 or are infinite:
+    attention gives what the step kernels' FP32 arithmetic gives."""
+    print(f"prefill over cached K {k_value}, V {v_value}", flush=True)
+    eng = qd.Engine(layers=LAYERS, vocab=VOCAB, capacity=128, max_batch=2)
+    eng.load_synthetic(3)
+    k = qo.fill_normal(80 * 128, 3, 0x200000, 0.0, 1.0).reshape(80, 128)
+    v = qo.fill_normal(80 * 128, 3, 0x200001, 0.0, 1.0).reshape(80, 128)
+    k[70, 3] *= np.float32(k_value)
+    v[70, 9] *= np.float32(v_value)
+    k[np.abs(k) > 3.4e38] = k_value
+    v[np.abs(v) > 3.4e38] = v_value
+    for seq in range(2):
+        for layer in range(LAYERS):
+            eng.write_kv(seq, layer, 0, k, v)
+        eng.kv_reset(seq, 80)
+    prompt = qo.fill_tokens(20, 5, 0x300000, VOCAB)
+    got = eng.prefill(0, prompt)[2]
+    for t in prompt.tolist():
+        want = eng.step(1, t)[2]
+    k0, k1 = (eng.read_kv(seq, 1, 80, 20)[0] for seq in range(2))
+    eng.close()
+    fine = np.isfinite(k1)
+    assert np.array_equal(np.isfinite(k0), fine) and np.array_equal(np.isfinite(got), np.isfinite(want))
+    if fine.any():
+        assert np.abs(k0[fine] - k1[fine]).max() <= RTOL * np.abs(k1[fine]).max()
