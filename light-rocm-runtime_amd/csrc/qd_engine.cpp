@@ -155,8 +155,13 @@ struct qd_engine {
   float *roles_slots = nullptr;             // hand-off slots
   size_t roles_slot_bytes = 0;
   uint32_t epoch = 0;                       // last launch epoch (1..4095)
-  uint32_t *resident_error = nullptr;       // [1 + kXcds]
+  uint32_t *resident_error = nullptr;       // [1 + kXcds], then the sticky word of layers-only launches
+  bool layers_pending = false;              // the sticky error word is due at the next sync
   uint32_t spin_limit = qd::kResidentSpinLimit;
+  // Layers of one qd_layer_decode from which a resident launch is the faster
+  // (us at context 701, resident / stream: 2 layers 96 / 90, 3 109 / 127, 24
+  // 394 / 900; BF16 94 / 83, 106 / 116, 388 / 819).
+  static constexpr size_t kResidentLayers = 3;
   int roles_grid = 0;                       // 0: resident path unavailable
   std::string resident_off_reason;
   // Prompt workspace (allocated on the first prefill) for chunks of up to
@@ -183,7 +188,7 @@ struct qd_engine {
 
   qd::SeqState *h_states = nullptr;  // pinned [max_batch]
   uint32_t *h_tokens = nullptr;      // pinned [capacity]
-  uint32_t *h_error = nullptr;       // pinned [1]: a resident launch's error word
+  uint32_t *h_error = nullptr;       // pinned [2]: a resident launch's error word, the sticky one
   std::vector<uint32_t> positions;   // host mirror of each slot's position
   bool loaded = false;
   qd_timing timing{};
@@ -615,17 +620,20 @@ struct qd_engine {
   hipError_t launch_resident(const qd::RolePlan &plan, uint32_t seq, uint32_t first_token,
                              uint32_t max_tokens, uint32_t eos, float *hist, int use_hist,
                              uint64_t *stage_ticks, uint64_t *trace = nullptr,
-                             uint32_t trace_token = 0) {
+                             uint32_t trace_token = 0, float *hidden_io = nullptr, size_t first_layer = 0,
+                             size_t layer_count = 0) {
+    if (!hidden_io) layer_count = L;
     epoch = epoch % 4095u + 1u;
     qd::ResidentArgs ra{};
-    ra.layer_ptrs = layer_ptrs_dev;
+    ra.layer_ptrs = layer_ptrs_dev + first_layer;
     ra.embed = embed;
     ra.head = lm_head;
     ra.final_norm = final_norm;
     ra.rope_cos = rope_cos;
     ra.rope_sin = rope_sin;
-    ra.k_cache = kv_slice(k_cache, seq, 0);
-    ra.v_cache = kv_slice(v_cache, seq, 0);
+    ra.k_cache = kv_slice(k_cache, seq, first_layer);
+    ra.v_cache = kv_slice(v_cache, seq, first_layer);
+    ra.hidden_io = hidden_io;
     ra.top = top_pairs;
     ra.slots = roles_slots;
     ra.logits = hist;
@@ -638,7 +646,7 @@ struct qd_engine {
     ra.history = use_hist;
     ra.capacity = static_cast<int>(CAP);
     ra.vocab = static_cast<int>(V);
-    ra.layers = static_cast<int>(L);
+    ra.layers = static_cast<int>(layer_count);
     ra.nq = static_cast<int>(NQ);
     ra.nkv = static_cast<int>(NKV);
     ra.eps = cfg.rms_eps;
@@ -664,7 +672,7 @@ struct qd_engine {
     // Error word and tickets zero, token 0's hand-off slots empty (all bits
     // set), the tag arena zero when the epoch counter wrapped.
     check(qd::launch_roles_prepare(stream, resident_error, roles_slots, roles_slot_bytes / (8 * L),
-                                   int(L), epoch == 1u ? top_pairs : nullptr, 4 * roles_grid),
+                                   int(layer_count), epoch == 1u ? top_pairs : nullptr, 4 * roles_grid),
           "resident prepare");
     return qd::launch_roles(stream, ra, roles_grid);
   }
@@ -715,7 +723,38 @@ struct qd_engine {
     return uint64_t(max_tokens) * (5 * L + 1) + 1 < (uint64_t(1) << qd::kTagSeqBits);
   }
 
-  void sync() { check(hipStreamSynchronize(stream), "hipStreamSynchronize"); }
+  // Waits for the stream; the errors of layers-only resident launches, which
+  // were asynchronous, surface here.
+  void sync() {
+    check(hipStreamSynchronize(stream), "hipStreamSynchronize");
+    if (layers_pending) {
+      layers_pending = false;
+      const uint32_t err = h_error[1];
+      if (err) check(hipMemsetAsync(resident_error + 1 + qd::kXcds, 0, 4, stream), "memset");
+      resident_status(err);
+    }
+  }
+  // Decoder layers [first, first + count) of slot seq on its device hidden
+  // vector at its position: one layers-only resident launch, or the stream
+  // kernels; the two compute the same values bit for bit.
+  void enqueue_layers(uint32_t seq, size_t first, size_t count) {
+    qd::RolePlan plan{};
+    if (count >= kResidentLayers && resident_plan(positions[seq], 1, &plan)) {
+      const hipError_t err = launch_resident(plan, seq, 0, 1, UINT32_MAX, nullptr, 0, nullptr, nullptr, 0,
+                                             hidden + seq * H, first, count);
+      if (err == hipSuccess) {
+        check(qd::launch_roles_export(stream, roles_slots, int(count) - 1, int(positions[seq]) + 1, q + seq * QD,
+                                      attn + seq * QD, act + seq * I, resident_error,
+                                      resident_error + 1 + qd::kXcds),
+              "resident export");
+        check(hipMemcpyAsync(h_error + 1, resident_error + 1 + qd::kXcds, 4, hipMemcpyDeviceToHost, stream), "D2H");
+        layers_pending = true;
+        return;
+      }
+      if (!resident_refused(err)) check(err, "resident launch");
+    }
+    for (size_t l = first; l < first + count; ++l) check(qd::launch_layer(stream, layer_args(seq, l)), "layer launch");
+  }
 };
 
 namespace {
@@ -902,7 +941,7 @@ qd_status qd_engine_create(const qd_config *config, qd_engine **out) {
     check(hipHostMalloc(reinterpret_cast<void **>(&e->h_tokens), e->CAP * sizeof(uint32_t),
                         hipHostMallocDefault),
           "hipHostMalloc");
-    check(hipHostMalloc(reinterpret_cast<void **>(&e->h_error), sizeof(uint32_t), hipHostMallocDefault),
+    check(hipHostMalloc(reinterpret_cast<void **>(&e->h_error), 2 * sizeof(uint32_t), hipHostMallocDefault),
           "hipHostMalloc");
     e->positions.assign(e->B, 0);
     e->build_rope_tables(c.rope_theta);
@@ -939,7 +978,8 @@ qd_status qd_engine_create(const qd_config *config, qd_engine **out) {
                             qd::roles_slot_floats(int(e->H), int(e->I), int(e->NQ), int(e->NKV));
       e->roles_slots = e->alloc<float>(e->roles_slot_bytes / 4);
     }
-    e->resident_error = e->alloc<uint32_t>(1 + qd::kXcds);
+    e->resident_error = e->alloc<uint32_t>(2 + qd::kXcds);
+    check(hipMemsetAsync(e->resident_error, 0, (2 + qd::kXcds) * 4, e->stream), "memset");
     {
       hipError_t err = hipSuccess;
       e->batch_scratch = qd::batch_scratch(c.device, &err);
@@ -1334,8 +1374,7 @@ qd_status qd_layer_decode(qd_engine *e, uint32_t seq, uint32_t first_layer, uint
     // this token is in flight (qd_tail completes it).
     e->positions[seq] = valid_keys - 1;
     check(qd::launch_set_state(e->stream, e->states + seq, valid_keys - 1, 0), "state launch");
-    for (uint32_t l = first_layer; l < first_layer + layer_count; ++l)
-      check(qd::launch_layer(e->stream, e->layer_args(seq, l)), "layer launch");
+    e->enqueue_layers(seq, first_layer, layer_count);
   });
 }
 

@@ -62,6 +62,10 @@ struct ResidentArgs {
   float *logits;                // [vocab] or [max_tokens][vocab]
   uint32_t *out_tokens;         // [max_tokens]
   SeqState *st;
+  float *hidden_io;             // nullptr, or [hidden]: layers only. Layer 0's input is this
+                                //   vector instead of the token's embedding, the last layer's
+                                //   output replaces it, and the launch ends without LM head,
+                                //   argmax and state (max_tokens 1)
   uint32_t *error;              // [1 + kXcds], zero at launch: kResident* bits, then each
                                 //   XCD's count of workgroups that have taken a position
   uint64_t *stage_ticks;        // nullptr, or [kResidentStages] 100 MHz ticks
@@ -126,6 +130,12 @@ hipError_t launch_roles(hipStream_t s, const ResidentArgs &args, int grid);
 // top_pairs (value, tag) pairs zero.
 hipError_t launch_roles_prepare(hipStream_t s, uint32_t *error, float *slots, size_t slot_floats,
                                int layers, void *top, int top_pairs);
+
+// After a layers-only launch: the last layer's query, attention output and
+// SwiGLU activation out of its hand-off slots (as the stream kernels leave
+// them), for a context of `length` positions; *sticky |= *error.
+hipError_t launch_roles_export(hipStream_t s, const float *slots, int last_layer, int length, float *q, float *attn,
+                               float *act, const uint32_t *error, uint32_t *sticky);
 // Largest co-resident grid of the role kernel for decoder matrices stored as
 // `weights_dtype` (kWeights*) on `device` (0 if the query fails).
 int roles_max_grid(int device, int weights_dtype);

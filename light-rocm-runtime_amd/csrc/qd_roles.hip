@@ -1122,6 +1122,15 @@ struct Roles {
         clock.at(traced, l);
         if (!layer(t, l, position)) return;
       }
+      if (a.hidden_io) {
+        // Layers only. Every CU that reads the input has, once the last
+        // layer's output is complete; loads still in flight (the next
+        // token's share) land before the CU goes.
+        if (blockIdx.x == 0 && gather_hid(t, a.layers - 1, 0, H, cm.vec))
+          for (int c = threadIdx.x; c < H; c += kT) a.hidden_io[c] = cm.vec[c];
+        vm_wait();
+        return;
+      }
       clock.at(traced, a.layers);
       if (!lm_head(t)) return;
       if (defer_first) pre_lds(0, position + 1);
@@ -1286,7 +1295,7 @@ struct Roles {
   // layer's output, or this token's embedding row at l = 0) -> dst.
   __device__ bool layer_input(uint32_t t, int l, int first4, int n4, float *dst) {
     if (l == 0) {
-      const float *e = a.embed + static_cast<size_t>(token) * H;
+      const float *e = a.hidden_io ? a.hidden_io : a.embed + static_cast<size_t>(token) * H;
       for (int c = threadIdx.x; c < n4; c += kT) reinterpret_cast<float4 *>(dst)[c] = ld_global4(e, first4 + c);
       vm_wait();
       lds_barrier();
@@ -2054,6 +2063,29 @@ const void *roles_fn(bool profile, int weights_dtype) {
   }
 }
 
+// One workgroup per query head: the head's attention output from its partial
+// records (the stream kernels' merge), and a share of the query and the
+// activation. Token 0's slot block of a layer, layout R. The launch's error
+// word is added to the sticky one.
+template <typename R>
+__global__ __launch_bounds__(256) void roles_export_kernel(const float *__restrict__ block, int length,
+                                                           float *__restrict__ q, float *__restrict__ attn,
+                                                           float *__restrict__ act,
+                                                           const uint32_t *__restrict__ error,
+                                                           uint32_t *__restrict__ sticky) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) *sticky |= *error;
+  const int h = blockIdx.x, heads = gridDim.x;
+  if (threadIdx.x < kHeadDim) {
+    const float *rec = block + R::kOffPart + h * kAttnMaxChunks * kRoleRecStride;
+    attn[h * kHeadDim + threadIdx.x] = attn_merge(
+        [&](int c, int k) { return rec[c * kRoleRecStride + (k < 2 ? k : k + 2)]; }, decode_chunks(length),
+        static_cast<int>(threadIdx.x));
+    q[h * kHeadDim + threadIdx.x] = block[R::kOffQkv + h * kHeadDim + threadIdx.x];
+  }
+  constexpr int kAct = R::kOffHid - R::kOffAct;
+  for (int i = h * blockDim.x + threadIdx.x; i < kAct; i += heads * blockDim.x) act[i] = block[R::kOffAct + i];
+}
+
 // What a resident launch expects at its start, in one dispatch: the error
 // word and the XCD tickets zero, and parity 0's block of every layer's
 // hand-off slots empty (token 0's). Parity 1's blocks need no clearing:
@@ -2183,6 +2215,15 @@ hipError_t launch_roles_prepare(hipStream_t s, uint32_t *error, float *slots, si
   hipLaunchKernelGGL(roles_prepare_kernel, grid, dim3(256), 0, s, error,
                      reinterpret_cast<uint4 *>(slots), block_u4, static_cast<uint2 *>(top),
                      top ? static_cast<uint32_t>(top_pairs) : 0u);
+  return hipGetLastError();
+}
+
+hipError_t launch_roles_export(hipStream_t s, const float *slots, int last_layer, int length, float *q, float *attn,
+                               float *act, const uint32_t *error, uint32_t *sticky) {
+  if (last_layer < 0 || length < 1) return hipErrorInvalidValue;
+  using R = Roles<896, 4864, 14, 2, false, float>;
+  roles_export_kernel<R><<<14, 256, 0, s>>>(slots + static_cast<size_t>(last_layer) * 2 * R::kSlotFloats, length, q,
+                                            attn, act, error, sticky);
   return hipGetLastError();
 }
 
