@@ -5,13 +5,17 @@
 // v_mfma_f32_16x16x4f32: the (up to) 16 sequences are the M dimension and a
 // 16-row tile of the weight matrix is N. Lane l of a wave supplies
 // A[l % 16][l / 16] and B[l / 16][l % 16] and result register r holds
-// D[(l / 16) * 4 + r][l % 16]; so lane l streams weight row (l % 16) of the
-// tile in float4 loads at k offset 4 * (l / 16) of each 16-wide k step and
-// multiplies it with the same k offsets of sequence (l % 16)'s operand row.
-// Each weight is read from HBM once per step for the whole batch. The waves
-// of a workgroup split K; their partial tiles are summed in LDS in a fixed
-// order and the 256 tile elements go through the fused epilogue (bias,
-// RoPE + KV write, residual add, SiLU gate, logits + top-1).
+// D[(l / 16) * 4 + r][l % 16]. Each weight is read from HBM once per step for
+// the whole batch. The waves of a workgroup split K; both operands reach them
+// through LDS rings filled by DMA (split_product); the waves' partial tiles are
+// summed in LDS in a fixed order and the 256 tile elements go through the fused
+// epilogue (bias, RoPE + KV write, residual add, SiLU gate). The LM head keeps
+// the operand rows in LDS and streams the vocabulary past them.
+//
+// What bounds a step (16 rows): the weights' 1.98 GB would stream in about
+// 280 us; a layer's five kernels take 8.0 (QKV), 16.8 (attention, contexts to
+// 2,048), 7.4 (O), 12.8 (gate/up) and 10 us (down), of which each kernel's
+// start, first load and split-K hand-over are most of the three small ones.
 //
 // Semantics per sequence are those of the batch-1 step (qd_kernels.hip):
 //   RMSNorm                 benchmarks/qwen_stateful_graph_kernel.cpp:665-701
@@ -39,10 +43,8 @@ typedef float f4v __attribute__((ext_vector_type(4)));
 
 constexpr int kH = 896;    // hidden = query width
 constexpr int kI = 4864;   // MLP intermediate
-constexpr int kStep = 16;  // k values one float4 load per lane covers per wave
 
 __device__ __forceinline__ int tile_col() { return lane_id() & 15; }     // N index (weight row)
-__device__ __forceinline__ int k_quad() { return (lane_id() >> 4) * 4; }  // k offset in a step
 
 __device__ __forceinline__ float4 ld4(const float *p) {
   return *reinterpret_cast<const float4 *>(p);
@@ -56,93 +58,131 @@ __device__ __forceinline__ f4v mfma4(float4 a, float4 b, f4v acc) {
   return acc;
 }
 
-// The raw operand slice of this lane for kSteps k-steps from kbase:
-// sequence row (lane % 16) of x (K floats per row), zero for rows >= rows.
-template <int kSteps, int K>
-__device__ __forceinline__ void load_operand(const float *__restrict__ x, int rows, int kbase,
-                                             float4 (&xa)[kSteps]) {
-  const int b = tile_col();
-  const int k0 = kbase + k_quad();
-  const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
-  if (b >= rows) {
+// RMSNorm folded into the GEMM: y = x * inv * g gives W.y = inv * W.(x g).
+// The kernel that finishes a hidden row stores x * g for the next norm's gain
+// (BatchLaunch::gained) and, per 16-column tile, the sum of the tile's squares
+// (BatchLaunch::squares); the GEMMs then load one operand and no gain (whose
+// registers kept the gate/up workgroups to two per CU, two rounds of them), and
+// their epilogue threads, 16 per sequence, add up the
+// row's squares themselves.
+__device__ __forceinline__ float row_inv(const BatchLaunch &p, int seq) {
+  const float *sq = p.squares + seq * kBatchTiles + (threadIdx.x & 15);
+  float s = 0.f;
 #pragma unroll
-    for (int s = 0; s < kSteps; ++s) xa[s] = zero;
-    return;
+  for (int j = 0; j < kBatchTiles / 16; ++j) s += sq[16 * j];
+  return rsqrtf(row16_sum(s) / static_cast<float>(kH) + p.eps);
+}
+
+// Element v of hidden row seq, column n0 + (t & 15) of tile `tile`, by the
+// tile's 256 threads: the row, its gained copy and its share of the squares.
+__device__ __forceinline__ void put_hidden(const BatchLaunch &p, int seq, int tile, float v, float gain) {
+  const int col = tile * 16 + (threadIdx.x & 15);
+  const float ss = row16_sum(v * v);
+  if (seq >= p.rows) return;
+  p.hidden[seq * kH + col] = v;
+  p.gained[seq * kH + col] = v * gain;
+  if ((threadIdx.x & 15) == 0) p.squares[seq * kBatchTiles + tile] = ss;
+}
+
+// ---- K slices through LDS -------------------------------------------------------
+// One wave's product of X[:, k] and W[rows, k] over 32-wide k slices
+// [s0, s1), both operands through the wave's own ring of kRing LDS stages
+// (2 KiB of X, 2 KiB of W each), filled by global -> LDS DMA. A DMA moves
+// whole 128-byte lines (8 rows of a slice), where a load into the operand
+// layout (16 rows x 64 bytes) takes every line in two halves; and no registers
+// wait for memory. The ring is the wave's own, so no barrier. Against operand
+// loads into registers, 16 rows, per layer: gate/up 19.1 -> 12.8 us, down
+// 12 -> 10, QKV 9.8 -> 8.0. (Rings of 2 or 4 stages: 1161 and 1173 us a step
+// against 1162; K = 896 in 3 or 4 splits and down in 6: 1178.)
+// Rows are 32 floats, 16-byte slot p holding piece p ^ ((row / 2) % 8): the 16
+// rows' reads of one piece fall on distinct banks.
+constexpr int kSlice = 32, kRing = 3, kStageFloats = 2 * 16 * kSlice, kRingFloats = kRing * kStageFloats;
+typedef __attribute__((address_space(3))) void ring_lds_void;
+// kOnce: bytes that no other workgroup reads (weights), not to be kept in L2
+// (LM head at 16 rows 113 -> 106 us).
+template <bool kOnce>
+__device__ __forceinline__ void ring_dma(const float *src, uint32_t lds) {
+  if constexpr (kOnce)
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off nt" ::"s"(lds), "v"(src) : "memory");
+  else
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(src) : "memory");
+}
+template <int n>
+__device__ __forceinline__ void ring_wait() {
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(n) : "memory");
+}
+// The DMA source of this lane for instruction i of a 16-row, 32-column slice:
+// its 16-byte piece of row 8 i + lane / 8.
+__device__ __forceinline__ int ring_row(int i) { return 8 * i + (lane_id() >> 3); }
+__device__ __forceinline__ int ring_piece(int row) { return 4 * ((lane_id() & 7) ^ ((row >> 1) & 7)); }
+__device__ __forceinline__ uint32_t ring_address(const float *ring) {
+  return static_cast<uint32_t>(
+      __builtin_amdgcn_readfirstlane(static_cast<int>(reinterpret_cast<uintptr_t>((ring_lds_void *)ring))));
+}
+// Operand float4s of k's 4 (l / 16) .. + 3 and 16 further on, row l % 16 of a slice.
+__device__ __forceinline__ void ring_read(const float *slice, float4 &a, float4 &b) {
+  const int row = lane_id() & 15, sw = (row >> 1) & 7, quad = lane_id() >> 4;
+  const float4 *r = reinterpret_cast<const float4 *>(slice) + row * 8;
+  a = r[quad ^ sw];
+  b = r[(4 + quad) ^ sw];
+}
+
+// This wave's part of X . W^T over K floats per row (X row i at x + i K, W row
+// j at wrow(j)), K dealt in slices to the waves of kSplits workgroups.
+template <int K, int kSplits, typename WRow>
+__device__ __forceinline__ f4v split_product(float (*rings)[kRingFloats], const float *x, WRow wrow) {
+  const int w = __builtin_amdgcn_readfirstlane(wave_id());
+  constexpr int kWaves = kWavesPerBlock * kSplits, kSlices = K / kSlice;
+  const int part = blockIdx.y * kWavesPerBlock + w;
+  const int s0 = part * kSlices / kWaves, n = (part + 1) * kSlices / kWaves - s0;
+  const float *ring = rings[w];
+  const uint32_t base = ring_address(ring);
+  const float *src[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int row = ring_row(i & 1);
+    src[i] = (i < 2 ? x + row * K : wrow(row)) + s0 * kSlice + ring_piece(row);
   }
-  const float *row = x + static_cast<size_t>(b) * K;
+  auto fetch = [&](int stage) {
 #pragma unroll
-  for (int s = 0; s < kSteps; ++s) xa[s] = ld4(row + k0 + kStep * s);
-}
-
-// The gain slice matching load_operand's k offsets.
-template <int kSteps>
-__device__ __forceinline__ void load_gain(int kbase, const float *__restrict__ gain,
-                                          float4 (&gv)[kSteps]) {
-  const int k0 = kbase + k_quad();
+    for (int i = 0; i < 4; ++i) {
+      const uint32_t dst = base + stage * kStageFloats * 4 + i * 1024;
+      if (i < 2)
+        ring_dma<false>(src[i], dst);
+      else
+        ring_dma<true>(src[i], dst);
+      src[i] += kSlice;
+    }
+  };
 #pragma unroll
-  for (int s = 0; s < kSteps; ++s) gv[s] = ld4(gain + k0 + kStep * s);
-}
-
-// RMSNorm folded into the GEMM: y = x * inv * g gives W.y = inv * W.(x g),
-// so the matrix cores take x * g and the epilogue scales by the row's inv.
-// Returns this lane's contribution to the sum of squares of its row and
-// scales the slice by the gain in place.
-template <int kSteps>
-__device__ __forceinline__ float gain_operand(const float4 (&gv)[kSteps], float4 (&xa)[kSteps]) {
-  float ss = 0.f;
-#pragma unroll
-  for (int s = 0; s < kSteps; ++s) {
-    const float4 g = gv[s];
-    float4 &x = xa[s];
-    ss = fmaf(x.x, x.x, ss);
-    ss = fmaf(x.y, x.y, ss);
-    ss = fmaf(x.z, x.z, ss);
-    ss = fmaf(x.w, x.w, ss);
-    x = make_float4(x.x * g.x, x.y * g.y, x.z * g.z, x.w * g.w);
+  for (int d = 0; d < kRing; ++d)
+    if (d < n) fetch(d);
+  f4v acc = {0.f, 0.f, 0.f, 0.f};
+  int stage = 0;
+  for (int s = 0; s < n; ++s) {
+    // Stage s has landed once at most the later stages' DMAs, four each, are
+    // outstanding.
+    static_assert(kRing == 3, "two later stages at most");
+    if (n - 1 - s >= 2)
+      ring_wait<8>();
+    else if (n - 1 - s == 1)
+      ring_wait<4>();
+    else
+      ring_wait<0>();
+    float4 x0, x1, w0, w1;
+    ring_read(ring + stage * kStageFloats, x0, x1);
+    ring_read(ring + stage * kStageFloats + 16 * kSlice, w0, w1);
+    acc = mfma4(x0, w0, acc);
+    acc = mfma4(x1, w1, acc);
+    // The operands are in registers: the stage can be filled again.
+    if (s + kRing < n) {
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      fetch(stage);
+    }
+    stage = stage + 1 == kRing ? 0 : stage + 1;
   }
-  return ss;
-}
-
-// Sums each row's squares over the workgroup's waves: lanes b, b + 16,
-// b + 32, b + 48 of every wave hold row b's pieces. ss[b] receives the sum.
-// Ends with a workgroup barrier.
-__device__ __forceinline__ void rows_sum_squares(float part, float (*wss)[16], float *ss) {
-  part += __shfl_xor(part, 16, kWave);
-  part += __shfl_xor(part, 32, kWave);
-  if (lane_id() < 16) wss[wave_id()][lane_id()] = part;
-  __syncthreads();
-  const int waves = blockDim.x / kWave;
-  if (threadIdx.x < 16) {
-    float t = 0.f;
-    for (int w = 0; w < waves; ++w) t += wss[w][threadIdx.x];
-    ss[threadIdx.x] = t;
-  }
-  __syncthreads();
-}
-
-// This lane's weight slice for kSteps k-steps from kbase of row wrow (K
-// floats per row): float4 s at k = kbase + 16 s + 4 (lane / 16).
-template <int kSteps>
-__device__ __forceinline__ void load_weights(const float *__restrict__ wrow, int kbase,
-                                             float4 (&wv)[kSteps]) {
-  const int k0 = kbase + k_quad();
-#pragma unroll
-  for (int s = 0; s < kSteps; ++s)
-    wv[s] = ld_weight(reinterpret_cast<const float4 *>(wrow + k0 + kStep * s));
-}
-
-// acc += X[:, k slice] . W[row, k slice]^T from the loaded slices.
-template <int kSteps>
-__device__ __forceinline__ f4v tile_mfma(const float4 (&xa)[kSteps], const float4 (&wv)[kSteps],
-                                         f4v acc) {
-#pragma unroll
-  for (int s = 0; s < kSteps; ++s) acc = mfma4(xa[s], wv[s], acc);
   return acc;
 }
-
-// Keeps the compiler from moving any instruction across this point: placed
-// after a kernel's loads so all of them are in flight before the first wait.
-__device__ __forceinline__ void issue_fence() { __builtin_amdgcn_sched_barrier(0); }
 
 // Sums the waves' partial tiles: red is [waves][4][64]; thread t < 256
 // returns element (register t / 64, lane t % 64), i.e. sequence
@@ -170,50 +210,35 @@ __device__ __forceinline__ int tile_seq(int t) { return ((t & 63) >> 4) * 4 + (t
 // s_waitcnt encoding: vmcnt 0, expcnt and lgkmcnt not waited on).
 __device__ __forceinline__ void wait_vm_stores() { __builtin_amdgcn_s_waitcnt(0x0F70); }
 
-// Split-K over workgroups: workgroup blockIdx.y of `splits` deposits its
-// partial tile (thread t < 256 holds element t) and, with kSsq, its row
-// sums of squares ss[0..16); the last workgroup of the tile to arrive sums
-// the deposits in split order (deterministic) into v and ss, resets the
-// tile's counter and returns true. Other workgroups return false. Deposits
-// use device-scope (sc1) stores and loads, which are coherent across the
-// XCDs' L2s without an L2 writeback or invalidate; each depositing thread
+// Split-K over workgroups: workgroup blockIdx.y of kSplits deposits its
+// partial tile (thread t < 256 holds element t); the last workgroup of the
+// tile to arrive sums the deposits in split order (deterministic) into v,
+// resets the tile's counter and returns true. Other workgroups return false.
+// Deposits use device-scope (sc1) stores and loads, which are coherent across
+// the XCDs' L2s without an L2 writeback or invalidate; each depositing thread
 // waits for its stores to complete before the workgroup's arrival is counted.
-constexpr int kSplitRec = 256 + 16;
-template <int kSplits, bool kSsq>
-__device__ bool split_gather(float &v, float *ss, float *__restrict__ ws, uint32_t *cnt, int tile) {
+constexpr int kSplitRec = 256;
+template <int kSplits>
+__device__ bool split_gather(float &v, float *__restrict__ ws, uint32_t *cnt, int tile) {
   __shared__ uint32_t last;
-  constexpr int splits = kSplits;
   const int t = threadIdx.x;
-  if (splits == 1) return true;
-  const Coherent dep(ws + static_cast<size_t>(tile) * splits * kSplitRec,
-                     static_cast<uint32_t>(splits * kSplitRec * sizeof(float)));
-  const uint32_t mine = blockIdx.y * kSplitRec;
-  if (t < 256) dep.st(mine + t, v);
-  if (kSsq && t < 16) dep.st(mine + 256 + t, ss[t]);
+  if (kSplits == 1) return true;
+  const Coherent dep(ws + static_cast<size_t>(tile) * kSplits * kSplitRec,
+                     static_cast<uint32_t>(kSplits * kSplitRec * sizeof(float)));
+  dep.st(blockIdx.y * kSplitRec + t, v);
   wait_vm_stores();
   __syncthreads();
-  if (t == 0) last = atomicAdd(cnt + tile, 1u) == static_cast<uint32_t>(splits - 1);
+  if (t == 0) last = atomicAdd(cnt + tile, 1u) == static_cast<uint32_t>(kSplits - 1);
   __syncthreads();
   if (!last) return false;
   // All deposits are requested before any is summed (one round trip).
-  float pv[kSplits], pq[kSplits];
+  float pv[kSplits];
 #pragma unroll
-  for (int s = 0; s < kSplits; ++s) {
-    pv[s] = t < 256 ? dep.ld(s * kSplitRec + t) : 0.f;
-    pq[s] = kSsq && t < 16 ? dep.ld(s * kSplitRec + 256 + t) : 0.f;
-  }
-  float sum = 0.f, sq = 0.f;
+  for (int s = 0; s < kSplits; ++s) pv[s] = dep.ld(s * kSplitRec + t);
+  float sum = 0.f;
 #pragma unroll
-  for (int s = 0; s < kSplits; ++s) {
-    sum += pv[s];
-    sq += pq[s];
-  }
+  for (int s = 0; s < kSplits; ++s) sum += pv[s];
   v = sum;
-  if (kSsq) {
-    __syncthreads();
-    if (t < 16) ss[t] = sq;
-    __syncthreads();
-  }
   if (t == 0) cnt[tile] = 0u;
   return true;
 }
@@ -228,14 +253,16 @@ __device__ __forceinline__ float *kv_rows(float *cache, uint32_t slot, int layer
 
 // ---- kernels --------------------------------------------------------------------
 
-__global__ __launch_bounds__(kBlock) void batch_embed_kernel(BatchLaunch p,
-                                                             const float *__restrict__ emb,
-                                                             int vocab) {
+__global__ __launch_bounds__(kBlock) void batch_embed_kernel(BatchLaunch p, const float *__restrict__ emb,
+                                                             const float *__restrict__ gain, int vocab) {
   const int b = blockIdx.x;
   const uint32_t tok = p.token[b];
   if (tok >= static_cast<uint32_t>(vocab)) return;
   const float *src = emb + static_cast<size_t>(tok) * kH;
-  for (int i = threadIdx.x; i < kH; i += kBlock) p.hidden[b * kH + i] = src[i];
+  for (int tile = threadIdx.x >> 4; tile < kH / 16; tile += kBlock / 16) {
+    const int col = tile * 16 + (threadIdx.x & 15);
+    put_hidden(p, b, tile, src[col], gain[col]);
+  }
 }
 
 // Attention RMSNorm + packed QKV + bias + RoPE + KV-cache write. Tile
@@ -244,24 +271,15 @@ __global__ __launch_bounds__(kBlock) void batch_embed_kernel(BatchLaunch p,
 // j + 8: the rotate-half partners sit in lanes l and l ^ 8. Heads [0, nq)
 // are queries, then nkv keys, then nkv values (not rotated). K = 896 is
 // split over kQkvSplit workgroups of four waves (two: 144 workgroups instead
-// of 72, 9.8 against 10.6 us per layer in a same-box A/B).
-#ifndef QD_BATCH_QKV_SPLIT
-#define QD_BATCH_QKV_SPLIT 2
-#endif
-constexpr int kQkvSplit = QD_BATCH_QKV_SPLIT;
-__global__ __launch_bounds__(kBlock) void batch_qkv_kernel(BatchLaunch p, const float *__restrict__ gain,
-                                                           const float *__restrict__ wqkv,
+// of 72).
+constexpr int kQkvSplit = 2;
+__global__ __launch_bounds__(kBlock) void batch_qkv_kernel(BatchLaunch p, const float *__restrict__ wqkv,
                                                            const float *__restrict__ bqkv, int layer) {
-  constexpr int kSteps = kH / kStep / kWavesPerBlock / kQkvSplit;  // 7
-  __shared__ float wss[kWavesPerBlock][16];
-  __shared__ float ss[16];
+  __shared__ __attribute__((aligned(16))) float ring[kWavesPerBlock][kRingFloats];
   __shared__ float red[kWavesPerBlock][4][kWave];
   const int tile = blockIdx.x;
   const int head = tile >> 2;
   const int i0 = (tile & 3) * 8;
-  const int kbase = (blockIdx.y * kWavesPerBlock + wave_id()) * kSteps * kStep;
-  const int j = tile_col();
-  const int wrow = head * kHeadDim + (j < 8 ? i0 + j : kRotary + i0 + j - 8);
   // Epilogue element of this thread: its bias and rotation are requested
   // with the weights.
   const int t = threadIdx.x;
@@ -273,21 +291,14 @@ __global__ __launch_bounds__(kBlock) void batch_qkv_kernel(BatchLaunch p, const 
   const float bias = bqkv[row];
   const float c = p.rope_cos[pos * kRotary + i];
   const float s = p.rope_sin[pos * kRotary + i];
-  float4 wv[kSteps], xa[kSteps];
-  load_weights<kSteps>(wqkv + static_cast<size_t>(wrow) * kH, kbase, wv);
-  float4 gv[kSteps];
-  load_operand<kSteps, kH>(p.hidden, p.rows, kbase, xa);
-  load_gain<kSteps>(kbase, gain, gv);
-  issue_fence();
-  const float part = gain_operand<kSteps>(gv, xa);
-  f4v acc = {0.f, 0.f, 0.f, 0.f};
-  acc = tile_mfma<kSteps>(xa, wv, acc);
-  rows_sum_squares(part, wss, ss);
+  const float inv = row_inv(p, seq);
+  const f4v acc = split_product<kH, kQkvSplit>(ring, p.gained, [&](int j) {
+    return wqkv + static_cast<size_t>(head * kHeadDim + (j < 8 ? i0 + j : kRotary + i0 + j - 8)) * kH;
+  });
   float v = tile_reduce<kWavesPerBlock>(acc, red);
-  if (!split_gather<kQkvSplit, true>(v, ss, p.split, p.counters + kCntQkv, tile)) return;
+  if (!split_gather<kQkvSplit>(v, p.split, p.counters + kCntQkv, tile)) return;
   // Epilogue over the 256 tile elements.
-  const float v0 = v;
-  v = v0 * rsqrtf(ss[seq] / static_cast<float>(kH) + p.eps) + bias;
+  v = v * inv + bias;
   const float other = __shfl_xor(v, 8, kWave);
   if (seq >= p.rows) return;
   const uint32_t slot = p.slot[seq];
@@ -306,23 +317,6 @@ __global__ __launch_bounds__(kBlock) void batch_qkv_kernel(BatchLaunch p, const 
     float *vc = kv_rows(p.v_cache, slot, layer, p.layers, p.capacity, kv_dim);
     vc[static_cast<size_t>(pos) * kv_dim + (head - p.nq - p.nkv) * kHeadDim + d] = v;
   }
-}
-
-// Sum / max over the 16 lanes of a DPP row (lanes 16q .. 16q+15); every
-// lane of the row receives the result.
-__device__ __forceinline__ float row16_sum(float v) {
-  v += dpp<kDppXor1>(v);
-  v += dpp<kDppXor2>(v);
-  v += dpp<kDppHalfMirror>(v);
-  v += dpp<kDppMirror>(v);
-  return v;
-}
-__device__ __forceinline__ float row16_max(float v) {
-  v = fmaxf(v, dpp<kDppXor1>(v));
-  v = fmaxf(v, dpp<kDppXor2>(v));
-  v = fmaxf(v, dpp<kDppHalfMirror>(v));
-  v = fmaxf(v, dpp<kDppMirror>(v));
-  return v;
 }
 
 // GQA decode attention on the matrix cores: workgroup (chunk, KV group g,
@@ -512,67 +506,40 @@ __global__ __launch_bounds__(kBlock) void batch_attn_kernel(BatchLaunch p, int l
 }
 
 // hidden[b][row] += Wo[row] . attn[b] for the 16 rows of tile blockIdx.x;
-// K = 896 split over kOSplit workgroups (two: 112 workgroups instead of 56,
-// 8.0 against 8.8 us per layer in a same-box A/B).
-#ifndef QD_BATCH_O_SPLIT
-#define QD_BATCH_O_SPLIT 2
-#endif
-constexpr int kOSplit = QD_BATCH_O_SPLIT;
-__global__ __launch_bounds__(kBlock) void batch_oproj_kernel(BatchLaunch p,
-                                                             const float *__restrict__ wo) {
-  constexpr int kSteps = kH / kStep / kWavesPerBlock / kOSplit;  // 7
+// K = 896 split over kOSplit workgroups (two: 112 workgroups instead of 56).
+constexpr int kOSplit = 2;
+__global__ __launch_bounds__(kBlock) void batch_oproj_kernel(BatchLaunch p, const float *__restrict__ wo,
+                                                             const float *__restrict__ next_gain) {
+  __shared__ __attribute__((aligned(16))) float ring[kWavesPerBlock][kRingFloats];
   __shared__ float red[kWavesPerBlock][4][kWave];
-  const int tile = blockIdx.x;
-  const int n0 = tile * 16;
-  const int kbase = (blockIdx.y * kWavesPerBlock + wave_id()) * kSteps * kStep;
-  float4 wv[kSteps], xa[kSteps];
-  load_weights<kSteps>(wo + static_cast<size_t>(n0 + tile_col()) * kH, kbase, wv);
-  load_operand<kSteps, kH>(p.attn, p.rows, kbase, xa);
-  issue_fence();
-  f4v acc = {0.f, 0.f, 0.f, 0.f};
-  acc = tile_mfma<kSteps>(xa, wv, acc);
+  const int tile = blockIdx.x, n0 = tile * 16;
+  const f4v acc = split_product<kH, kOSplit>(ring, p.attn, [&](int j) { return wo + static_cast<size_t>(n0 + j) * kH; });
   float v = tile_reduce<kWavesPerBlock>(acc, red);
-  if (!split_gather<kOSplit, false>(v, nullptr, p.split, p.counters + kCntO, tile)) return;
-  const int t = threadIdx.x;
-  const int seq = tile_seq(t);
-  if (seq < p.rows) p.hidden[seq * kH + n0 + (t & 15)] += v;
+  const int t = threadIdx.x, seq = tile_seq(t);
+  const float gain = next_gain[n0 + (t & 15)];
+  if (!split_gather<kOSplit>(v, p.split, p.counters + kCntO, tile)) return;
+  put_hidden(p, seq, tile, p.hidden[seq * kH + n0 + (t & 15)] + v, gain);
 }
 
 // MLP RMSNorm + gate/up + SiLU: act[b][row] = silu(g) * u. Tile blockIdx.x
 // covers rows n0 .. n0 + 7 of the activation: tile column j < 8 is gate row
-// n0 + j and column j + 8 the up row n0 + j, so each lane streams one weight
-// row and the 608 tiles (of 57 KB each) spread evenly over the CUs. The up
+// n0 + j and column j + 8 the up row n0 + j, and the 608 tiles (of 57 KB each) spread evenly over the CUs. The up
 // sum crosses to its gate lane (column j + 8 -> j) by a lane exchange.
-__global__ __launch_bounds__(kBlock) void batch_gateup_kernel(BatchLaunch p,
-                                                              const float *__restrict__ gain,
-                                                              const float *__restrict__ wg,
+__global__ __launch_bounds__(kBlock) void batch_gateup_kernel(BatchLaunch p, const float *__restrict__ wg,
                                                               const float *__restrict__ wu) {
-  constexpr int kSteps = kH / kStep / kWavesPerBlock;  // 14
-  __shared__ float wss[kWavesPerBlock][16];
-  __shared__ float ss[16];
+  __shared__ __attribute__((aligned(16))) float ring[kWavesPerBlock][kRingFloats];
   __shared__ float red[kWavesPerBlock][4][kWave];
   const int n0 = blockIdx.x * 8;
-  const int kbase = wave_id() * kSteps * kStep;
-  const int col = tile_col();
-  const float *wrow = (col < 8 ? wg : wu) + static_cast<size_t>(n0 + (col & 7)) * kH;
-  float4 wv[kSteps], xa[kSteps];
-  load_weights<kSteps>(wrow, kbase, wv);
-  float4 gv[kSteps];
-  load_operand<kSteps, kH>(p.hidden, p.rows, kbase, xa);
-  load_gain<kSteps>(kbase, gain, gv);
-  issue_fence();
-  const float part = gain_operand<kSteps>(gv, xa);
-  f4v acc = {0.f, 0.f, 0.f, 0.f};
-  acc = tile_mfma<kSteps>(xa, wv, acc);
-  rows_sum_squares(part, wss, ss);
+  const int t = threadIdx.x;
+  const int seq = tile_seq(t);
+  const float inv = row_inv(p, seq);
+  const f4v acc = split_product<kH, 1>(
+      ring, p.gained, [&](int j) { return (j < 8 ? wg : wu) + static_cast<size_t>(n0 + (j & 7)) * kH; });
   const float v = tile_reduce<kWavesPerBlock>(acc, red);
   // Thread t < 256 holds (sequence tile_seq(t), column t & 15); its partner
   // column t ^ 8 sits in lane (t ^ 8) of the same wave.
   const float other = __shfl_xor(v, 8, kWave);
-  const int t = threadIdx.x;
-  const int seq = tile_seq(t);
-  if (t < 4 * kWave && (t & 15) < 8 && seq < p.rows) {
-    const float inv = rsqrtf(ss[seq] / static_cast<float>(kH) + p.eps);
+  if ((t & 15) < 8 && seq < p.rows) {
     const float g = v * inv, u = other * inv;
     p.act[seq * kI + n0 + (t & 7)] = g / (1.f + expf(-g)) * u;
   }
@@ -581,98 +548,150 @@ __global__ __launch_bounds__(kBlock) void batch_gateup_kernel(BatchLaunch p,
 // hidden[b][row] += Wd[row] . act[b]; K = 4864 split over kDownSplit
 // workgroups of four waves.
 constexpr int kDownSplit = 4;
-__global__ __launch_bounds__(kBlock) void batch_down_kernel(BatchLaunch p,
-                                                            const float *__restrict__ wd) {
-  constexpr int kSteps = kI / kStep / kWavesPerBlock / kDownSplit;  // 19
+__global__ __launch_bounds__(kBlock) void batch_down_kernel(BatchLaunch p, const float *__restrict__ wd,
+                                                            const float *__restrict__ next_gain) {
+  __shared__ __attribute__((aligned(16))) float ring[kWavesPerBlock][kRingFloats];
   __shared__ float red[kWavesPerBlock][4][kWave];
-  const int tile = blockIdx.x;
-  const int n0 = tile * 16;
-  const int kbase = (blockIdx.y * kWavesPerBlock + wave_id()) * kSteps * kStep;
-  float4 wv[kSteps], xa[kSteps];
-  load_weights<kSteps>(wd + static_cast<size_t>(n0 + tile_col()) * kI, kbase, wv);
-  load_operand<kSteps, kI>(p.act, p.rows, kbase, xa);
-  issue_fence();
-  f4v acc = {0.f, 0.f, 0.f, 0.f};
-  acc = tile_mfma<kSteps>(xa, wv, acc);
+  const int tile = blockIdx.x, n0 = tile * 16;
+  const f4v acc = split_product<kI, kDownSplit>(ring, p.act, [&](int j) { return wd + static_cast<size_t>(n0 + j) * kI; });
   float v = tile_reduce<kWavesPerBlock>(acc, red);
-  if (!split_gather<kDownSplit, false>(v, nullptr, p.split, p.counters + kCntDown, tile)) return;
-  const int t = threadIdx.x;
-  const int seq = tile_seq(t);
-  if (seq < p.rows) p.hidden[seq * kH + n0 + (t & 15)] += v;
+  const int t = threadIdx.x, seq = tile_seq(t);
+  const float gain = next_gain[n0 + (t & 15)];
+  if (!split_gather<kDownSplit>(v, p.split, p.counters + kCntDown, tile)) return;
+  put_hidden(p, seq, tile, p.hidden[seq * kH + n0 + (t & 15)] + v, gain);
 }
 
-// Final RMSNorm + tied LM head + per-workgroup top-1 of every batch row.
-// Workgroups loop over 16-row vocabulary tiles (grid stride); each wave
-// keeps its K quarter of the gain-scaled operand in registers and the next
-// tile's weights in flight while the current tile is reduced.
-__global__ __launch_bounds__(kBlock) void batch_lmhead_kernel(BatchLaunch p, BatchTail tl) {
-  constexpr int kSteps = kH / kStep / kWavesPerBlock;  // 14
-  __shared__ float wss[kWavesPerBlock][16];
-  __shared__ float ss[16];
-  __shared__ float red[2][kWavesPerBlock][4][kWave];
-  const int kbase = wave_id() * kSteps * kStep;
-  const int k0 = kbase + k_quad();
-  const int tiles = (tl.vocab + 15) / 16;
-  auto load_tile = [&](int tile, float4 (&wv)[kSteps]) {
-    const int r = min(tile * 16 + tile_col(), tl.vocab - 1);
-    const float *w = tl.head + static_cast<size_t>(r) * kH + k0;
+// Final RMSNorm + tied LM head + per-workgroup top-1 of every batch row. One
+// workgroup of eight waves per CU: the gain-scaled rows sit in LDS (57 KiB) as
+// the matrix operand of every wave; a wave streams whole vocabulary tiles of 16
+// rows on its own through a ring of kLmRing LDS slices (2 KiB each), with no
+// barrier and no sum across waves. 16 rows: 106 us for 545 MB (5.1 TB/s; a plain
+// copy reaches 5.2), against 125 with four-way split tiles through registers.
+constexpr int kLmWaves = 8, kLmThreads = kLmWaves * kWave;
+constexpr int kLmRing = 6, kLmSlice = 16 * kSlice;  // floats of a slice
+constexpr int kLmRow = kH + 4;  // LDS row stride: the 16 rows' reads on distinct banks
+__global__ __launch_bounds__(kLmThreads) void batch_lmhead_kernel(BatchLaunch p, BatchTail tl) {
+  __shared__ __attribute__((aligned(16))) float xs[16 * kLmRow];
+  __shared__ __attribute__((aligned(16))) float rings[kLmWaves][kLmRing * kLmSlice];
+  __shared__ float invs[16];
+  __shared__ float wv[kLmWaves][16];
+  __shared__ uint32_t wi[kLmWaves][16];
+  const int tiles = (tl.vocab + 15) / 16, stride = gridDim.x * kLmWaves;
+  const int n = tile_col(), lane = lane_id(), w = __builtin_amdgcn_readfirstlane(wave_id()), lg = lane >> 4;
+  for (int i = threadIdx.x; i < 16 * kH / 4; i += kLmThreads) {
+    const int b = i / (kH / 4), c = i % (kH / 4);
+    *reinterpret_cast<float4 *>(xs + b * kLmRow + 4 * c) =
+        b < p.rows ? ld4(p.gained + b * kH + 4 * c) : make_float4(0.f, 0.f, 0.f, 0.f);
+  }
+  if (threadIdx.x < 256) {
+    const float inv = row_inv(p, tile_seq(threadIdx.x));
+    if ((threadIdx.x & 15) == 0) invs[tile_seq(threadIdx.x)] = inv;
+  }
+  __syncthreads();
+  // This lane's sequences 4 lg + r: scale, logits row, running top-1.
+  float inv[4], best[4];
+  uint32_t best_i[4];
+  float *out[4];
 #pragma unroll
-    for (int s = 0; s < kSteps; ++s) wv[s] = ld_weight(reinterpret_cast<const float4 *>(w + kStep * s));
+  for (int r = 0; r < 4; ++r) {
+    const int seq = 4 * lg + r;
+    inv[r] = invs[seq];
+    best[r] = -INFINITY;
+    best_i[r] = UINT32_MAX;
+    out[r] = seq < p.rows ? tl.logits + static_cast<size_t>(p.slot[seq]) * tl.vocab : nullptr;
+  }
+  const float *ring = rings[w];
+  const uint32_t base = ring_address(ring);
+  const float *x = xs + n * kLmRow + 4 * lg;
+  constexpr int kSlices = kH / kSlice;  // 28 per tile
+  int tile = blockIdx.x + w * gridDim.x;
+  // The slices to fetch, kLmRing ahead of the one multiplied: next_slice of
+  // next_tile. Past the last tile the last one is fetched again, so that every
+  // slice is followed by the same number of DMAs.
+  int next_tile = tile, next_slice = 0;
+  const float *src[2];
+  auto aim = [&] {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int row = ring_row(i);
+      src[i] = tl.head + static_cast<size_t>(min(next_tile * 16 + row, tl.vocab - 1)) * kH + ring_piece(row);
+    }
   };
-  float4 wcur[kSteps];
-  int tile = blockIdx.x;
-  if (tile < tiles) load_tile(tile, wcur);
-  float4 xa[kSteps], gv[kSteps];
-  load_operand<kSteps, kH>(p.hidden, p.rows, kbase, xa);
-  load_gain<kSteps>(kbase, tl.final_norm, gv);
-  const float part = gain_operand<kSteps>(gv, xa);
-  rows_sum_squares(part, wss, ss);
-  const int t = threadIdx.x;
-  const int seq = tile_seq(t);
-  const float inv = rsqrtf(ss[seq] / static_cast<float>(kH) + p.eps);
-  float *out = seq < p.rows ? tl.logits + static_cast<size_t>(p.slot[seq]) * tl.vocab : nullptr;
-  float best = -INFINITY;
-  uint32_t best_i = UINT32_MAX;
-  for (int it = 0; tile < tiles; tile += gridDim.x, ++it) {
-    float4 wnext[kSteps];
-    const int next = tile + gridDim.x;
-    if (next < tiles) load_tile(next, wnext);
+  auto fetch = [&](int stage) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      ring_dma<true>(src[i], base + (stage * kLmSlice + i * 256) * 4);
+      src[i] += kSlice;
+    }
+    if (++next_slice == kSlices) {
+      next_slice = 0;
+      next_tile = next_tile + stride < tiles ? next_tile + stride : next_tile;
+      aim();
+    }
+  };
+  int stage = 0;
+  if (tile < tiles) {
+    aim();
+#pragma unroll
+    for (int d = 0; d < kLmRing; ++d) fetch(d);
+  }
+  for (; tile < tiles; tile += stride) {
     f4v acc = {0.f, 0.f, 0.f, 0.f};
+    for (int s = 0; s < kSlices; ++s) {
+      // (The logits' stores count too: a wait that finds them outstanding
+      // only waits for more.)
+      ring_wait<2 * (kLmRing - 1)>();
+      float4 w0, w1;
+      ring_read(ring + stage * kLmSlice, w0, w1);
+      const float4 x0 = ld4(x + s * kSlice), x1 = ld4(x + s * kSlice + 16);
+      acc = mfma4(x0, w0, acc);
+      acc = mfma4(x1, w1, acc);
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      fetch(stage);
+      stage = stage + 1 == kLmRing ? 0 : stage + 1;
+    }
+    const int row = tile * 16 + n;
 #pragma unroll
-    for (int s = 0; s < kSteps; ++s) acc = mfma4(xa[s], wcur[s], acc);
-    float (*rb)[4][kWave] = red[it & 1];
-#pragma unroll
-    for (int r = 0; r < 4; ++r) rb[wave_id()][r][lane_id()] = acc[r];
-    __syncthreads();
-    float v = 0.f;
-#pragma unroll
-    for (int u = 0; u < kWavesPerBlock; ++u) v += rb[u][t >> 6][t & 63];
-    v *= inv;
-    const int n = tile * 16 + (t & 15);
-    if (out && n < tl.vocab) {
-      out[n] = v;
-      if (better(v, static_cast<uint32_t>(n), best, best_i)) {
-        best = v;
-        best_i = static_cast<uint32_t>(n);
+    for (int r = 0; r < 4; ++r) {
+      const float v = acc[r] * inv[r];
+      if (out[r] && row < tl.vocab) {
+        out[r][row] = v;
+        if (better(v, static_cast<uint32_t>(row), best[r], best_i[r])) {
+          best[r] = v;
+          best_i[r] = static_cast<uint32_t>(row);
+        }
       }
     }
-#pragma unroll
-    for (int s = 0; s < kSteps; ++s) wcur[s] = wnext[s];
   }
-  // The 16 threads of a sequence are lanes q*16 .. q*16+15 of one wave.
+  ring_wait<0>();  // the ring's last fetches land before the workgroup goes
 #pragma unroll
-  for (int o = 1; o < 16; o <<= 1) {
-    const float ov = __shfl_xor(best, o, kWave);
-    const uint32_t oi = __shfl_xor(best_i, o, kWave);
-    if (better(ov, oi, best, best_i)) {
-      best = ov;
-      best_i = oi;
+  for (int r = 0; r < 4; ++r) {
+#pragma unroll
+    for (int o = 1; o < 16; o <<= 1) {
+      const float ov = __shfl_xor(best[r], o, kWave);
+      const uint32_t oi = __shfl_xor(best_i[r], o, kWave);
+      if (better(ov, oi, best[r], best_i[r])) {
+        best[r] = ov;
+        best_i[r] = oi;
+      }
+    }
+    if (n == 0) {
+      wv[w][4 * lg + r] = best[r];
+      wi[w][4 * lg + r] = best_i[r];
     }
   }
-  if ((t & 15) == 0 && seq < p.rows) {
-    tl.part_val[seq * kBatchLmParts + blockIdx.x] = best;
-    tl.part_idx[seq * kBatchLmParts + blockIdx.x] = best_i;
-  }
+  __syncthreads();
+  if (threadIdx.x >= p.rows) return;
+  float top = wv[0][threadIdx.x];
+  uint32_t top_i = wi[0][threadIdx.x];
+#pragma unroll
+  for (int u = 1; u < kLmWaves; ++u)
+    if (better(wv[u][threadIdx.x], wi[u][threadIdx.x], top, top_i)) {
+      top = wv[u][threadIdx.x];
+      top_i = wi[u][threadIdx.x];
+    }
+  tl.part_val[threadIdx.x * kBatchLmParts + blockIdx.x] = top;
+  tl.part_idx[threadIdx.x * kBatchLmParts + blockIdx.x] = top_i;
 }
 
 // Per batch row: reduces the top-1 partials and writes the slot's state as
@@ -757,7 +776,7 @@ size_t round256(size_t bytes) { return (bytes + 255) / 256 * 256; }
 
 size_t batch_workspace_bytes(int nq) {
   const size_t r = kBatchRows, qd = size_t(nq) * kHeadDim;
-  return round256(r * kH * 4) + 2 * round256(r * qd * 4) + round256(r * kI * 4) +
+  return 2 * round256(r * kH * 4) + round256(r * kBatchTiles * 4) + 2 * round256(r * qd * 4) + round256(r * kI * 4) +
          round256(r * nq * kAttnMaxChunks * kPartStride * 4) + round256(size_t(kBatchSplitFloats) * 4) +
          round256(size_t(kBatchCounters) * 4) + 2 * round256(r * kBatchLmParts * 4) + 2 * round256(r * 4);
 }
@@ -772,6 +791,8 @@ BatchWorkspace carve_batch_workspace(void *base, int nq) {
   const size_t r = kBatchRows, qd = size_t(nq) * kHeadDim;
   BatchWorkspace w{};
   w.hidden = static_cast<float *>(take(r * kH * 4));
+  w.gained = static_cast<float *>(take(r * kH * 4));
+  w.squares = static_cast<float *>(take(r * kBatchTiles * 4));
   w.q = static_cast<float *>(take(r * qd * 4));
   w.attn = static_cast<float *>(take(r * qd * 4));
   w.act = static_cast<float *>(take(r * kI * 4));
@@ -834,24 +855,24 @@ static bool batch_shape_ok(const BatchLaunch &b) {
          (b.nq + 2 * b.nkv) * 4 <= kCntO - kCntQkv;
 }
 
-hipError_t launch_batch_embed(hipStream_t s, const BatchLaunch &b, const float *embed, int vocab,
-                              Marker *m) {
+hipError_t launch_batch_embed(hipStream_t s, const BatchLaunch &b, const float *embed, const float *first_gain,
+                              int vocab, Marker *m) {
   if (!batch_shape_ok(b)) return hipErrorInvalidValue;
   for (int i = 0; i < b.rows; ++i)
     if (b.pos[i] >= static_cast<uint32_t>(b.capacity) || b.token[i] >= static_cast<uint32_t>(vocab))
       return hipErrorInvalidValue;
   Scope scope(m, kBEmbed);
-  batch_embed_kernel<<<b.rows, kBlock, 0, s>>>(b, embed, vocab);
+  batch_embed_kernel<<<b.rows, kBlock, 0, s>>>(b, embed, first_gain, vocab);
   return hipGetLastError();
 }
 
 hipError_t launch_batch_layer(hipStream_t s, const BatchLaunch &b, const LayerPtrs &w, int layer,
-                              Marker *m) {
+                              const float *next_gain, Marker *m) {
   if (!batch_shape_ok(b)) return hipErrorInvalidValue;
   {
     Scope scope(m, kBQkvRope);
     batch_qkv_kernel<<<dim3((b.nq + 2 * b.nkv) * 4, kQkvSplit), kBlock, 0, s>>>(
-        b, w.attn_norm, w.wqkv, w.bqkv, layer);
+        b, w.wqkv, w.bqkv, layer);
   }
   {
     Scope scope(m, kBAttn);
@@ -859,15 +880,15 @@ hipError_t launch_batch_layer(hipStream_t s, const BatchLaunch &b, const LayerPt
   }
   {
     Scope scope(m, kBOproj);
-    batch_oproj_kernel<<<dim3(kH / 16, kOSplit), kBlock, 0, s>>>(b, w.wo);
+    batch_oproj_kernel<<<dim3(kH / 16, kOSplit), kBlock, 0, s>>>(b, w.wo, w.mlp_norm);
   }
   {
     Scope scope(m, kBGateUp);
-    batch_gateup_kernel<<<kI / 8, kBlock, 0, s>>>(b, w.mlp_norm, w.wg, w.wu);
+    batch_gateup_kernel<<<kI / 8, kBlock, 0, s>>>(b, w.wg, w.wu);
   }
   {
     Scope scope(m, kBDown);
-    batch_down_kernel<<<dim3(kH / 16, kDownSplit), kBlock, 0, s>>>(b, w.wd);
+    batch_down_kernel<<<dim3(kH / 16, kDownSplit), kBlock, 0, s>>>(b, w.wd, next_gain);
   }
   return hipGetLastError();
 }
@@ -876,7 +897,7 @@ hipError_t launch_batch_tail(hipStream_t s, const BatchLaunch &b, const BatchTai
   if (!batch_shape_ok(b) || t.vocab <= 0) return hipErrorInvalidValue;
   {
     Scope scope(m, kBLmHead);
-    batch_lmhead_kernel<<<kBatchLmParts, kBlock, 0, s>>>(b, t);
+    batch_lmhead_kernel<<<kBatchLmParts, kLmThreads, 0, s>>>(b, t);
   }
   {
     Scope scope(m, kBArgmax);

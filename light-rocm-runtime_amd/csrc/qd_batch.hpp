@@ -15,7 +15,7 @@
 namespace qd {
 
 constexpr int kBatchRows = 16;      // sequences per launch (the MFMA M dimension)
-constexpr int kBatchLmParts = 512;  // LM-head workgroups = top-1 partials per sequence
+constexpr int kBatchLmParts = 256;  // LM-head workgroups = top-1 partials per sequence
 
 // Buffers and geometry of one batched step. Row b of every activation buffer
 // belongs to sequence slot slot[b], which consumes token[b] at KV position
@@ -29,6 +29,9 @@ struct BatchLaunch {
   uint32_t token[kBatchRows];
   SeqState *states;             // [max_batch]; the argmax kernel writes slot[b]'s
   float *hidden;                // [kBatchRows][896] residual stream
+  float *gained;                // [kBatchRows][896] hidden times the next norm's gain
+  float *squares;               // [kBatchRows][kBatchTiles] sums of squares of hidden's 16-column
+                                //   tiles (56; the places beyond stay zero)
   float *q;                     // [kBatchRows][nq * 64] rotated queries
   float *attn;                  // [kBatchRows][nq * 64]
   float *act;                   // [kBatchRows][4864]
@@ -47,11 +50,11 @@ struct BatchLaunch {
 };
 
 // Workspace sizes of BatchLaunch::split and ::counters.
-constexpr int kBatchSplitFloats = 4 * 128 * (256 + 16);
+constexpr int kBatchSplitFloats = 4 * 128 * 256;
+constexpr int kBatchTiles = 64;  // 16-column tiles of a hidden row (56), rounded up to whole 16s
 constexpr int kBatchCounters = 1024;
 
 struct BatchTail {
-  const float *final_norm;
   const float *head;     // [vocab, 896]
   float *logits;         // [max_batch][vocab]: batch row b writes the row of its slot, slot[b]
   float *part_val;       // [kBatchRows][kBatchLmParts]
@@ -66,6 +69,8 @@ struct BatchTail {
 // this order from one block, each region 256-byte aligned.
 struct BatchWorkspace {
   float *hidden;        // [kBatchRows][896]
+  float *gained;        // [kBatchRows][896]
+  float *squares;       // [kBatchRows][kBatchTiles], the last 8 of a row zero before a step
   float *q;             // [kBatchRows][nq * 64]
   float *attn;          // [kBatchRows][nq * 64]
   float *act;           // [kBatchRows][4864]
@@ -109,10 +114,12 @@ enum BatchKernelId : int {
 };
 const char *batch_kernel_name(int id);
 
-hipError_t launch_batch_embed(hipStream_t s, const BatchLaunch &b, const float *embed, int vocab,
-                              Marker *m = nullptr);
+// first_gain: layer 0's attention norm; next_gain: the norm after this layer
+// (the next layer's attention norm, the final norm after the last).
+hipError_t launch_batch_embed(hipStream_t s, const BatchLaunch &b, const float *embed, const float *first_gain,
+                              int vocab, Marker *m = nullptr);
 hipError_t launch_batch_layer(hipStream_t s, const BatchLaunch &b, const LayerPtrs &w, int layer,
-                              Marker *m = nullptr);
+                              const float *next_gain, Marker *m = nullptr);
 hipError_t launch_batch_tail(hipStream_t s, const BatchLaunch &b, const BatchTail &t,
                              Marker *m = nullptr);
 

@@ -177,7 +177,7 @@ struct qd_engine {
   // Batched-step workspace (allocated on the first batched step): rows of
   // up to kBatchRows sequences, attention and split-K partials, arrival
   // counters, the LM-head top-1 partials and each row's greedy result.
-  float *bt_h = nullptr, *bt_q = nullptr, *bt_attn = nullptr, *bt_act = nullptr,
+  float *bt_h = nullptr, *bt_hg = nullptr, *bt_sq = nullptr, *bt_q = nullptr, *bt_attn = nullptr, *bt_act = nullptr,
         *bt_part = nullptr, *bt_split = nullptr, *bt_val = nullptr, *bt_top = nullptr;
   uint32_t *bt_idx = nullptr, *bt_counters = nullptr, *bt_token = nullptr;
   uint32_t *h_bt_out = nullptr;  // pinned [max_batch] tokens then [max_batch] top logits
@@ -406,7 +406,8 @@ struct qd_engine {
   qd::BatchLaunch batch_args(const uint32_t *slots, const uint32_t *tokens, int rows) {
     if (!bt_h) {
       const size_t r = qd::kBatchRows;
-      bt_h = alloc<float>(r * H);
+      bt_hg = alloc<float>(r * H);
+      bt_sq = alloc<float>(r * qd::kBatchTiles);
       bt_q = alloc<float>(r * QD);
       bt_attn = alloc<float>(r * QD);
       bt_act = alloc<float>(r * I);
@@ -417,10 +418,12 @@ struct qd_engine {
       bt_idx = alloc<uint32_t>(r * qd::kBatchLmParts);
       bt_token = alloc<uint32_t>(B);
       bt_top = alloc<float>(B);
+      check(hipMemsetAsync(bt_sq, 0, r * qd::kBatchTiles * sizeof(float), stream), "memset");
       check(hipMemsetAsync(bt_counters, 0, qd::kBatchCounters * sizeof(uint32_t), stream), "memset");
       check(hipHostMalloc(reinterpret_cast<void **>(&h_bt_out), 2 * B * sizeof(uint32_t),
                           hipHostMallocDefault),
             "hipHostMalloc");
+      bt_h = alloc<float>(r * H);
     }
     qd::BatchLaunch b{};
     b.rows = rows;
@@ -431,6 +434,8 @@ struct qd_engine {
     }
     b.states = states;
     b.hidden = bt_h;
+    b.gained = bt_hg;
+    b.squares = bt_sq;
     b.q = bt_q;
     b.attn = bt_attn;
     b.act = bt_act;
@@ -454,7 +459,6 @@ struct qd_engine {
   // qd_read_logits finds them), greedy results to bt_token/bt_top.
   qd::BatchTail batch_tail(size_t first) const {
     qd::BatchTail t{};
-    t.final_norm = final_norm;
     t.head = lm_head;
     t.logits = logits;
     t.part_val = bt_val;
@@ -468,11 +472,16 @@ struct qd_engine {
   // Embedding + every layer + LM head + argmax of one batch group (states
   // and slot list already on the device).
   void enqueue_batch(const qd::BatchLaunch &b, size_t first, qd::Marker *m = nullptr) {
-    check(qd::launch_batch_embed(stream, b, embed, static_cast<int>(V), m), "batch embed launch");
+    enqueue_batch(b, batch_tail(first), m);
+  }
+  void enqueue_batch(const qd::BatchLaunch &b, const qd::BatchTail &t, qd::Marker *m = nullptr) {
+    check(qd::launch_batch_embed(stream, b, embed, layers[0].attn_norm, static_cast<int>(V), m),
+          "batch embed launch");
     for (size_t l = 0; l < L; ++l)
-      check(qd::launch_batch_layer(stream, b, layers[l], static_cast<int>(l), m),
+      check(qd::launch_batch_layer(stream, b, layers[l], static_cast<int>(l),
+                                   l + 1 < L ? layers[l + 1].attn_norm : final_norm, m),
             "batch layer launch");
-    check(qd::launch_batch_tail(stream, b, batch_tail(first), m), "batch tail launch");
+    check(qd::launch_batch_tail(stream, b, t, m), "batch tail launch");
   }
 
   // Floating-point operations of one launch of `kernel` (multiply-add = 2).
@@ -1704,6 +1713,8 @@ qd_status qd_step_batch_noalloc(qd_engine *e, uint32_t n_seq, const uint32_t *se
     }
     b.states = e->states;
     b.hidden = w.hidden;
+    b.gained = w.gained;
+    b.squares = w.squares;
     b.q = w.q;
     b.attn = w.attn;
     b.act = w.act;
@@ -1720,7 +1731,6 @@ qd_status qd_step_batch_noalloc(qd_engine *e, uint32_t n_seq, const uint32_t *se
     b.nkv = static_cast<int>(e->NKV);
     b.eps = e->cfg.rms_eps;
     qd::BatchTail t{};
-    t.final_norm = e->final_norm;
     t.head = e->lm_head;
     t.logits = e->logits;
     t.part_val = w.part_val;
@@ -1729,12 +1739,10 @@ qd_status qd_step_batch_noalloc(qd_engine *e, uint32_t n_seq, const uint32_t *se
     t.out_top = w.out_top;
     t.vocab = static_cast<int>(e->V);
     // The workspace keeps the last call's contents: the arrival counters
-    // start at zero (a fill kernel, no memset node).
+    // start at zero (a fill kernel, no memset node). The places of `squares`
+    // past the 56 tiles are never written: zero as the array was.
     check(qd::launch_batch_clear_counters(e->stream, w.counters), "counter clear");
-    check(qd::launch_batch_embed(e->stream, b, e->embed, static_cast<int>(e->V)), "batch embed launch");
-    for (size_t l = 0; l < e->L; ++l)
-      check(qd::launch_batch_layer(e->stream, b, e->layers[l], static_cast<int>(l)), "batch layer launch");
-    check(qd::launch_batch_tail(e->stream, b, t), "batch tail launch");
+    e->enqueue_batch(b, t);
     if (greedy)
       check(hipMemcpyAsync(greedy, w.out_token, n_seq * 4, hipMemcpyDeviceToHost, e->stream), "D2H");
     if (logits)
