@@ -251,6 +251,21 @@ __device__ __forceinline__ float *kv_rows(float *cache, uint32_t slot, int layer
   return cache + (static_cast<size_t>(slot) * layers + layer) * capacity * kv_dim;
 }
 
+// Rows of a K or V cache through a buffer descriptor that ends with the last
+// one wanted: a load past it returns zeros and touches no memory.
+struct KvRows {
+  __amdgpu_buffer_rsrc_t r;
+  __device__ __forceinline__ KvRows(const float *base, uint32_t bytes)
+      : r(__builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(base), 0, static_cast<int>(bytes), kRsrcWord3)) {}
+  __device__ __forceinline__ float ld(uint32_t i) const {
+    return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, i * 4u, 0, 0));
+  }
+  __device__ __forceinline__ float4 ld4(uint32_t i) const {
+    const f32x4 v = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(r, i * 4u, 0, 0));
+    return make_float4(v[0], v[1], v[2], v[3]);
+  }
+};
+
 // ---- kernels --------------------------------------------------------------------
 
 __global__ __launch_bounds__(kBlock) void batch_embed_kernel(BatchLaunch p, const float *__restrict__ emb,
@@ -322,47 +337,80 @@ __global__ __launch_bounds__(kBlock) void batch_qkv_kernel(BatchLaunch p, const 
 // GQA decode attention on the matrix cores: workgroup (chunk, KV group g,
 // batch row b) serves all query heads of the group (up to 16), so every K/V
 // row of the chunk is read once. Waves take 16-position tiles (wave w: tile
-// w of each 64-position pass). Per tile:
+// w of each 128-position pass). Per tile:
 //   S[head][pos] = (Q / 8) . K^T    16x16x4 MFMAs, lane l supplies
 //                                   Q[head l%16] and K[pos l%16] at dims
 //                                   16 s + 4 (l/16) + c (float4 loads)
 //   online softmax per head row     (S register r of lane l is head
 //                                   4 (l/16) + r, position l%16: row
 //                                   reductions over the 16-lane DPP rows)
-//   O[head][d] += P . V             P and the V tile go through the wave's
-//                                   LDS to become MFMA A / B operands.
-// The four wave partials are merged into one record (m, l, acc[64]) per
-// head; the last chunk of (b, g) to finish merges all chunks (the same
-// merge as attn_merge) into attn[b][h*64 + d]. Q is scaled by
-// kScoreScaleLog2 = log2(e) / sqrt(64), so scores and maxima are in base-2
-// units and every softmax exponential is one v_exp_f32 (2^x).
+//   O[head][d] += P . V             P goes through the wave's LDS to become
+//                                   the A operand; V is loaded as B operands.
+// The wave partials are merged into one record (m, l, acc[64]) per head; the
+// last chunk of (b, g) to finish merges all chunks (the same merge as
+// attn_merge) into attn[b][h*64 + d]. Q is scaled by kScoreScaleLog2 =
+// log2(e) / sqrt(64), so scores and maxima are in base-2 units and every
+// softmax exponential is one v_exp_f32 (2^x).
+//
+// Bound by latency (a layer's K/V rows of 16 contexts to 2,048, 19 MB, stream
+// in 3 us): one round trip for the K and V of a wave's only tile, which are
+// requested before anything else, then the record and counter round trips.
+// Per layer 18.0 -> 14.8 us at 16 rows (five rows, contexts to 300: 11.3 ->
+// 10.7) against chunks of four waves that passed over up to three tiles each,
+// V through LDS.
+constexpr int kAttnWaves = 8, kAttnThreads = kAttnWaves * kWave, kAttnTileRows = 16;
 struct GqaLds {
-  float ps[kWavesPerBlock][16][17];   // P tile [head][pos]
-  float vs[kWavesPerBlock][16][68];   // V tile [pos][dim]
-  float wm[kWavesPerBlock][16];
-  float wl[kWavesPerBlock][16];
-  float wo[kWavesPerBlock][16][65];   // wave partial O [head][dim]
+  float ps[kAttnWaves][16][17];   // P tile [head][pos]
+  float wm[kAttnWaves][16];
+  float wl[kAttnWaves][16];
+  float wo[kAttnWaves][16][65];   // wave partial O [head][dim]
 };
 
-__global__ __launch_bounds__(kBlock) void batch_attn_kernel(BatchLaunch p, int layer) {
+// Positions per chunk: one tile per wave while kAttnMaxChunks such chunks hold
+// the context (2,048 positions), then the fewest tiles that hold it.
+__device__ __forceinline__ int batch_chunk_len(int length) {
+  return max(attn_chunk_len(length, kAttnMaxChunks, kAttnTileRows), kAttnWaves * kAttnTileRows);
+}
+
+__global__ __launch_bounds__(kAttnThreads, 4) void batch_attn_kernel(BatchLaunch p, int layer) {
   __shared__ GqaLds sh;
   __shared__ uint32_t last;
   const int b = blockIdx.z, g = blockIdx.y, chunk = blockIdx.x;
   const uint32_t slot = p.slot[b];
   const int position = static_cast<int>(p.pos[b]);
   const int length = position + 1;
-  const int chunks = attn_chunks(length);
+  const int chunk_len = batch_chunk_len(length);
+  const int chunks = (length + chunk_len - 1) / chunk_len;
   if (chunk >= chunks) return;
-  const int chunk_len = attn_chunk_len(length);
   const int begin = chunk * chunk_len;
   const int end = min(length, begin + chunk_len);
   const int group = p.nq / p.nkv;
   const int kv_dim = p.nkv * kHeadDim;
-  const float *kb = kv_rows(p.k_cache, slot, layer, p.layers, p.capacity, kv_dim) + g * kHeadDim;
-  const float *vb = kv_rows(p.v_cache, slot, layer, p.layers, p.capacity, kv_dim) + g * kHeadDim;
-  const int w = wave_id(), col = tile_col(), quad = lane_id() >> 4;
+  const int w = __builtin_amdgcn_readfirstlane(wave_id()), col = tile_col(), quad = lane_id() >> 4;
   const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
 
+  // The chunk's K and V rows of the group: the descriptor ends after row
+  // end - 1, and rows past it read as zeros.
+  const size_t first = static_cast<size_t>(begin) * kv_dim + g * kHeadDim;
+  const uint32_t bytes = ((end - begin) * kv_dim - g * kHeadDim) * sizeof(float);
+  const KvRows kr(kv_rows(p.k_cache, slot, layer, p.layers, p.capacity, kv_dim) + first, bytes);
+  const KvRows vr(kv_rows(p.v_cache, slot, layer, p.layers, p.capacity, kv_dim) + first, bytes);
+  float4 kc[4];
+  float vc[4][4];
+  auto load_k = [&](int row) {
+#pragma unroll
+    for (int s = 0; s < 4; ++s) kc[s] = kr.ld4((row + col) * kv_dim + 16 * s + 4 * quad);
+  };
+  auto load_v = [&](int row) {
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+#pragma unroll
+      for (int n = 0; n < 4; ++n) vc[s][n] = vr.ld((row + 4 * s + quad) * kv_dim + 16 * n + col);
+  };
+  const int rows = end - begin;
+  int row = kAttnTileRows * w;
+  load_k(row);
+  load_v(row);
   float4 qa[4];
   if (col < group) {
     const float *qr = p.q + b * (p.nq * kHeadDim) + (g * group + col) * kHeadDim + 4 * quad;
@@ -376,20 +424,6 @@ __global__ __launch_bounds__(kBlock) void batch_attn_kernel(BatchLaunch p, int l
 #pragma unroll
     for (int s = 0; s < 4; ++s) qa[s] = zero;
   }
-  auto load_tile = [&](int p0, float4 (&kr)[4], float4 (&vr)[4]) {
-    const int pos = p0 + col;
-    if (pos < end) {
-      const size_t off = static_cast<size_t>(pos) * kv_dim + 4 * quad;
-#pragma unroll
-      for (int s = 0; s < 4; ++s) {
-        kr[s] = ld4(kb + off + 16 * s);
-        vr[s] = ld4(vb + off + 16 * s);
-      }
-    } else {
-#pragma unroll
-      for (int s = 0; s < 4; ++s) kr[s] = vr[s] = zero;
-    }
-  };
 
   float m[4], lsum[4];
   f4v o[4];
@@ -399,19 +433,13 @@ __global__ __launch_bounds__(kBlock) void batch_attn_kernel(BatchLaunch p, int l
     lsum[r] = 0.f;
     o[r] = f4v{0.f, 0.f, 0.f, 0.f};
   }
-  float4 kc[4], vc[4];
-  load_tile(begin + 16 * w, kc, vc);
-  for (int base = begin; base < end; base += kAttnPass) {
-    const int p0 = base + 16 * w;
-    float4 kn[4], vn[4];
-    if (base + kAttnPass < end) load_tile(p0 + kAttnPass, kn, vn);
-#pragma unroll
-    for (int s = 0; s < 4; ++s)
-      *reinterpret_cast<float4 *>(&sh.vs[w][col][16 * s + 4 * quad]) = vc[s];
+  for (; row < rows; row += kAttnTileRows * kAttnWaves) {
+    const bool more = row + kAttnTileRows * kAttnWaves < rows;
     f4v sacc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int s = 0; s < 4; ++s) sacc = mfma4(qa[s], kc[s], sacc);
-    const bool valid = p0 + col < end;
+    if (more) load_k(row + kAttnTileRows * kAttnWaves);
+    const bool valid = row + col < rows;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const float sv = valid ? sacc[r] : -INFINITY;
@@ -424,20 +452,15 @@ __global__ __launch_bounds__(kBlock) void batch_attn_kernel(BatchLaunch p, int l
       for (int n = 0; n < 4; ++n) o[n][r] *= corr;
       sh.ps[w][4 * quad + r][col] = pv;
     }
-    // The wave's own LDS tiles: LDS operations of a wave complete in order.
+    // The wave's own LDS tile: LDS operations of a wave complete in order.
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
       const float a = sh.ps[w][col][4 * s + quad];
 #pragma unroll
       for (int n = 0; n < 4; ++n)
-        o[n] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, sh.vs[w][4 * s + quad][16 * n + col], o[n],
-                                                     0, 0, 0);
+        o[n] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, vc[s][n], o[n], 0, 0, 0);
     }
-#pragma unroll
-    for (int s = 0; s < 4; ++s) {
-      kc[s] = kn[s];
-      vc[s] = vn[s];
-    }
+    if (more) load_v(row + kAttnTileRows * kAttnWaves);
   }
   // Wave partials -> one record per head of the group.
 #pragma unroll
@@ -452,14 +475,14 @@ __global__ __launch_bounds__(kBlock) void batch_attn_kernel(BatchLaunch p, int l
   __syncthreads();
   const Coherent recs(p.part + (static_cast<size_t>(b) * p.nq + g * group) * kAttnMaxChunks * kPartStride,
                       group * kAttnMaxChunks * kPartStride * sizeof(float));
-  for (int i = threadIdx.x; i < group * kHeadDim; i += kBlock) {
+  for (int i = threadIdx.x; i < group * kHeadDim; i += kAttnThreads) {
     const int h = i / kHeadDim, d = i % kHeadDim;
     float mx = -INFINITY;
 #pragma unroll
-    for (int v = 0; v < kWavesPerBlock; ++v) mx = fmaxf(mx, sh.wm[v][h]);
+    for (int v = 0; v < kAttnWaves; ++v) mx = fmaxf(mx, sh.wm[v][h]);
     float lt = 0.f, a = 0.f;
 #pragma unroll
-    for (int v = 0; v < kWavesPerBlock; ++v) {
+    for (int v = 0; v < kAttnWaves; ++v) {
       const float f = sh.wm[v][h] == -INFINITY ? 0.f : exp2_fast(sh.wm[v][h] - mx);
       lt = fmaf(f, sh.wl[v][h], lt);
       a = fmaf(f, sh.wo[v][h][d], a);
@@ -477,7 +500,7 @@ __global__ __launch_bounds__(kBlock) void batch_attn_kernel(BatchLaunch p, int l
   if (threadIdx.x == 0) last = atomicAdd(cnt, 1u) == static_cast<uint32_t>(chunks - 1);
   __syncthreads();
   if (!last) return;
-  for (int i = threadIdx.x; i < group * kHeadDim; i += kBlock) {
+  for (int i = threadIdx.x; i < group * kHeadDim; i += kAttnThreads) {
     const int h = i / kHeadDim, d = i % kHeadDim;
     const uint32_t head_rec = h * kAttnMaxChunks * kPartStride;
     // Every chunk's (m, l, acc_d) is requested before any is used.
@@ -876,7 +899,7 @@ hipError_t launch_batch_layer(hipStream_t s, const BatchLaunch &b, const LayerPt
   }
   {
     Scope scope(m, kBAttn);
-    batch_attn_kernel<<<dim3(kAttnMaxChunks, b.nkv, b.rows), kBlock, 0, s>>>(b, layer);
+    batch_attn_kernel<<<dim3(kAttnMaxChunks, b.nkv, b.rows), kAttnThreads, 0, s>>>(b, layer);
   }
   {
     Scope scope(m, kBOproj);

@@ -15,8 +15,8 @@ constexpr int kMaxGroup = 16;          // query heads per KV head
 
 // Split-KV attention geometry (qd_attention.hpp): chunks are whole grains
 // of positions, at most kAttnMaxChunks per head; a partial record is (m, l,
-// acc[64]). The batched kernel cuts chunks in passes of 64 (16 positions per
-// wave of its four-wave unit); the batch-1 decode paths by decode_chunk_len.
+// acc[64]). The batched kernel cuts chunks by batch_chunk_len, the batch-1
+// decode paths by decode_chunk_len.
 constexpr int kAttnPass = 64;
 constexpr int kAttnGrain = 16;
 constexpr int kAttnMaxChunks = 16;
@@ -24,15 +24,10 @@ constexpr int kPartStride = kHeadDim + 2;
 
 // Chunks of a context of `length` positions split `parts` ways (parts <=
 // kAttnMaxChunks): whole grains per chunk.
-__host__ __device__ inline int attn_chunk_len(int length, int parts = kAttnMaxChunks, int grain = kAttnPass) {
+__host__ __device__ inline int attn_chunk_len(int length, int parts, int grain) {
   const int grains = (length + grain - 1) / grain;
   const int per_chunk = (grains + parts - 1) / parts;
   return per_chunk * grain;
-}
-
-__host__ __device__ inline int attn_chunks(int length, int parts = kAttnMaxChunks, int grain = kAttnPass) {
-  const int cl = attn_chunk_len(length, parts, grain);
-  return (length + cl - 1) / cl;
 }
 
 // Chunk length of the batch-1 decode paths, a function of the context alone so

@@ -57,3 +57,23 @@ def test_batch_rows_match_oracle(pair, rows):
         assert int(greedy[i]) == int(np.argmax(logits[i]))
         gk, gv = eng.read_kv(s, LAYERS - 1, len(prompts[s]) - 1, 1)
         assert rel_err(gk[0], k) <= RTOL and rel_err(gv[0], v) <= RTOL
+
+
+def test_batch_attention_chunk_edges():
+    """Contexts at the edges of a wave's 16 positions, a chunk's 128 and the
+    longest split into chunks of 128 (2,048), each against the batch-1 step."""
+    lengths = [1, 15, 16, 17, 127, 128, 129, 143, 144, 255, 257, 1025, 2047, 2048, 2049, 2299]
+    eng = qd.Engine(layers=LAYERS, vocab=1003, capacity=2300, max_batch=len(lengths))
+    eng.load_synthetic(3)
+    prompt = qo.fill_tokens(2300, 3, 0x600000, 1003)
+    slots = list(range(len(lengths)))
+    for s, n in zip(slots, lengths):
+        eng.kv_reset(s, 0)
+        eng.prefill(s, prompt[:n], want_logits=False)
+    print("batch over", lengths, flush=True)
+    _, logits = eng.step_batch(slots, [int(prompt[n]) for n in lengths])
+    for s, n in zip(slots, lengths):
+        eng.kv_reset(s, n)
+        _, _, single = eng.step(s, int(prompt[n]))
+        assert rel_err(logits[s], single) <= RTOL, n
+    eng.close()
