@@ -35,6 +35,7 @@ namespace {
 
 constexpr uint32_t kAbiVersion = 4;
 constexpr int kLmHeadParts = 1024;  // LM-head workgroups = top-1 partials
+constexpr size_t kExportBytes = 256 * 1024;  // below, the runtime's copy is as fast as read_rows' export
 
 thread_local std::string g_error;
 
@@ -188,6 +189,11 @@ struct qd_engine {
 
   qd::SeqState *h_states = nullptr;  // pinned [max_batch]
   uint32_t *h_tokens = nullptr;      // pinned [capacity]
+  // Logits rows on their way to the caller (read_rows); nullptr if the pinned
+  // memory was refused. Then one flag per piece of a row; epoch: the last export.
+  float *h_rows = nullptr;           // pinned [min(max_batch, kExportRows)][vocab]
+  uint32_t *h_rows_flags = nullptr;  // pinned
+  uint32_t h_rows_epoch = 0;
   uint32_t *h_error = nullptr;       // pinned [2]: a resident launch's error word, the sticky one
   std::vector<uint32_t> positions;   // host mirror of each slot's position
   bool loaded = false;
@@ -206,6 +212,8 @@ struct qd_engine {
     if (h_states) (void)hipHostFree(h_states);
     if (h_tokens) (void)hipHostFree(h_tokens);
     if (h_error) (void)hipHostFree(h_error);
+    if (h_rows) (void)hipHostFree(h_rows);
+    if (h_rows_flags) (void)hipHostFree(h_rows_flags);
     if (h_bt_out) (void)hipHostFree(h_bt_out);
     if (ev_begin) (void)hipEventDestroy(ev_begin);
     if (ev_end) (void)hipEventDestroy(ev_end);
@@ -743,6 +751,68 @@ struct qd_engine {
       resident_status(err);
     }
   }
+  size_t export_rows() const { return std::min<size_t>(B, qd::kExportRows); }
+  void alloc_export() {
+    const size_t flags = export_rows() * qd::export_pieces(V) * sizeof(uint32_t);
+    if (hipHostMalloc(reinterpret_cast<void **>(&h_rows), export_rows() * V * 4, hipHostMallocDefault) != hipSuccess ||
+        hipHostMalloc(reinterpret_cast<void **>(&h_rows_flags), flags, hipHostMallocDefault) != hipSuccess) {
+      (void)hipGetLastError();
+      if (h_rows) (void)hipHostFree(h_rows);
+      h_rows = nullptr;
+      h_rows_flags = nullptr;
+      return;
+    }
+    std::memset(h_rows_flags, 0, flags);
+  }
+  // Rows slots[0 .. n) of src ([..][vocab]) to out, after the work queued so
+  // far; the caller synchronises. A copy into pageable memory goes through the
+  // runtime's staging at 17 GB/s (16 rows 563 us, one 33), so where `out` is
+  // that, a kernel writes the rows to pinned memory over the link (50 GB/s) and
+  // this thread copies each piece on as it arrives (248 and 26 us). Pages of
+  // `out` that the process has never touched cost 0.4 us each: they are touched
+  // while the GPU works, not in the copy.
+  void read_rows(const float *src, const uint32_t *slots, size_t n, float *out) {
+    hipPointerAttribute_t attr{};
+    bool pageable = false;
+    if (h_rows && n * V * 4 >= kExportBytes) {
+      const hipError_t err = hipPointerGetAttributes(&attr, out);
+      pageable = err == hipErrorInvalidValue || (err == hipSuccess && attr.type == hipMemoryTypeUnregistered);
+      if (err != hipSuccess) (void)hipGetLastError();
+    }
+    if (!pageable) {
+      for (size_t i = 0; i < n; ++i)
+        check(hipMemcpyAsync(out + i * V, src + size_t(slots[i]) * V, V * 4, hipMemcpyDeviceToHost, stream), "D2H");
+      return;
+    }
+    const size_t pieces = qd::export_pieces(V);
+    const auto landed = [&](size_t i) { return __atomic_load_n(h_rows_flags + i, __ATOMIC_ACQUIRE) == h_rows_epoch; };
+    size_t touched = 0;
+    for (size_t first = 0; first < n; first += export_rows()) {
+      const size_t rows = std::min(export_rows(), n - first);
+      qd::ExportRows which{};
+      std::copy(slots + first, slots + first + rows, which.slot);
+      ++h_rows_epoch;
+      check(qd::launch_export_rows(stream, src, V, which, int(rows), h_rows, h_rows_flags, h_rows_epoch), "export");
+      for (; touched < n * V && !landed(0); touched += 1024) {
+        volatile float *page = out + touched;
+        *page = *page;
+      }
+      for (size_t i = 0; i < rows * pieces; ++i) {
+        for (uint32_t spin = 1; !landed(i); ++spin) {
+          __builtin_ia32_pause();
+          if (spin % 4096 != 0) continue;
+          // Every piece has landed once the stream is idle, or none will.
+          const hipError_t err = hipStreamQuery(stream);
+          if (err == hipErrorNotReady) continue;
+          check(err, "hipStreamQuery");
+          if (!landed(i)) fail(QD_ERROR_DEVICE_FAULT, "logits copy incomplete");
+        }
+        const size_t begin = i / pieces * V + i % pieces * qd::kExportPiece;
+        const size_t len = std::min<size_t>(qd::kExportPiece, V - i % pieces * qd::kExportPiece);
+        std::memcpy(out + first * V + begin, h_rows + begin, len * 4);
+      }
+    }
+  }
   // Decoder layers [first, first + count) of slot seq on its device hidden
   // vector at its position: one layers-only resident launch, or the stream
   // kernels; the two compute the same values bit for bit.
@@ -952,6 +1022,7 @@ qd_status qd_engine_create(const qd_config *config, qd_engine **out) {
           "hipHostMalloc");
     check(hipHostMalloc(reinterpret_cast<void **>(&e->h_error), 2 * sizeof(uint32_t), hipHostMallocDefault),
           "hipHostMalloc");
+    e->alloc_export();
     e->positions.assign(e->B, 0);
     e->build_rope_tables(c.rope_theta);
 
@@ -1403,7 +1474,7 @@ qd_status qd_tail(qd_engine *e, uint32_t seq, float *logits_out, uint32_t *greed
     check(hipMemcpyAsync(&e->h_states[seq], e->states + seq, sizeof(qd::SeqState),
                          hipMemcpyDeviceToHost, e->stream), "D2H");
     if (logits_out)
-      check(hipMemcpyAsync(logits_out, dev_logits, e->V * 4, hipMemcpyDeviceToHost, e->stream), "D2H");
+      e->read_rows(e->logits, &seq, 1, logits_out);
     e->sync();
     e->positions[seq] += 1;
     if (greedy) *greedy = e->h_states[seq].token;
@@ -1417,8 +1488,7 @@ qd_status qd_read_logits(qd_engine *e, uint32_t seq, float *out, size_t count) {
     e->check_seq(seq);
     if (count != e->V) fail(QD_ERROR_INVALID_ARGUMENT, "logits have %zu elements, caller asked %zu", e->V, count);
     e->set_device();
-    check(hipMemcpyAsync(out, e->logits + size_t(seq) * e->V, e->V * 4, hipMemcpyDeviceToHost, e->stream),
-          "D2H");
+    e->read_rows(e->logits, &seq, 1, out);
     e->sync();
   });
 }
@@ -1462,7 +1532,7 @@ qd_status step_common(qd_engine *e, uint32_t seq, uint32_t token, float *logits_
                          hipMemcpyDeviceToHost, e->stream), "D2H");
     if (resident) e->enqueue_resident_error();
     if (logits_out)
-      check(hipMemcpyAsync(logits_out, dev_logits, e->V * 4, hipMemcpyDeviceToHost, e->stream), "D2H");
+      e->read_rows(e->logits, &seq, 1, logits_out);
     e->sync();
     if (resident) {
       e->resident_status(*e->h_error);
@@ -1646,7 +1716,7 @@ qd_status qd_prefill(qd_engine *e, uint32_t seq, const uint32_t *tokens, uint32_
     check(hipMemcpyAsync(&e->h_states[seq], e->states + seq, sizeof(qd::SeqState),
                          hipMemcpyDeviceToHost, e->stream), "D2H");
     if (last_logits)
-      check(hipMemcpyAsync(last_logits, e->logits + seq * e->V, e->V * 4, hipMemcpyDeviceToHost, e->stream), "D2H");
+      e->read_rows(e->logits, &seq, 1, last_logits);
     e->sync();
     if (greedy) *greedy = e->h_states[seq].token;
     if (top_logit) *top_logit = e->h_states[seq].top_logit;
@@ -1664,11 +1734,7 @@ qd_status qd_step_batch(qd_engine *e, uint32_t n_seq, const uint32_t *seq_ids, c
     check(hipMemcpyAsync(e->h_bt_out, e->bt_token, n_seq * 4, hipMemcpyDeviceToHost, e->stream), "D2H");
     check(hipMemcpyAsync(e->h_bt_out + e->B, e->bt_top, n_seq * 4, hipMemcpyDeviceToHost, e->stream),
           "D2H");
-    if (logits)
-      for (uint32_t i = 0; i < n_seq; ++i)
-        check(hipMemcpyAsync(logits + size_t(i) * e->V, e->logits + size_t(seq_ids[i]) * e->V, e->V * 4,
-                             hipMemcpyDeviceToHost, e->stream),
-              "D2H");
+    if (logits) e->read_rows(e->logits, seq_ids, n_seq, logits);
     e->sync();
     for (uint32_t i = 0; i < n_seq; ++i) {
       e->positions[seq_ids[i]] += 1;

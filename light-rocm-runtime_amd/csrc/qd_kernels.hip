@@ -379,6 +379,35 @@ __global__ __launch_bounds__(kBlock) void argmax_finalize_kernel(
 
 // Writes a slot's decode state for a step-mode token at `position` from
 // kernel arguments (no host buffer stays referenced after the launch).
+// Bound by the host link (16 rows of 151,936 logits: 9.7 MB in 180 us). Few
+// workgroups, which take the pieces in order: the host copies a piece on while
+// the next arrive. (With a workgroup per piece they all arrive at the end:
+// 412 us to the caller's buffer against 248; 16 or 32 workgroups 247 and 258.)
+__global__ __launch_bounds__(kBlock) void export_rows_kernel(const float *__restrict__ src, size_t n, int pieces,
+                                                             int rows, ExportRows which, float *__restrict__ dst,
+                                                             uint32_t *flags, uint32_t epoch) {
+  constexpr int kPer = 8;
+  for (int p = blockIdx.x; p < rows * pieces; p += gridDim.x) {
+    const int row = p / pieces;
+    const size_t begin = static_cast<size_t>(p % pieces) * kExportPiece;
+    const int len = static_cast<int>(n - begin < kExportPiece ? n - begin : kExportPiece);
+    const float *from = src + which.slot[row] * n + begin;
+    float *to = dst + row * n + begin;
+    for (int i0 = threadIdx.x; i0 < len; i0 += kPer * kBlock) {
+      float v[kPer];
+#pragma unroll
+      for (int j = 0; j < kPer; ++j)
+        if (i0 + j * kBlock < len) v[j] = from[i0 + j * kBlock];
+#pragma unroll
+      for (int j = 0; j < kPer; ++j)
+        if (i0 + j * kBlock < len) to[i0 + j * kBlock] = v[j];
+    }
+    __threadfence_system();
+    __syncthreads();
+    if (threadIdx.x == 0) __hip_atomic_store(flags + p, epoch, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+}
+
 __global__ void set_state_kernel(SeqState *__restrict__ st, uint32_t position, uint32_t token) {
   if (threadIdx.x != 0) return;
   SeqState s{};
@@ -502,6 +531,13 @@ hipError_t probe_hbm(int device, size_t bytes, uint32_t iters, double *read_gbs,
     (copy ? *copy_gbs : *read_gbs) = best;
   }
   cleanup();
+  return hipGetLastError();
+}
+
+hipError_t launch_export_rows(hipStream_t s, const float *src, size_t n, const ExportRows &which, int rows,
+                              float *dst, uint32_t *flags, uint32_t epoch) {
+  if (rows <= 0 || rows > kExportRows || n == 0) return hipErrorInvalidValue;
+  export_rows_kernel<<<8, kBlock, 0, s>>>(src, n, static_cast<int>(export_pieces(n)), rows, which, dst, flags, epoch);
   return hipGetLastError();
 }
 

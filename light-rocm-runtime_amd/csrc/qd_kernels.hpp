@@ -78,6 +78,16 @@ hipError_t launch_tail(hipStream_t s, const TailLaunch &p, Marker *m = nullptr);
 hipError_t probe_hbm(int device, size_t bytes, uint32_t iters, double *read_gbs, double *copy_gbs);
 // Sets a slot's state to a step-mode token at `position` (device side).
 hipError_t launch_set_state(hipStream_t s, SeqState *st, uint32_t position, uint32_t token);
+// Rows slot[0 .. rows) of src ([..][n] floats) to pinned host memory dst
+// ([rows][n]), in pieces of kExportPiece floats; piece i of row r raises
+// flags[r * pieces + i] (pinned too) to `epoch` once the host can read it.
+constexpr int kExportRows = 16, kExportPiece = 4096;
+inline size_t export_pieces(size_t n) { return (n + kExportPiece - 1) / kExportPiece; }
+struct ExportRows {
+  uint32_t slot[kExportRows];
+};
+hipError_t launch_export_rows(hipStream_t s, const float *src, size_t n, const ExportRows &which, int rows,
+                              float *dst, uint32_t *flags, uint32_t epoch);
 // Rewrites every NaN of x[0, n) (x 16-byte aligned) as 0x7FC00000.
 hipError_t launch_canonical_nan(hipStream_t s, float *x, size_t n);
 

@@ -1,0 +1,46 @@
+"""Logits rows on their way to the caller: in pieces through pinned memory for
+pageable buffers, directly for pinned ones, for rows below and above the size
+that takes the pieces, whole pieces and a remainder, more rows than one export
+holds. Every route returns the same bytes, and only the rows asked for."""
+import ctypes as C
+
+import numpy as np
+import pytest
+import torch
+
+import qwen_decode as qd
+import qwen_oracle as qo
+
+pytestmark = pytest.mark.gpu
+
+PIECE, EXPORT_BYTES, SLOTS = 4096, 256 * 1024, 18
+
+
+@pytest.mark.parametrize("vocab", [1003, EXPORT_BYTES // 4 - 1, EXPORT_BYTES // 4, 20 * PIECE, 20 * PIECE + 7])
+def test_every_route_returns_the_same_logits(vocab):
+    print(f"logits of vocabulary {vocab}", flush=True)
+    eng = qd.Engine(layers=1, vocab=vocab, capacity=8, max_batch=SLOTS)
+    eng.load_synthetic(3)
+    slots = [(7 * i + 3) % SLOTS for i in range(SLOTS)]
+    tokens = [int(t) for t in qo.fill_tokens(SLOTS, 3, 0x700000, vocab)]
+    for n in (SLOTS, 16, 5, 1):
+        for s in slots:
+            eng.kv_reset(s, 0)
+        _, logits = eng.step_batch(slots[:n], tokens[:n])
+        # The row whose end the copy could overrun, in a larger buffer.
+        guarded = np.full(vocab + 2 * PIECE, 7.0, np.float32)
+        for i, s in enumerate(slots[:n]):
+            assert np.array_equal(eng.read_logits(s), logits[i])
+            out = guarded[PIECE:PIECE + vocab]
+            qd._check(qd.lib().qd_read_logits(eng.handle, s, out.ctypes.data_as(C.POINTER(C.c_float)), vocab))
+            assert np.array_equal(out, logits[i])
+            assert (guarded[:PIECE] == 7).all() and (guarded[PIECE + vocab:] == 7).all()
+        pinned = torch.empty((n, vocab), dtype=torch.float32, pin_memory=True).numpy()
+        for s in slots:
+            eng.kv_reset(s, 0)
+        ids, toks = np.array(slots[:n], np.uint32), np.array(tokens[:n], np.uint32)
+        greedy = np.empty(n, np.uint32)
+        qd._check(qd.lib().qd_step_batch(eng.handle, n, qd._u(ids), qd._u(toks), qd._f(pinned), qd._u(greedy)))
+        assert np.array_equal(pinned, logits)
+        assert np.array_equal(greedy, np.argmax(logits, axis=1))
+    eng.close()
