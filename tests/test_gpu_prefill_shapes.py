@@ -63,6 +63,18 @@ def test_rows_match_oracle(pair, rows):
     assert rel_err(v, cache.layer(LAYERS - 1, True)[:rows]) <= RTOL
 
 
+@pytest.mark.parametrize("rows", [1, 2, 33, 513, 2048, 2049, LONGEST])
+def test_last_row_matches_a_step_after_the_rows_before(pair, rows):
+    """The last layer runs for the prompt's last row alone."""
+    eng, prompt, _ = pair
+    print(f"prefill {eng.config.decoder_dtype} {rows} rows, last row", flush=True)
+    eng.kv_reset(0, 0)
+    _, _, logits = eng.prefill(0, prompt[:rows])
+    eng.kv_reset(0, rows - 1)
+    _, _, step = eng.step(0, int(prompt[rows - 1]))
+    assert rel_err(logits, step) <= RTOL
+
+
 def write_bundle(directory, layers, tail):
     for i, tensors in enumerate(layers):
         d = os.path.join(directory, f"layer_{i}")
