@@ -263,7 +263,10 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_split_kernel(Args<W> g, int 
     }
   };
 
-  f16v lead[RB][CB] = {}, tail[RB][CB] = {};
+  // Two chains of leading products, of every other 16 k's each, halve the
+  // roundings of large sums per chain; the 128-row tile has no registers for it.
+  constexpr int kLeads = RB < 4 ? 2 : 1;
+  f16v lead[kLeads][RB][CB] = {}, tail[RB][CB] = {};
 #pragma unroll
   for (int d = 0; d < NS - 1; ++d)
     if (d < n) fetch(d);
@@ -304,7 +307,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_split_kernel(Args<W> g, int 
           for (int cb = 0; cb < CB; ++cb)
             acc[rb][cb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[rb][pa], wv[cb][pw], acc[rb][cb], 0, 0, 0);
       };
-      mac(lead, 0, 0);
+      mac(lead[j % kLeads], 0, 0);
       if constexpr (Op::kParts > 1) mac(tail, 0, 1);
       mac(tail, 1, 0);
       if constexpr (Op::kParts > 1) mac(tail, 1, 1);
@@ -318,7 +321,10 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_split_kernel(Args<W> g, int 
   constexpr int kRegs = RB * CB * 16 / WK;
   float v[kRegs];
   auto sum = [&](int i) {
-    return lead[i / (16 * CB)][i / 16 % CB][i % 16] + tail[i / (16 * CB)][i / 16 % CB][i % 16];
+    const int rb = i / (16 * CB), cb = i / 16 % CB, r = i % 16;
+    float s = lead[0][rb][cb][r];
+    if constexpr (kLeads == 2) s += lead[1][rb][cb][r];
+    return s + tail[rb][cb][r];
   };
   if constexpr (WK == 1) {
 #pragma unroll

@@ -475,13 +475,13 @@ __global__ __launch_bounds__(kBlock) void attention_merge_kernel(AttnArgs g) {
 // ---- GEMM launches ------------------------------------------------------------------
 
 // Tile shapes of the split GEMM, by the number of rows.
-enum Shape : int { kRows32K4 = 0, kRows32, kRows64, kRows128 };
+enum Shape : int { kRows32K4 = 0, kRows32, kRows64, kRows96, kRows128 };
 struct ShapeInfo {
   int rows, cols, wk;
 };
-constexpr ShapeInfo kShapes[] = {{32, 32, 4}, {32, 64, 2}, {64, 128, 1}, {128, 128, 1}};
+constexpr ShapeInfo kShapes[] = {{32, 32, 4}, {32, 64, 2}, {64, 128, 1}, {96, 128, 1}, {128, 128, 1}};
 // The gate/up GEMM's 64-row shape splits k over two waves, not n.
-constexpr ShapeInfo kSwiGLUShapes[] = {{32, 32, 4}, {32, 64, 2}, {64, 64, 2}, {128, 128, 1}};
+constexpr ShapeInfo kSwiGLUShapes[] = {{32, 32, 4}, {32, 64, 2}, {64, 64, 2}, {96, 128, 1}, {128, 128, 1}};
 
 // Up to 32 rows the waves split k, so that 32 columns make a workgroup;
 // beyond, larger tiles reuse each staged weight for more rows as soon as there
@@ -489,10 +489,22 @@ constexpr ShapeInfo kSwiGLUShapes[] = {{32, 32, 4}, {32, 64, 2}, {64, 64, 2}, {1
 // (128-row tile: 2048 only), gate/up: 12.2 / 20.4 / 31.4 with 32 rows and four
 // k waves, 15.6 / 17.2 / 29.4 with two, 18.1 / 18.7 / 26.9 / 70 with 64 rows,
 // 77 (512) / 237 (2048) with 128 rows (64 rows: 267 at 2048).
-Shape gemm_shape(int m, bool swiglu) {
+//
+// Gate/up from 193 to 864 rows: 96 x 128 tiles do less per product outside
+// the matrix cores, but are few, and a round of 256 that they hardly begin
+// costs as much as a full one; so they are taken where they fill more than two
+// fifths of their last round. us with 64 / 96 rows, FP32 (F16): m = 200
+// 42.6 / 40.7 (37.8 / 33.4), 288 46.5 / 41.8 (39.2 / 36.5), 512 66.8 / 65.8
+// (59.1 / 55.4), 860 110.8 / 99.7 (95.9 / 79.6); and where not taken, 300
+// 45.1 / 56.8 (40.6 / 48.9), 640 75.4 / 94.3 (65.0 / 73.0), 960 113.6 / 118.4
+// (97.0 / 101.3).
+Shape gemm_shape(int m, int n, bool swiglu) {
   if (m <= 32) return kRows32K4;
   if (m <= (swiglu ? 64 : 128)) return kRows32;
-  return m <= 1024 ? kRows64 : kRows128;
+  if (m > 1024) return kRows128;
+  if (!swiglu || m <= 192 || m > 864) return kRows64;
+  const int workgroups = (m + 95) / 96 * (n / 64);
+  return ((workgroups - 1) % 256 + 1) * 5 > 256 * 2 ? kRows96 : kRows64;
 }
 
 template <int RB, int WM, int WN, int WK, typename W, bool kSwiGLU>
@@ -505,7 +517,7 @@ void launch_shape(hipStream_t s, const gemm::Args<W> &g) {
 
 template <typename W>
 hipError_t launch_gemm_as(hipStream_t s, gemm::Args<W> g, bool swiglu) {
-  const Shape shape = gemm_shape(g.m, swiglu);
+  const Shape shape = gemm_shape(g.m, g.n, swiglu);
   const ShapeInfo &i = (swiglu ? kSwiGLUShapes : kShapes)[shape];
   // Whole tiles of columns and whole slices of k (rows are masked).
   if (g.m <= 0 || g.k % (gemm::kSliceK * i.wk) != 0 || g.n % (swiglu ? i.cols / 2 : i.cols) != 0 ||
@@ -516,6 +528,7 @@ hipError_t launch_gemm_as(hipStream_t s, gemm::Args<W> g, bool swiglu) {
       case kRows32K4: launch_shape<1, 1, 1, 4, W, true>(s, g); break;
       case kRows32: launch_shape<1, 1, 2, 2, W, true>(s, g); break;
       case kRows64: launch_shape<2, 1, 2, 2, W, true>(s, g); break;
+      case kRows96: launch_shape<3, 1, 4, 1, W, true>(s, g); break;
       case kRows128: launch_shape<4, 1, 4, 1, W, true>(s, g); break;
     }
   } else {
@@ -523,6 +536,7 @@ hipError_t launch_gemm_as(hipStream_t s, gemm::Args<W> g, bool swiglu) {
       case kRows32K4: launch_shape<1, 1, 1, 4, W, false>(s, g); break;
       case kRows32: launch_shape<1, 1, 2, 2, W, false>(s, g); break;
       case kRows64: launch_shape<2, 1, 4, 1, W, false>(s, g); break;
+      case kRows96: return hipErrorInvalidValue;  // gate/up only
       case kRows128: launch_shape<4, 1, 4, 1, W, false>(s, g); break;
     }
   }
@@ -563,7 +577,7 @@ hipError_t launch_gemm(hipStream_t s, int dtype, const PartRows &a, int m, const
 }  // namespace
 
 int gemm_splits(int m, int n, int k) {
-  const ShapeInfo &i = kShapes[gemm_shape(m, false)];
+  const ShapeInfo &i = kShapes[gemm_shape(m, n, false)];
   const int tiles = (m + i.rows - 1) / i.rows * (n / i.cols);
   // Enough workgroups for the 256 CUs, more where k is long (at m = 512 and
   // k = 4864: 32.7 us with 8 or 9 slices, 35.8 with 4; at k = 896: 13.2 with 3,

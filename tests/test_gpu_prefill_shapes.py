@@ -63,6 +63,11 @@ def test_rows_match_oracle(pair, rows):
     assert rel_err(v, cache.layer(LAYERS - 1, True)[:rows]) <= RTOL
 
 
+@pytest.mark.parametrize("rows", [192, 193, 256, 288, 289, 385, 481, 576, 577])
+def test_rows_match_oracle_at_the_96_row_tiles(pair, rows):
+    test_rows_match_oracle(pair, rows)
+
+
 @pytest.mark.parametrize("rows", [1, 2, 33, 513, 2048, 2049, LONGEST])
 def test_last_row_matches_a_step_after_the_rows_before(pair, rows):
     """The last layer runs for the prompt's last row alone."""
