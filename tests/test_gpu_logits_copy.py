@@ -6,7 +6,6 @@ import ctypes as C
 
 import numpy as np
 import pytest
-import torch
 
 import qwen_decode as qd
 import qwen_oracle as qo
@@ -14,6 +13,16 @@ import qwen_oracle as qo
 pytestmark = pytest.mark.gpu
 
 PIECE, EXPORT_BYTES, SLOTS = 4096, 256 * 1024, 18
+
+
+def pinned_rows(n, vocab):
+    """Pinned memory of the HIP runtime the library runs on, for the process."""
+    hip = C.CDLL(None)
+    if not hasattr(hip, "hipHostMalloc"):
+        hip = C.CDLL("libamdhip64.so.7")
+    ptr = C.c_void_p()
+    assert hip.hipHostMalloc(C.byref(ptr), C.c_size_t(n * vocab * 4), C.c_uint(0)) == 0
+    return np.ctypeslib.as_array(C.cast(ptr, C.POINTER(C.c_float)), (n, vocab))
 
 
 @pytest.mark.parametrize("vocab", [1003, EXPORT_BYTES // 4 - 1, EXPORT_BYTES // 4, 20 * PIECE, 20 * PIECE + 7])
@@ -35,7 +44,7 @@ def test_every_route_returns_the_same_logits(vocab):
             qd._check(qd.lib().qd_read_logits(eng.handle, s, out.ctypes.data_as(C.POINTER(C.c_float)), vocab))
             assert np.array_equal(out, logits[i])
             assert (guarded[:PIECE] == 7).all() and (guarded[PIECE + vocab:] == 7).all()
-        pinned = torch.empty((n, vocab), dtype=torch.float32, pin_memory=True).numpy()
+        pinned = pinned_rows(n, vocab)
         for s in slots:
             eng.kv_reset(s, 0)
         ids, toks = np.array(slots[:n], np.uint32), np.array(tokens[:n], np.uint32)
