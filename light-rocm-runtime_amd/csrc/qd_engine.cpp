@@ -189,6 +189,7 @@ struct qd_engine {
 
   qd::SeqState *h_states = nullptr;  // pinned [max_batch]
   uint32_t *h_tokens = nullptr;      // pinned [capacity]
+  uint32_t *h_hidden = nullptr;      // pinned [hidden]: a hidden vector on its way to the device
   // Logits rows on their way to the caller (read_rows); nullptr if the pinned
   // memory was refused. Then one flag per piece of a row; epoch: the last export.
   float *h_rows = nullptr;           // pinned [min(max_batch, kExportRows)][vocab]
@@ -211,6 +212,7 @@ struct qd_engine {
     for (void *p : allocs) (void)hipFree(p);
     if (h_states) (void)hipHostFree(h_states);
     if (h_tokens) (void)hipHostFree(h_tokens);
+    if (h_hidden) (void)hipHostFree(h_hidden);
     if (h_error) (void)hipHostFree(h_error);
     if (h_rows) (void)hipHostFree(h_rows);
     if (h_rows_flags) (void)hipHostFree(h_rows_flags);
@@ -238,6 +240,18 @@ struct qd_engine {
 
   void upload(float *dst, const float *src, size_t n) {
     check(hipMemcpyAsync(dst, src, n * sizeof(float), hipMemcpyHostToDevice, stream),
+          "hipMemcpyAsync H2D");
+  }
+
+  // A caller's hidden vector to slot seq, every NaN as 0x7FC00000: a layers-only
+  // resident launch takes the vector as its input, and a NaN equal to kSlotEmpty
+  // would reach a hand-off slot with its payload. The caller synchronises before
+  // it returns (h_hidden is used again).
+  void upload_hidden(uint32_t seq, const float *src) {
+    std::memcpy(h_hidden, src, H * sizeof(float));
+    for (size_t i = 0; i < H; ++i)
+      if ((h_hidden[i] & 0x7FFFFFFFu) > 0x7F800000u) h_hidden[i] = 0x7FC00000u;
+    check(hipMemcpyAsync(hidden + size_t(seq) * H, h_hidden, H * sizeof(float), hipMemcpyHostToDevice, stream),
           "hipMemcpyAsync H2D");
   }
 
@@ -1033,6 +1047,8 @@ qd_status qd_engine_create(const qd_config *config, qd_engine **out) {
     check(hipHostMalloc(reinterpret_cast<void **>(&e->h_tokens), e->CAP * sizeof(uint32_t),
                         hipHostMallocDefault),
           "hipHostMalloc");
+    check(hipHostMalloc(reinterpret_cast<void **>(&e->h_hidden), e->H * sizeof(float), hipHostMallocDefault),
+          "hipHostMalloc");
     check(hipHostMalloc(reinterpret_cast<void **>(&e->h_error), 2 * sizeof(uint32_t), hipHostMallocDefault),
           "hipHostMalloc");
     e->alloc_export();
@@ -1419,7 +1435,7 @@ qd_status qd_layer_step(qd_engine *e, uint32_t seq, uint32_t layer, float *hidde
       fail(QD_ERROR_INVALID_ARGUMENT, "sequence %u is full (capacity %zu)", seq, e->CAP);
     e->set_device();
     e->push_state(seq, 0, qd::kModeStep, UINT32_MAX, 0);
-    e->upload(e->hidden + seq * e->H, hidden, e->H);
+    e->upload_hidden(seq, hidden);
     check(qd::launch_layer(e->stream, e->layer_args(seq, layer)), "layer launch");
     check(hipMemcpyAsync(hidden, e->hidden + seq * e->H, e->H * 4, hipMemcpyDeviceToHost, e->stream), "D2H");
     e->sync();
@@ -1431,7 +1447,7 @@ qd_status qd_load_hidden(qd_engine *e, uint32_t seq, const float *hidden) {
     if (!e || !hidden) fail(QD_ERROR_INVALID_ARGUMENT, "null argument");
     e->check_seq(seq);
     e->set_device();
-    e->upload(e->hidden + size_t(seq) * e->H, hidden, e->H);
+    e->upload_hidden(seq, hidden);
     e->sync();
   });
 }

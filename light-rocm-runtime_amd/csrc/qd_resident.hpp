@@ -103,8 +103,8 @@ constexpr int kTagSeqBits = 20;
 // h1 [hidden], the MLP activation [intermediate] and the layer output
 // [hidden]. A slot holds kSlotEmpty until written: a NaN bit pattern (every
 // payload bit set) that the kernels' arithmetic never produces, since the
-// engine canonicalises every NaN it loads (weights, embeddings, K/V rows)
-// to 0x7FC00000.
+// engine canonicalises every NaN it loads (weights, embeddings, K/V rows,
+// hidden vectors) to 0x7FC00000.
 constexpr int kRoleRecStride = 68;
 constexpr uint32_t kSlotEmpty = 0xFFFFFFFFu;
 // The layer output is published in segments: down CU r writes its rows

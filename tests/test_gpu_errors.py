@@ -5,8 +5,9 @@
   (the call returns) and the engine keeps working. The give-up is forced
   with QD_RESIDENT_SPIN_LIMIT=1 at engine creation: waits then give up after
   a few polls, long before any producer publishes.
-* NaN payloads never survive a load: K/V rows written through qd_write_kv
-  and weights loaded from a bundle hold only the canonical NaN 0x7FC00000,
+* NaN payloads never survive a load: K/V rows written through qd_write_kv,
+  hidden vectors of qd_load_hidden and qd_layer_step and weights loaded from a
+  bundle hold only the canonical NaN 0x7FC00000,
   so a NaN whose bits equal the resident kernel's empty-slot pattern
   (0xFFFFFFFF) cannot stall a hand-off; a NaN model decodes to NaN logits on
   the resident path without waiting.
@@ -83,6 +84,45 @@ def test_write_kv_canonicalises_nan():
             assert np.array_equal(np.isnan(got), nan)
             assert (got.view(np.uint32)[nan] == CANONICAL).all()
             assert np.array_equal(got.view(np.uint32)[~nan], want.view(np.uint32)[~nan])
+    finally:
+        eng.close()
+
+
+def hidden_with_nans():
+    h = qo.fill_normal(896, 3, 0x600000, 0.0, 1.0)
+    h[0], h[7], h[500], h[895] = nan_bits(0xFFFFFFFF, 0x7FFFFFFF, 0xFFC00001, 0x7F800001)
+    return h
+
+
+def test_load_hidden_canonicalises_nan():
+    say("load_hidden NaN payloads, then six layers from the vector")
+    eng = qd.Engine(**dict(SMALL, layers=6))
+    try:
+        eng.load_synthetic(5)
+        h = hidden_with_nans()
+        eng.load_hidden(0, h)
+        got, nan = eng.read_activation(0, 0), np.isnan(h)
+        assert np.array_equal(np.isnan(got), nan) and (got.view(np.uint32)[nan] == CANONICAL).all()
+        assert np.array_equal(got[~nan], h[~nan])
+        # The resident kernel reads the vector: NaN everywhere, and no wait
+        # for a slot that only looks empty.
+        assert eng.resident_grid() > 0
+        eng.layer_decode(0, 0, 6, 1)
+        assert np.isnan(eng.read_activation(0, 0)).all()
+    finally:
+        eng.close()
+
+
+def test_layer_step_canonicalises_nan():
+    say("layer_step NaN payloads: hidden vector and the K/V row derived from it")
+    eng = qd.Engine(**SMALL)
+    try:
+        eng.load_synthetic(5)
+        out = eng.layer_step(0, 1, hidden_with_nans())
+        k, v = eng.read_kv(0, 1, 0, 1)
+        for got in (out, k, v):
+            bits = np.ascontiguousarray(got).view(np.uint32)
+            assert np.isnan(got).all() and not (bits == 0xFFFFFFFF).any() and not (bits == 0x7FFFFFFF).any()
     finally:
         eng.close()
 
