@@ -146,7 +146,8 @@ struct qd_engine {
   float *part_val = nullptr;
   uint32_t *part_idx = nullptr;
   uint32_t *tokens_dev = nullptr;  // [capacity]
-  qd::SeqState *states = nullptr;  // [max_batch]
+  qd::SeqState *states = nullptr;  // [max_batch], then the state that advance puts back
+  bool state_kept = false;         // advance's fn has called keep_state
   float *history = nullptr;        // generate-mode logits [capacity][vocab]
   size_t history_rows = 0;
 
@@ -778,6 +779,30 @@ struct qd_engine {
       resident_status(err);
     }
   }
+  // Runs fn, which advances slot seq past decoder layers whose errors surface
+  // when it waits. If it fails, the slot is where it was: its position, and its
+  // device state if fn has called keep_state.
+  template <typename Fn>
+  void advance(uint32_t seq, Fn &&fn) {
+    const uint32_t position = positions[seq];
+    state_kept = false;
+    try {
+      fn();
+    } catch (...) {
+      positions[seq] = position;
+      if (state_kept) {
+        (void)hipMemcpyAsync(states + seq, states + B, sizeof(qd::SeqState), hipMemcpyDeviceToDevice, stream);
+        (void)hipStreamSynchronize(stream);
+      }
+      throw;
+    }
+  }
+  // The slot's state becomes a step-mode token at its position; the one before
+  // is kept for advance.
+  void keep_state(uint32_t seq, uint32_t token) {
+    check(qd::launch_set_state(stream, states + seq, positions[seq], token, states + B), "state launch");
+    state_kept = true;
+  }
   size_t export_rows() const { return std::min<size_t>(B, qd::kExportRows); }
   void alloc_export() {
     const size_t flags = export_rows() * qd::export_pieces(V) * sizeof(uint32_t);
@@ -1037,10 +1062,10 @@ qd_status qd_engine_create(const qd_config *config, qd_engine **out) {
     e->part_val = e->alloc<float>(kLmHeadParts);
     e->part_idx = e->alloc<uint32_t>(kLmHeadParts);
     e->tokens_dev = e->alloc<uint32_t>(e->CAP);
-    e->states = e->alloc<qd::SeqState>(e->B);
+    e->states = e->alloc<qd::SeqState>(e->B + 1);
     check(hipMemsetAsync(e->k_cache, 0, e->B * e->L * e->CAP * e->KVD * 4, e->stream), "memset");
     check(hipMemsetAsync(e->v_cache, 0, e->B * e->L * e->CAP * e->KVD * 4, e->stream), "memset");
-    check(hipMemsetAsync(e->states, 0, e->B * sizeof(qd::SeqState), e->stream), "memset");
+    check(hipMemsetAsync(e->states, 0, (e->B + 1) * sizeof(qd::SeqState), e->stream), "memset");
     check(hipHostMalloc(reinterpret_cast<void **>(&e->h_states), e->B * sizeof(qd::SeqState),
                         hipHostMallocDefault),
           "hipHostMalloc");
@@ -1497,15 +1522,17 @@ qd_status qd_tail(qd_engine *e, uint32_t seq, float *logits_out, uint32_t *greed
     e->set_device();
     // A fresh step-mode state at the slot's position (a layer_decode call
     // left this; a qd_step or prefill left the position after its token).
-    check(qd::launch_set_state(e->stream, e->states + seq, e->positions[seq], 0), "state launch");
-    float *dev_logits = e->logits + size_t(seq) * e->V;
-    check(qd::launch_tail(e->stream, e->tail_args(seq, dev_logits, 0, nullptr)), "tail launch");
-    check(hipMemcpyAsync(&e->h_states[seq], e->states + seq, sizeof(qd::SeqState),
-                         hipMemcpyDeviceToHost, e->stream), "D2H");
-    if (logits_out)
-      e->read_rows(e->logits, &seq, 1, logits_out);
-    e->sync();
-    e->positions[seq] += 1;
+    e->advance(seq, [&] {
+      e->keep_state(seq, 0);
+      float *dev_logits = e->logits + size_t(seq) * e->V;
+      check(qd::launch_tail(e->stream, e->tail_args(seq, dev_logits, 0, nullptr)), "tail launch");
+      check(hipMemcpyAsync(&e->h_states[seq], e->states + seq, sizeof(qd::SeqState),
+                           hipMemcpyDeviceToHost, e->stream), "D2H");
+      if (logits_out)
+        e->read_rows(e->logits, &seq, 1, logits_out);
+      e->sync();
+      e->positions[seq] += 1;
+    });
     if (greedy) *greedy = e->h_states[seq].token;
     if (top_logit) *top_logit = e->h_states[seq].top_logit;
   });
@@ -1683,7 +1710,10 @@ void run_prefill(qd_engine *e, uint32_t seq, const uint32_t *tokens, uint32_t n,
   qd::RolePlan plan{};
   if (!m && (n == 1 || (n == 2 && e->resident_plan(e->positions[seq], n, &plan)))) {
     for (uint32_t i = 0; i < n; ++i) {
-      check(qd::launch_set_state(e->stream, e->states + seq, e->positions[seq], tokens[i]), "state launch");
+      if (i == 0)
+        e->keep_state(seq, tokens[0]);
+      else
+        check(qd::launch_set_state(e->stream, e->states + seq, e->positions[seq], tokens[i]), "state launch");
       check(qd::launch_embed(e->stream, e->embed, e->states + seq, e->hidden + size_t(seq) * e->H,
                              static_cast<int>(e->H), static_cast<int>(e->V)),
             "embed launch");
@@ -1760,12 +1790,14 @@ qd_status qd_prefill(qd_engine *e, uint32_t seq, const uint32_t *tokens, uint32_
                      uint32_t *greedy, float *top_logit) {
   return guard([&] {
     check_prefill(e, seq, tokens, n);
-    run_prefill(e, seq, tokens, n, nullptr);
-    check(hipMemcpyAsync(&e->h_states[seq], e->states + seq, sizeof(qd::SeqState),
-                         hipMemcpyDeviceToHost, e->stream), "D2H");
-    if (last_logits)
-      e->read_rows(e->logits, &seq, 1, last_logits);
-    e->sync();
+    e->advance(seq, [&] {
+      run_prefill(e, seq, tokens, n, nullptr);
+      check(hipMemcpyAsync(&e->h_states[seq], e->states + seq, sizeof(qd::SeqState),
+                           hipMemcpyDeviceToHost, e->stream), "D2H");
+      if (last_logits)
+        e->read_rows(e->logits, &seq, 1, last_logits);
+      e->sync();
+    });
     if (greedy) *greedy = e->h_states[seq].token;
     if (top_logit) *top_logit = e->h_states[seq].top_logit;
   });

@@ -377,8 +377,6 @@ __global__ __launch_bounds__(kBlock) void argmax_finalize_kernel(
   }
 }
 
-// Writes a slot's decode state for a step-mode token at `position` from
-// kernel arguments (no host buffer stays referenced after the launch).
 // Bound by the host link (16 rows of 151,936 logits: 9.7 MB in 180 us). Few
 // workgroups, which take the pieces in order: the host copies a piece on while
 // the next arrive. (With a workgroup per piece they all arrive at the end:
@@ -408,8 +406,13 @@ __global__ __launch_bounds__(kBlock) void export_rows_kernel(const float *__rest
   }
 }
 
-__global__ void set_state_kernel(SeqState *__restrict__ st, uint32_t position, uint32_t token) {
+// Writes a slot's decode state for a step-mode token at `position` from
+// kernel arguments (no host buffer stays referenced after the launch).
+// With `kept`, the state that it replaces goes there.
+__global__ void set_state_kernel(SeqState *__restrict__ st, uint32_t position, uint32_t token,
+                                 SeqState *__restrict__ kept) {
   if (threadIdx.x != 0) return;
+  if (kept) *kept = *st;
   SeqState s{};
   s.position = position;
   s.token = token;
@@ -541,8 +544,8 @@ hipError_t launch_export_rows(hipStream_t s, const float *src, size_t n, const E
   return hipGetLastError();
 }
 
-hipError_t launch_set_state(hipStream_t s, SeqState *st, uint32_t position, uint32_t token) {
-  set_state_kernel<<<1, kWave, 0, s>>>(st, position, token);
+hipError_t launch_set_state(hipStream_t s, SeqState *st, uint32_t position, uint32_t token, SeqState *kept) {
+  set_state_kernel<<<1, kWave, 0, s>>>(st, position, token, kept);
   return hipGetLastError();
 }
 

@@ -76,8 +76,10 @@ hipError_t launch_tail(hipStream_t s, const TailLaunch &p, Marker *m = nullptr);
 // Best-of-`iters` streaming read and copy bandwidth (GB/s, bytes moved per
 // second) over a `bytes` buffer on `device` (current), with temporary buffers.
 hipError_t probe_hbm(int device, size_t bytes, uint32_t iters, double *read_gbs, double *copy_gbs);
-// Sets a slot's state to a step-mode token at `position` (device side).
-hipError_t launch_set_state(hipStream_t s, SeqState *st, uint32_t position, uint32_t token);
+// Sets a slot's state to a step-mode token at `position` (device side); the
+// state before goes to `kept` (nullable).
+hipError_t launch_set_state(hipStream_t s, SeqState *st, uint32_t position, uint32_t token,
+                            SeqState *kept = nullptr);
 // Rows slot[0 .. rows) of src ([..][n] floats) to pinned host memory dst
 // ([rows][n]), in pieces of kExportPiece floats; piece i of row r raises
 // flags[r * pieces + i] (pinned too) to `epoch` once the host can read it.

@@ -65,6 +65,50 @@ def test_resident_wait_give_up_reports_device_fault(monkeypatch):
         ref.close()
 
 
+def state_of(eng):
+    s = eng.decode_state(0)
+    return {name: getattr(s, name) for name, *_ in s._fields_}
+
+
+@pytest.mark.parametrize("call", ["prefill 1", "prefill 2", "tail"])
+def test_failed_layers_leave_the_slot_where_it_was(monkeypatch, call):
+    say(f"layers-only launch gives up under {call}")
+    config = dict(SMALL, layers=6)
+    monkeypatch.setenv("QD_RESIDENT_SPIN_LIMIT", "1")
+    eng = qd.Engine(**config)
+    monkeypatch.delenv("QD_RESIDENT_SPIN_LIMIT")
+    ref = qd.Engine(**config)
+    try:
+        prompt = qo.fill_tokens(7, 5, 0x300000, SMALL["vocab"])
+        for e in (eng, ref):
+            e.load_synthetic(5)
+            e.prefill(0, prompt[:5], want_logits=False)
+            assert e.resident_grid() > 0
+        if call == "tail":
+            eng.embed_hidden(0, int(prompt[5]))
+            eng.layer_decode(0, 0, 6, 6)
+        before = None if call == "tail" else state_of(eng)
+        with pytest.raises(qd.QdError) as err:
+            if call == "tail":
+                eng.tail(0)
+            else:
+                eng.prefill(0, prompt[5:5 + int(call[-1])])
+        assert err.value.status == qd.DEVICE_FAULT
+        if before:
+            assert state_of(eng) == before
+        assert eng.decode_state(0).token_position == 5
+        # Its next step writes and attends over the rows that the reference's does.
+        tok, _, logits = eng.step_graph(0, int(prompt[5]))
+        tok2, _, logits2 = ref.step_graph(0, int(prompt[5]))
+        assert tok == tok2 and np.array_equal(logits, logits2)
+        for layer in range(6):
+            for a, b in zip(eng.read_kv(0, layer, 0, 6), ref.read_kv(0, layer, 0, 6)):
+                assert np.array_equal(a, b)
+    finally:
+        eng.close()
+        ref.close()
+
+
 def nan_bits(*patterns):
     return np.array(patterns, np.uint32).view(np.float32)
 
