@@ -133,6 +133,7 @@ struct qd_engine {
   hipEvent_t ev_begin = nullptr, ev_end = nullptr;
   std::vector<void *> allocs;
   uint64_t device_bytes = 0;
+  uint64_t byte_limit = UINT64_MAX;  // QD_DEVICE_BYTES_LIMIT: most device memory the engine may hold
 
   float *weights = nullptr;  // arena of all layer weights
   size_t weights_floats = 0;
@@ -166,16 +167,21 @@ struct qd_engine {
   static constexpr size_t kResidentLayers = 3;
   int roles_grid = 0;                       // 0: resident path unavailable
   std::string resident_off_reason;
-  // Prompt workspace (allocated on the first prefill) for chunks of up to
-  // kPrefillRows positions: rows of the hidden states and the rotated queries,
-  // the GEMMs' left operands in parts (RMSNorm output, attention output,
-  // SwiGLU activation), their partial products, the attention's partial
-  // records and the chunk's token ids.
+  // Prompt workspace for chunks of up to `rows` positions, carved from one
+  // allocation, so that it is there as a whole or not at all: rows of the hidden
+  // states and the rotated queries, the GEMMs' left operands in parts (RMSNorm
+  // output, attention output, SwiGLU activation), their partial products, the
+  // attention's partial records and the chunk's token ids.
   // Longer chunks read each weight for more rows (the 128-row GEMM tiles).
-  static constexpr size_t kPrefillRows = 2048;
-  float *pf_h = nullptr, *pf_q = nullptr, *pf_split = nullptr, *pf_rec = nullptr;
-  qd::PartRows pf_xn{}, pf_attn{}, pf_act{};
-  uint32_t *pf_tokens = nullptr;
+  static constexpr size_t kPrefillRows = 2048, kShortPrefillRows = 512;  // 160 and 70 MB
+  struct PromptWorkspace {
+    char *block;
+    size_t bytes, rows;
+    float *h, *q, *split, *rec;
+    qd::PartRows xn, attn, act;
+    uint32_t *tokens;
+  };
+  PromptWorkspace pf{};
   // Batched-step workspace (allocated on the first batched step): rows of
   // up to kBatchRows sequences, attention and split-K partials, arrival
   // counters, the LM-head top-1 partials and each row's greedy result.
@@ -227,10 +233,21 @@ struct qd_engine {
   T *alloc(size_t count) {
     void *p = nullptr;
     const size_t bytes = std::max<size_t>(count * sizeof(T), 256);
-    check(hipMalloc(&p, bytes), "hipMalloc");
+    if (bytes > byte_limit - device_bytes)
+      fail(QD_ERROR_RUNTIME, "%zu bytes more than the engine's %llu would pass QD_DEVICE_BYTES_LIMIT", bytes,
+           static_cast<unsigned long long>(device_bytes));
+    const hipError_t err = hipMalloc(&p, bytes);
+    if (err != hipSuccess) (void)hipGetLastError();  // not the next launch's error
+    check(err, "hipMalloc");
     allocs.push_back(p);
     device_bytes += bytes;
     return static_cast<T *>(p);
+  }
+  // Frees alloc's `bytes` at p (waits for the device).
+  void release(void *p, size_t bytes) {
+    check(hipFree(p), "hipFree");
+    allocs.erase(std::find(allocs.begin(), allocs.end(), p));
+    device_bytes -= std::max<size_t>(bytes, 256);
   }
 
   float *kv_slice(float *base, size_t seq, size_t layer) const {
@@ -572,56 +589,90 @@ struct qd_engine {
     return {0, 0};
   }
 
-  // One chunk of a prompt (n <= kPrefillRows tokens at positions
+  // The workspace for chunks of `rows` positions, from `base` on (nullptr: its size only).
+  PromptWorkspace carve_prompt_workspace(char *base, size_t rows) const {
+    PromptWorkspace w{};
+    w.block = base;
+    w.rows = rows;
+    auto take = [&](size_t bytes) {
+      char *p = base ? base + w.bytes : nullptr;
+      w.bytes += (bytes + 255) / 256 * 256;
+      return p;
+    };
+    auto floats = [&](size_t n) { return reinterpret_cast<float *>(take(n * sizeof(float))); };
+    auto parts = [&](size_t width) {
+      return qd::PartRows{reinterpret_cast<uint16_t *>(take(3 * rows * width * sizeof(uint16_t))), rows * width};
+    };
+    size_t split = 0;
+    for (int m = 1; m <= int(rows); ++m)
+      for (const auto &[cols, k] : {std::pair<size_t, size_t>{QKV, H}, {H, QD}, {H, I}})
+        split = std::max(split, size_t(qd::gemm_splits(m, int(cols), int(k))) * size_t(m) * cols);
+    w.h = floats(rows * H);
+    w.q = floats(rows * QD);
+    w.xn = parts(H);
+    w.attn = parts(QD);
+    w.act = parts(I);
+    w.split = floats(split);
+    w.rec = floats(size_t(qd::kAttnRecRows) * qd::kAttnRecFloats);
+    w.tokens = reinterpret_cast<uint32_t *>(take(rows * sizeof(uint32_t)));
+    return w;
+  }
+  // Makes pf hold a prompt of n tokens in as few chunks as it can, and returns
+  // the rows of a chunk. Prompts of up to kShortPrefillRows tokens get the small
+  // one; where the device has no room for the large one, long prompts run in
+  // chunks of the small one's rows.
+  uint32_t prompt_workspace(size_t n) {
+    auto grow = [&](size_t rows) {
+      const size_t bytes = carve_prompt_workspace(nullptr, rows).bytes;
+      char *block = alloc<char>(bytes);
+      if (pf.block) release(pf.block, pf.bytes);
+      pf = carve_prompt_workspace(block, rows);
+    };
+    const size_t want = n <= kShortPrefillRows ? kShortPrefillRows : kPrefillRows;
+    if (pf.rows < want) {
+      try {
+        grow(want);
+      } catch (const QdError &) {
+        if (want == kShortPrefillRows) throw;
+        if (!pf.rows) grow(kShortPrefillRows);
+      }
+    }
+    return uint32_t(pf.rows);
+  }
+
+  // One chunk of a prompt (n <= pf.rows tokens at positions
   // pos0 .. pos0 + n - 1 of slot seq) through every layer with the prompt
   // kernels; leaves the final hidden row of the last token in row n - 1 of
-  // pf_h. Of the last layer's rows only K and V are read again, but for the
+  // pf.h. Of the last layer's rows only K and V are read again, but for the
   // prompt's last token: the rest of that layer runs for its row alone, and not
   // at all in a chunk before the prompt's last (1,999 rows: 0.4 of 11.6 ms).
   // With m (nullable) every launch is timed and every row is computed.
   void prefill_chunk(uint32_t seq, const uint32_t *tokens, int n, int pos0, bool last, qd::Marker *m = nullptr) {
-    if (!pf_h) {
-      pf_h = alloc<float>(kPrefillRows * H);
-      pf_q = alloc<float>(kPrefillRows * QD);
-      auto parts = [&](size_t width) {
-        return qd::PartRows{alloc<uint16_t>(3 * kPrefillRows * width), kPrefillRows * width};
-      };
-      pf_xn = parts(H);
-      pf_attn = parts(QD);
-      pf_act = parts(I);
-      pf_tokens = alloc<uint32_t>(kPrefillRows);
-      size_t split = 0;
-      for (int rows = 1; rows <= int(kPrefillRows); ++rows)
-        for (const auto &[cols, k] : {std::pair<size_t, size_t>{QKV, H}, {H, QD}, {H, I}})
-          split = std::max(split, size_t(qd::gemm_splits(rows, int(cols), int(k))) * size_t(rows) * cols);
-      pf_split = alloc<float>(split);
-      pf_rec = alloc<float>(size_t(qd::kAttnRecRows) * qd::kAttnRecFloats);
-    }
-    check(hipMemcpyAsync(pf_tokens, tokens, size_t(n) * 4, hipMemcpyHostToDevice, stream), "H2D");
+    check(hipMemcpyAsync(pf.tokens, tokens, size_t(n) * 4, hipMemcpyHostToDevice, stream), "H2D");
     const int h = int(H), in = int(I), qkv = int(QKV), qd = int(QD);
     auto span = [&](int id, const char *what, auto &&launch) {
       if (m) m->before(id);
       check(launch(), what);
       if (m) m->after(id);
     };
-    // Rows [first, first + rows) of the chunk; pf_xn, pf_attn and pf_act hold
+    // Rows [first, first + rows) of the chunk; pf.xn, pf.attn and pf.act hold
     // them from row 0 on.
     int first = 0, rows = n;
     // Partials of one projection, then the row kernel that finishes its rows.
     auto project = [&](const qd::PartRows &a, const float *w, int cols, int k, auto &&finish) {
       const int splits = qd::gemm_splits(rows, cols, k);
-      const hipError_t err = qd::launch_gemm_partials(stream, wdtype, a, rows, w, cols, k, pf_split, splits);
+      const hipError_t err = qd::launch_gemm_partials(stream, wdtype, a, rows, w, cols, k, pf.split, splits);
       return err != hipSuccess ? err : finish(splits);
     };
     span(kPEmbed, "embed rows + norm", [&] {
-      return qd::launch_embed_norm(stream, embed, pf_tokens, n, layers[0].attn_norm, cfg.rms_eps, pf_h, pf_xn);
+      return qd::launch_embed_norm(stream, embed, pf.tokens, n, layers[0].attn_norm, cfg.rms_eps, pf.h, pf.xn);
     });
     for (size_t l = 0; l < L; ++l) {
       const qd::LayerPtrs &w = layers[l];
       float *kc = kv_slice(k_cache, seq, l), *vc = kv_slice(v_cache, seq, l);
       span(kPGemmQkv, "qkv gemm + rope", [&] {
-        return project(pf_xn, w.wqkv, qkv, h, [&](int splits) {
-          return qd::launch_qkv_rope(stream, pf_split, splits, n, w.bqkv, pos0, rope_cos, rope_sin, pf_q, kc, vc);
+        return project(pf.xn, w.wqkv, qkv, h, [&](int splits) {
+          return qd::launch_qkv_rope(stream, pf.split, splits, n, w.bqkv, pos0, rope_cos, rope_sin, pf.q, kc, vc);
         });
       });
       if (l + 1 == L && !m) {
@@ -630,21 +681,21 @@ struct qd_engine {
         rows = 1;
       }
       span(kPAttn, "attention", [&] {
-        return qd::launch_attention_prefill(stream, pf_q + size_t(first) * QD, rows, pos0 + first, kc, vc, pf_rec,
-                                            pf_attn);
+        return qd::launch_attention_prefill(stream, pf.q + size_t(first) * QD, rows, pos0 + first, kc, vc, pf.rec,
+                                            pf.attn);
       });
       span(kPGemmO, "o gemm + norm", [&] {
-        return project(pf_attn, w.wo, h, qd, [&](int splits) {
-          return qd::launch_residual_norm(stream, pf_split, splits, rows, pf_h + size_t(first) * H, w.mlp_norm,
-                                          cfg.rms_eps, pf_xn);
+        return project(pf.attn, w.wo, h, qd, [&](int splits) {
+          return qd::launch_residual_norm(stream, pf.split, splits, rows, pf.h + size_t(first) * H, w.mlp_norm,
+                                          cfg.rms_eps, pf.xn);
         });
       });
       span(kPGemmGateUp, "gate/up gemm + swiglu",
-           [&] { return qd::launch_gemm_swiglu(stream, wdtype, pf_xn, rows, w.wg, w.wu, in, h, pf_act); });
+           [&] { return qd::launch_gemm_swiglu(stream, wdtype, pf.xn, rows, w.wg, w.wu, in, h, pf.act); });
       span(kPGemmDown, "down gemm + norm", [&] {
-        return project(pf_act, w.wd, h, in, [&](int splits) {
-          return qd::launch_residual_norm(stream, pf_split, splits, rows, pf_h + size_t(first) * H,
-                                          l + 1 < L ? layers[l + 1].attn_norm : nullptr, cfg.rms_eps, pf_xn);
+        return project(pf.act, w.wd, h, in, [&](int splits) {
+          return qd::launch_residual_norm(stream, pf.split, splits, rows, pf.h + size_t(first) * H,
+                                          l + 1 < L ? layers[l + 1].attn_norm : nullptr, cfg.rms_eps, pf.xn);
         });
       });
     }
@@ -1014,6 +1065,12 @@ qd_status qd_engine_create(const qd_config *config, qd_engine **out) {
     e->wdtype = c.decoder_dtype == QD_DTYPE_BF16 ? qd::kWeightsBf16
                 : c.decoder_dtype == QD_DTYPE_F16  ? qd::kWeightsF16
                                                    : qd::kWeightsF32;
+    // QD_DEVICE_BYTES_LIMIT bounds the engine's device memory: an allocation
+    // past it fails as one that the device has no room for.
+    if (const char *lim = std::getenv("QD_DEVICE_BYTES_LIMIT")) {
+      const unsigned long long v = std::strtoull(lim, nullptr, 10);
+      if (v) e->byte_limit = v;
+    }
     e->set_device();
     check(hipStreamCreateWithFlags(&e->stream, hipStreamNonBlocking), "hipStreamCreate");
     check(hipEventCreate(&e->ev_begin), "hipEventCreate");
@@ -1698,7 +1755,7 @@ void check_prefill(qd_engine *e, uint32_t seq, const uint32_t *tokens, uint32_t 
   e->set_device();
 }
 
-// The prompt in chunks of up to kPrefillRows positions, each through all
+// The prompt in chunks of up to the workspace's rows, each through all
 // layers at once (dense GEMMs); then the tail (final norm, LM head, argmax)
 // on the last position, which advances the slot to pos0 + n. m (nullable)
 // times every launch.
@@ -1725,8 +1782,9 @@ void run_prefill(qd_engine *e, uint32_t seq, const uint32_t *tokens, uint32_t n,
     e->positions[seq] += 1;
     return;
   }
+  const uint32_t chunk = e->prompt_workspace(n);
   for (uint32_t done = 0; done < n;) {
-    const uint32_t rows = std::min<uint32_t>(n - done, uint32_t(qd_engine::kPrefillRows));
+    const uint32_t rows = std::min(n - done, chunk);
     if (m) {
       m->ctx_a = rows;
       m->ctx_b = e->positions[seq] + done;
@@ -1734,10 +1792,10 @@ void run_prefill(qd_engine *e, uint32_t seq, const uint32_t *tokens, uint32_t n,
     e->prefill_chunk(seq, tokens + done, int(rows), int(e->positions[seq] + done), done + rows == n, m);
     done += rows;
     if (done == n)
-      check(hipMemcpyAsync(e->hidden + size_t(seq) * e->H, e->pf_h + size_t(rows - 1) * e->H, e->H * 4,
+      check(hipMemcpyAsync(e->hidden + size_t(seq) * e->H, e->pf.h + size_t(rows - 1) * e->H, e->H * 4,
                            hipMemcpyDeviceToDevice, e->stream),
             "D2D");
-    e->sync();  // the next chunk's token upload reuses pf_tokens
+    e->sync();  // the next chunk's token upload reuses pf.tokens
   }
   e->positions[seq] += n - 1;
   e->push_state(seq, tokens[n - 1], qd::kModeStep, UINT32_MAX, 0);
@@ -1919,9 +1977,9 @@ qd_status qd_generate_resident(qd_engine *e, uint32_t seq, uint32_t first_token,
     if (all_logits) {
       if (e->history_rows < max_tokens) {
         if (e->history) {
-          check(hipFree(e->history), "hipFree");
-          e->allocs.erase(std::find(e->allocs.begin(), e->allocs.end(), static_cast<void *>(e->history)));
-          e->device_bytes -= std::max<size_t>(e->history_rows * e->V * 4, 256);
+          e->release(e->history, e->history_rows * e->V * 4);
+          e->history = nullptr;
+          e->history_rows = 0;
         }
         e->history = e->alloc<float>(size_t(max_tokens) * e->V);
         e->history_rows = max_tokens;

@@ -5,6 +5,9 @@
   (the call returns) and the engine keeps working. The give-up is forced
   with QD_RESIDENT_SPIN_LIMIT=1 at engine creation: waits then give up after
   a few polls, long before any producer publishes.
+* A prompt whose workspace the device has no room for fails and can be tried
+  again (QD_DEVICE_BYTES_LIMIT refuses the allocation); long prompts make do
+  with the workspace of a short one.
 * NaN payloads never survive a load: K/V rows written through qd_write_kv,
   hidden vectors of qd_load_hidden and qd_layer_step and weights loaded from a
   bundle hold only the canonical NaN 0x7FC00000,
@@ -107,6 +110,56 @@ def test_failed_layers_leave_the_slot_where_it_was(monkeypatch, call):
     finally:
         eng.close()
         ref.close()
+
+
+def test_prompt_without_room_for_its_workspace(monkeypatch):
+    say("prompt workspace allocations refused by QD_DEVICE_BYTES_LIMIT")
+    config = dict(SMALL, capacity=700)
+    prompt = qo.fill_tokens(600, 5, 0x300000, SMALL["vocab"])
+    engines = []
+
+    def engine(limit=None):
+        if limit:
+            monkeypatch.setenv("QD_DEVICE_BYTES_LIMIT", str(limit))
+        engines.append(qd.Engine(**config))
+        monkeypatch.delenv("QD_DEVICE_BYTES_LIMIT", raising=False)
+        engines[-1].load_synthetic(5)
+        return engines[-1]
+
+    try:
+        ref = engine()
+        base = ref.device_bytes()
+        _, _, want = ref.prefill(0, prompt[:3])
+        short = ref.device_bytes() - base
+        ref.prefill(0, prompt[3:600])
+        full = ref.device_bytes() - base  # the short one is given back
+        say(f"workspace bytes: {short} for 3 tokens, {full} for 597")
+        assert 0 < short < full
+        # No room at all: an error each time, nothing kept, and steps still run.
+        none = engine(base + short // 2)
+        for _ in range(2):
+            with pytest.raises(qd.QdError) as err:
+                none.prefill(0, prompt[:3])
+            assert err.value.status == qd.RUNTIME and none.device_bytes() == base
+            assert none.decode_state(0).token_position == 0
+        for t in prompt[:3].tolist():
+            _, _, got = none.step(0, t)
+        assert np.abs(got - want).max() <= 1e-5 * np.abs(want).max()
+        # Room for the short one: a long prompt runs in its chunks.
+        some = engine(base + short)
+        some.kv_reset(0, 0)
+        _, _, got = some.prefill(0, prompt)
+        assert some.device_bytes() == base + short
+        ref.kv_reset(0, 0)
+        ref.prefill(0, prompt[:512], want_logits=False)
+        _, _, want = ref.prefill(0, prompt[512:])
+        assert np.array_equal(got, want)
+        for layer in range(SMALL["layers"]):
+            for a, b in zip(some.read_kv(0, layer, 0, 600), ref.read_kv(0, layer, 0, 600)):
+                assert np.array_equal(a, b)
+    finally:
+        for e in engines:
+            e.close()
 
 
 def nan_bits(*patterns):
