@@ -231,9 +231,9 @@ QD_API qd_status qd_embed_hidden(qd_engine *engine, uint32_t seq,
  * writes its K/V row there, attends over positions 0..valid_keys - 1 and
  * leaves its output on the device as the next layer's input. Sets the
  * slot's position to valid_keys - 1 (the token in flight; qd_tail
- * completes it). Three or more layers run as one launch of the resident
- * kernel when the engine has it, fewer as the stream-ordered kernels; the two
- * compute the same values bit for bit. Asynchronous: errors surface at the next synchronising
+ * completes it). From three layers on (BF16: four below 64 positions) they run
+ * as one launch of the resident kernel when the engine has it, else as the
+ * stream-ordered kernels; the two compute the same values bit for bit. Asynchronous: errors surface at the next synchronising
  * call. Replaces DecoderLayer::decode_to_hidden_state / decode_to_buffer
  * (examples/triton/mini_decoder_layer.hpp:345-372), whose valid_keys it
  * takes. */

@@ -161,10 +161,17 @@ struct qd_engine {
   uint32_t *resident_error = nullptr;       // [1 + kXcds], then the sticky word of layers-only launches
   bool layers_pending = false;              // the sticky error word is due at the next sync
   uint32_t spin_limit = qd::kResidentSpinLimit;
-  // Layers of one qd_layer_decode from which a resident launch is the faster
-  // (us at context 701, resident / stream: 2 layers 96 / 90, 3 109 / 127, 24
-  // 394 / 900; BF16 94 / 83, 106 / 116, 388 / 819).
-  static constexpr size_t kResidentLayers = 3;
+  // Layers of one token from which a resident launch is the faster. us at
+  // contexts 1 / 48 / 129 / 701 / 1,500 / 4,000, resident against stream:
+  //   3 layers FP32 102 102 102 108 116 123 against 110 114 117 126 125 136
+  //            FP16  99  99 100 106 113 122 against 100 102 107 120 120 130
+  //            BF16  99  99 100 105 114 122 against  94  97 101 114 113 123
+  //   4 layers BF16 112 112 113 118 128 137 against 123 125 131 146 145 159
+  // (two layers FP32 at 701: 96 against 90). BF16 rows cost the stream kernels
+  // least: there it takes four layers below 64 positions.
+  size_t resident_layers(uint32_t position) const {
+    return wdtype == qd::kWeightsBf16 && position < 64 ? 4 : 3;
+  }
   int roles_grid = 0;                       // 0: resident path unavailable
   std::string resident_off_reason;
   // Prompt workspace for chunks of up to `rows` positions, carved from one
@@ -916,12 +923,17 @@ struct qd_engine {
       }
     }
   }
+  // Whether `count` decoder layers of the token at `position` run as one
+  // layers-only resident launch, and its plan.
+  bool layers_resident(uint32_t position, size_t count, qd::RolePlan *plan) const {
+    return count >= resident_layers(position) && resident_fits(1) && resident_plan(position, 1, plan);
+  }
   // Decoder layers [first, first + count) of slot seq on its device hidden
   // vector at its position: one layers-only resident launch, or the stream
   // kernels; the two compute the same values bit for bit.
   void enqueue_layers(uint32_t seq, size_t first, size_t count) {
     qd::RolePlan plan{};
-    if (count >= kResidentLayers && resident_plan(positions[seq], 1, &plan)) {
+    if (layers_resident(positions[seq], count, &plan)) {
       const hipError_t err = launch_resident(plan, seq, 0, 1, UINT32_MAX, nullptr, 0, nullptr, nullptr, 0,
                                              hidden + seq * H, first, count);
       if (err == hipSuccess) {
@@ -1760,12 +1772,13 @@ void check_prefill(qd_engine *e, uint32_t seq, const uint32_t *tokens, uint32_t 
 // on the last position, which advances the slot to pos0 + n. m (nullable)
 // times every launch.
 void run_prefill(qd_engine *e, uint32_t seq, const uint32_t *tokens, uint32_t n, EventMarker *m) {
-  // One token, and two where the resident kernel takes them, run position by
+  // One token, and two where the resident kernel takes each, run position by
   // position through the decode layers: 500 to 580 us and 860 to 1,030 with the
   // tail, against 1,300 to 1,630 through the prompt kernels' nine launches per
   // layer (800 to 1,120 for one token on the stream kernels). Three would tie.
   qd::RolePlan plan{};
-  if (!m && (n == 1 || (n == 2 && e->resident_plan(e->positions[seq], n, &plan)))) {
+  if (!m && (n == 1 || (n == 2 && e->layers_resident(e->positions[seq], e->L, &plan) &&
+                        e->layers_resident(e->positions[seq] + 1, e->L, &plan)))) {
     for (uint32_t i = 0; i < n; ++i) {
       if (i == 0)
         e->keep_state(seq, tokens[0]);
