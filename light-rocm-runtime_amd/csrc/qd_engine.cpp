@@ -1613,7 +1613,9 @@ qd_status qd_read_logits(qd_engine *e, uint32_t seq, float *out, size_t count) {
     e->check_seq(seq);
     if (count != e->V) fail(QD_ERROR_INVALID_ARGUMENT, "logits have %zu elements, caller asked %zu", e->V, count);
     e->set_device();
-    e->read_rows(e->logits, &seq, 1, out);
+    // Every call that writes the row has waited for it, so the export's launch
+    // would have nothing to hide behind: 34.2 us against 35.8.
+    check(hipMemcpyAsync(out, e->logits + size_t(seq) * e->V, e->V * 4, hipMemcpyDeviceToHost, e->stream), "D2H");
     e->sync();
   });
 }

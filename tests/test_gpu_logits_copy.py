@@ -53,3 +53,16 @@ def test_every_route_returns_the_same_logits(vocab):
         assert np.array_equal(pinned, logits)
         assert np.array_equal(greedy, np.argmax(logits, axis=1))
     eng.close()
+
+
+@pytest.mark.parametrize("vocab", [EXPORT_BYTES // 4 - 1, EXPORT_BYTES // 4, 20 * PIECE + 7])
+def test_a_step_writes_its_row_and_nothing_beside_it(vocab):
+    print(f"a step's logits of vocabulary {vocab} into a larger buffer", flush=True)
+    eng = qd.Engine(layers=1, vocab=vocab, capacity=8, max_batch=2)
+    eng.load_synthetic(3)
+    guarded = np.full(vocab + 2 * PIECE, 7.0, np.float32)
+    out = guarded[PIECE:PIECE + vocab]
+    qd._check(qd.lib().qd_step(eng.handle, 1, 5, qd._f(out), None, None))
+    assert np.array_equal(out, eng.read_logits(1))
+    assert (guarded[:PIECE] == 7).all() and (guarded[PIECE + vocab:] == 7).all()
+    eng.close()
