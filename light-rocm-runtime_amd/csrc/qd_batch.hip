@@ -103,9 +103,11 @@ typedef __attribute__((address_space(3))) void ring_lds_void;
 template <bool kOnce>
 __device__ __forceinline__ void ring_dma(const float *src, uint32_t lds) {
   if constexpr (kOnce)
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off nt" ::"s"(lds), "v"(src) : "memory");
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off nt" ::"s"(lds), "v"(src)
+                 : "memory", "m0");
   else
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(src) : "memory");
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(src)
+                 : "memory", "m0");
 }
 template <int n>
 __device__ __forceinline__ void ring_wait() {
