@@ -100,6 +100,8 @@ constexpr int kSlice = 32, kRing = 3, kStageFloats = 2 * 16 * kSlice, kRingFloat
 typedef __attribute__((address_space(3))) void ring_lds_void;
 // kOnce: bytes that no other workgroup reads (weights), not to be kept in L2
 // (LM head at 16 rows 113 -> 106 us).
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"  // m0 is reserved: set before each use, never saved
 template <bool kOnce>
 __device__ __forceinline__ void ring_dma(const float *src, uint32_t lds) {
   if constexpr (kOnce)
@@ -109,6 +111,7 @@ __device__ __forceinline__ void ring_dma(const float *src, uint32_t lds) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(src)
                  : "memory", "m0");
 }
+#pragma clang diagnostic pop
 template <int n>
 __device__ __forceinline__ void ring_wait() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(n) : "memory");

@@ -157,9 +157,12 @@ typedef __attribute__((address_space(3))) void gemm_lds_void;
 // One 16-byte global -> LDS DMA per lane (lane l's bytes land at LDS address
 // lds + 16 l). Issued from inline assembly: the compiler would otherwise guard
 // every later LDS read with a wait for all DMAs in flight.
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"  // m0 is reserved: set before each use, never saved
 __device__ __forceinline__ void dma16(const void *src, uint32_t lds) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(src) : "memory", "m0");
 }
+#pragma clang diagnostic pop
 // Workgroup barrier over LDS only: this wave's LDS operations are complete.
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
