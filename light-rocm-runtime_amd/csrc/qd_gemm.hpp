@@ -150,6 +150,7 @@ struct Args {
 };
 
 constexpr int kThreads = 256;
+constexpr int kStages = 2;  // LDS stages: one is filled while the other is multiplied
 constexpr int kDealXcds = 8;  // consecutive workgroups go to consecutive XCDs
 
 typedef __attribute__((address_space(3))) void gemm_lds_void;
@@ -184,33 +185,27 @@ __device__ __forceinline__ float fp32_element(const Args<W> &g, int row, const W
   return s;
 }
 
-// Waits until at most n of this wave's vector memory operations (its DMAs, the
-// only ones of the main loop) are outstanding.
-template <int n>
-__device__ __forceinline__ void dma_wait() {
-  static_assert(n < 64, "vmcnt is six bits");
-  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(n) : "memory");
-}
+// Waits for this wave's DMAs.
+__device__ __forceinline__ void dma_wait() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
 // Workgroup of four waves, WM along m, WN along n and WK along k; a wave
-// multiplies RB x CB blocks of 32 x 32, so the output tile is 32 RB WM rows by
-// 32 CB WN columns (SwiGLU: 16 CB WN gate columns and the same up columns).
-// A's parts and W's values go through NS LDS stages of 32 WK k's, filled by
-// DMA while earlier ones feed the matrix cores; a wave splits the weights it
-// reads. WK waves' partial tiles are summed through LDS in k order.
+// multiplies RB blocks of 32 x 32, so the output tile is 32 RB WM rows by 32 WN
+// columns (SwiGLU: 16 WN gate columns and the same up columns). A's parts and
+// W's values go through the LDS stages, 32 WK k's each, by DMA; a wave splits the
+// weights it reads. WK waves' partial tiles are summed through LDS in k order.
 // Operand layout of v_mfma_f32_32x32x16_bf16: lane l supplies A[l % 32] and
 // B[l % 32] at k's 8 (l / 32) .. + 7; accumulator register r of lane l holds
 // D[(r / 4) * 8 + (l / 32) * 4 + r % 4][l % 32].
-template <int RB, int CB, int WM, int WN, int WK, int NS, typename W, bool kSwiGLU>
+template <int RB, int WM, int WN, int WK, typename W, bool kSwiGLU>
 __global__ __launch_bounds__(kThreads, 2) void gemm_split_kernel(Args<W> g, int mtiles, int pairs) {
   static_assert(WM * WN * WK == 4, "four waves");
   using Op = WeightOp<W>;
-  constexpr int kRows = 32 * RB * WM, kCols = 32 * CB * WN;
+  constexpr int kRows = 32 * RB * WM, kCols = 32 * WN;
   constexpr int kPlane = kRows * kSliceK * 2;               // bytes of one plane of one k wave's slice
   constexpr int kWRow = kSliceK * static_cast<int>(sizeof(W));  // bytes of a weight row's slice
   constexpr int kABytes = WK * 3 * kPlane, kStage = kABytes + WK * kCols * kWRow;
-  constexpr int kReduce = WK > 1 ? 4 * RB * CB * 16 * kWave * 4 : 0;
-  __shared__ __attribute__((aligned(16))) unsigned char lds[NS * kStage > kReduce ? NS * kStage : kReduce];
+  constexpr int kReduce = WK > 1 ? 4 * RB * 16 * kWave * 4 : 0;
+  __shared__ __attribute__((aligned(16))) unsigned char lds[kStages * kStage > kReduce ? kStages * kStage : kReduce];
 
   // Workgroups of one (column tile, split) pair, which read the same weights,
   // are dealt to one XCD, next to each other in its order.
@@ -269,26 +264,21 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_split_kernel(Args<W> g, int 
   // Two chains of leading products, of every other 16 k's each, halve the
   // roundings of large sums per chain; the 128-row tile has no registers for it.
   constexpr int kLeads = RB < 4 ? 2 : 1;
-  f16v lead[kLeads][RB][CB] = {}, tail[RB][CB] = {};
-#pragma unroll
-  for (int d = 0; d < NS - 1; ++d)
-    if (d < n) fetch(d);
+  f16v lead[kLeads][RB] = {}, tail[RB] = {};
+  if (n > 0) fetch(0);
   int b = 0;
   for (int s = 0; s < n; ++s) {
-    // Stage s has landed once at most the DMAs of the stages after it are
-    // outstanding; after the barrier every wave's part has, and every wave is
-    // done with the stage before, whose place is filled next.
-    if (NS > 2 && n - 1 - s >= NS - 2)
-      dma_wait<(NS - 2) * kIssue>();
-    else
-      dma_wait<0>();
+    // This wave's part of slice s has landed; after the barrier every wave's
+    // has, and every wave is done with the slice before, whose stage is filled
+    // next. (With the stages as b and b ^ 1 the F16 kernels are 1 % slower.)
+    dma_wait();
     lds_barrier();
-    if (s + NS - 1 < n) fetch(b == 0 ? NS - 1 : b - 1);
+    if (s + 1 < n) fetch(b == 0 ? kStages - 1 : b - 1);
     const unsigned char *st = lds + b * kStage;
-    b = b + 1 == NS ? 0 : b + 1;
+    b = b + 1 == kStages ? 0 : b + 1;
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
-      bf8v av[RB][3], wv[CB][Op::kParts];
+      bf8v av[RB][3], wv[Op::kParts];
 #pragma unroll
       for (int rb = 0; rb < RB; ++rb) {
         const int row = 32 * (wm * RB + rb) + lr;
@@ -297,18 +287,13 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_split_kernel(Args<W> g, int 
         for (int p = 0; p < 3; ++p)
           av[rb][p] = *reinterpret_cast<const bf8v *>(st + (wk * 3 + p) * kPlane + row * kSliceK * 2 + 16 * slot);
       }
-#pragma unroll
-      for (int cb = 0; cb < CB; ++cb) {
-        const int c = 32 * (wn * CB + cb) + lr;
-        Op::operand(reinterpret_cast<const u4v *>(st + kABytes + (wk * kCols + c) * kWRow), Op::swizzle(c), 2 * j + half,
-                    wv[cb]);
-      }
-      auto mac = [&](f16v (&acc)[RB][CB], int pa, int pw) {
+      const int c = 32 * wn + lr;
+      Op::operand(reinterpret_cast<const u4v *>(st + kABytes + (wk * kCols + c) * kWRow), Op::swizzle(c), 2 * j + half,
+                  wv);
+      auto mac = [&](f16v (&acc)[RB], int pa, int pw) {
 #pragma unroll
         for (int rb = 0; rb < RB; ++rb)
-#pragma unroll
-          for (int cb = 0; cb < CB; ++cb)
-            acc[rb][cb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[rb][pa], wv[cb][pw], acc[rb][cb], 0, 0, 0);
+          acc[rb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[rb][pa], wv[pw], acc[rb], 0, 0, 0);
       };
       mac(lead[j % kLeads], 0, 0);
       if constexpr (Op::kParts > 1) mac(tail, 0, 1);
@@ -321,13 +306,12 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_split_kernel(Args<W> g, int 
 
   // The wave's elements of the tile: all, or with WK waves along k the 1 / WK
   // of the accumulator registers that this wave finishes.
-  constexpr int kRegs = RB * CB * 16 / WK;
+  constexpr int kRegs = RB * 16 / WK;
   float v[kRegs];
   auto sum = [&](int i) {
-    const int rb = i / (16 * CB), cb = i / 16 % CB, r = i % 16;
-    float s = lead[0][rb][cb][r];
-    if constexpr (kLeads == 2) s += lead[1][rb][cb][r];
-    return s + tail[rb][cb][r];
+    float s = lead[0][i / 16][i % 16];
+    if constexpr (kLeads == 2) s += lead[1][i / 16][i % 16];
+    return s + tail[i / 16][i % 16];
   };
   if constexpr (WK == 1) {
 #pragma unroll
@@ -336,21 +320,21 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_split_kernel(Args<W> g, int 
     float *red = reinterpret_cast<float *>(lds);
     lds_barrier();
 #pragma unroll
-    for (int i = 0; i < RB * CB * 16; ++i) red[(w * RB * CB * 16 + i) * kWave + lane] = sum(i);
+    for (int i = 0; i < RB * 16; ++i) red[(w * RB * 16 + i) * kWave + lane] = sum(i);
     lds_barrier();
 #pragma unroll
     for (int i = 0; i < kRegs; ++i) {
       v[i] = 0.f;
 #pragma unroll
       for (int u = 0; u < WK; ++u)
-        v[i] += red[((u * WM * WN + wm * WN + wn) * RB * CB * 16 + wk * kRegs + i) * kWave + lane];
+        v[i] += red[((u * WM * WN + wm * WN + wn) * RB * 16 + wk * kRegs + i) * kWave + lane];
     }
   }
-  // Column and row of element i within the tile.
-  auto tile_col = [&](int i) { return 32 * (wn * CB + (wk * kRegs + i) / 16 % CB) + lr; };
+  // Column of the wave's elements and row of element i within the tile.
+  const int tile_col = 32 * wn + lr;
   auto tile_row = [&](int i) {
     const int r = wk * kRegs + i;
-    return 32 * (wm * RB + r / (16 * CB)) + ((r % 16) / 4) * 8 + half * 4 + r % 4;
+    return 32 * (wm * RB + r / 16) + ((r % 16) / 4) * 8 + half * 4 + r % 4;
   };
   float probe = 0.f;  // 0 as long as every element is finite
 #pragma unroll
@@ -359,7 +343,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_split_kernel(Args<W> g, int 
 #pragma unroll
     for (int i = 0; i < kRegs; ++i)
       if (!__builtin_isfinite(v[i]) && m0 + tile_row(i) < g.m)
-        v[i] = fp32_element(g, m0 + tile_row(i), weight_row(tile_col(i)), s0 * WK * kSliceK, (s0 + n) * WK * kSliceK);
+        v[i] = fp32_element(g, m0 + tile_row(i), weight_row(tile_col), s0 * WK * kSliceK, (s0 + n) * WK * kSliceK);
   }
   if constexpr (kSwiGLU) {
     // Elements i and i + 1 are adjacent rows; lanes lr < 16 hold their gate
@@ -371,7 +355,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_split_kernel(Args<W> g, int 
       const int row = m0 + tile_row(i) + (lr >> 4);
       const Parts out = split_value(silu_mul(v[i], v[i + 1]));
       if (row < g.m) {
-        uint16_t *y = g.y + static_cast<size_t>(row) * g.n + (tile * (kCols / 32) + tile_col(i) / 32) * 16 + (lr & 15);
+        uint16_t *y = g.y + static_cast<size_t>(row) * g.n + (tile * (kCols / 32) + wn) * 16 + (lr & 15);
         y[0] = out.p[0];
         y[g.y_plane] = out.p[1];
         y[2 * g.y_plane] = out.p[2];
@@ -381,7 +365,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_split_kernel(Args<W> g, int 
 #pragma unroll
     for (int i = 0; i < kRegs; ++i) {
       const int row = m0 + tile_row(i);
-      if (row < g.m) g.c[(static_cast<size_t>(z) * g.m + row) * g.n + tile * kCols + tile_col(i)] = v[i];
+      if (row < g.m) g.c[(static_cast<size_t>(z) * g.m + row) * g.n + tile * kCols + tile_col] = v[i];
     }
   }
 }

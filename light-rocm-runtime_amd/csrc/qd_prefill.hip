@@ -474,14 +474,14 @@ __global__ __launch_bounds__(kBlock) void attention_merge_kernel(AttnArgs g) {
 
 // ---- GEMM launches ------------------------------------------------------------------
 
-// Tile shapes of the split GEMM, by the number of rows.
-enum Shape : int { kRows32K4 = 0, kRows32, kRows64, kRows96, kRows128 };
+// Tile shapes of the split GEMM, by the number of rows (96: gate/up only).
+enum Shape : int { kRows32K4 = 0, kRows32, kRows64, kRows128, kRows96 };
 struct ShapeInfo {
   int rows, cols, wk;
 };
-constexpr ShapeInfo kShapes[] = {{32, 32, 4}, {32, 64, 2}, {64, 128, 1}, {96, 128, 1}, {128, 128, 1}};
+constexpr ShapeInfo kShapes[] = {{32, 32, 4}, {32, 64, 2}, {64, 128, 1}, {128, 128, 1}};
 // The gate/up GEMM's 64-row shape splits k over two waves, not n.
-constexpr ShapeInfo kSwiGLUShapes[] = {{32, 32, 4}, {32, 64, 2}, {64, 64, 2}, {96, 128, 1}, {128, 128, 1}};
+constexpr ShapeInfo kSwiGLUShapes[] = {{32, 32, 4}, {32, 64, 2}, {64, 64, 2}, {128, 128, 1}, {96, 128, 1}};
 
 // Up to 32 rows the waves split k, so that 32 columns make a workgroup;
 // beyond, larger tiles reuse each staged weight for more rows as soon as there
@@ -512,7 +512,7 @@ void launch_shape(hipStream_t s, const gemm::Args<W> &g) {
   const int mtiles = (g.m + 32 * RB * WM - 1) / (32 * RB * WM);
   const int pairs = g.n / ((kSwiGLU ? 16 : 32) * WN) * g.splits;
   const int grid = (pairs + gemm::kDealXcds - 1) / gemm::kDealXcds * gemm::kDealXcds * mtiles;
-  gemm::gemm_split_kernel<RB, 1, WM, WN, WK, 2, W, kSwiGLU><<<grid, gemm::kThreads, 0, s>>>(g, mtiles, pairs);
+  gemm::gemm_split_kernel<RB, WM, WN, WK, W, kSwiGLU><<<grid, gemm::kThreads, 0, s>>>(g, mtiles, pairs);
 }
 
 template <typename W>
@@ -536,7 +536,7 @@ hipError_t launch_gemm_as(hipStream_t s, gemm::Args<W> g, bool swiglu) {
       case kRows32K4: launch_shape<1, 1, 1, 4, W, false>(s, g); break;
       case kRows32: launch_shape<1, 1, 2, 2, W, false>(s, g); break;
       case kRows64: launch_shape<2, 1, 4, 1, W, false>(s, g); break;
-      case kRows96: return hipErrorInvalidValue;  // gate/up only
+      case kRows96: break;  // not chosen
       case kRows128: launch_shape<4, 1, 4, 1, W, false>(s, g); break;
     }
   }
