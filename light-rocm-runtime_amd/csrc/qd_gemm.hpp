@@ -8,7 +8,7 @@
 // multiplication) are left out and the other six are accumulated in FP32 by
 // v_mfma_f32_32x32x16_bf16, which multiplies 16 times as fast as the FP32
 // matrix instruction: 2.7 times the FP32 rate after the factor six. The
-// leading product a0 w0 has an accumulator of its own and the five small ones
+// leading products a0 w0 have accumulators of their own and the five small ones
 // share another, so the sum over k is rounded once per 16 k's instead of once
 // per product. BF16 weights are their own first part (three products, exact)
 // and FP16 weights two parts (five products).
@@ -261,13 +261,21 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_split_kernel(Args<W> g, int 
     }
   };
 
-  // Two chains of leading products, of every other 16 k's each, halve the
-  // roundings of large sums per chain; the 128-row tile has no registers for it.
-  constexpr int kLeads = RB < 4 ? 2 : 1;
+  // Sums of many leading products are rounded at their own size, so they are
+  // kept short: where a wave multiplies all of its split's k's, their chain is
+  // added to a total every kFold slices; else (at most 14 slices to a wave) two
+  // chains take every other 16 k's each. The 128-row tile has no registers for
+  // a second accumulator (30 spilt, 13.9 ms for 1,999 rows instead of 11.2).
+  // Errors of the last of two layers' K rows against 64 bits, two chains / folded
+  // / a step per token, 1e-7, BF16: 200 rows 3.22 / 2.92 / 3.11, 512 3.44 / 3.18
+  // / 3.18, 1,000 3.92 / 3.64 / 3.58. Folding costs 0.5 % of a 512-row prompt and
+  // 1.5 % of 200 rows in F16.
+  constexpr bool kFolds = WK == 1 && RB < 4;
+  constexpr int kFold = 4, kLeads = RB < 4 ? 2 : 1;
   f16v lead[kLeads][RB] = {}, tail[RB] = {};
   if (n > 0) fetch(0);
-  int b = 0;
-  for (int s = 0; s < n; ++s) {
+  int b = 0, s = 0;
+  auto slice = [&] {
     // This wave's part of slice s has landed; after the barrier every wave's
     // has, and every wave is done with the slice before, whose stage is filled
     // next. (With the stages as b and b ^ 1 the F16 kernels are 1 % slower.)
@@ -295,12 +303,23 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_split_kernel(Args<W> g, int 
         for (int rb = 0; rb < RB; ++rb)
           acc[rb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[rb][pa], wv[pw], acc[rb], 0, 0, 0);
       };
-      mac(lead[j % kLeads], 0, 0);
+      mac(lead[kFolds ? 0 : j % kLeads], 0, 0);
       if constexpr (Op::kParts > 1) mac(tail, 0, 1);
       mac(tail, 1, 0);
       if constexpr (Op::kParts > 1) mac(tail, 1, 1);
       if constexpr (Op::kParts > 2) mac(tail, 0, 2);
       mac(tail, 2, 0);
+    }
+  };
+  while (s < n) {
+    const int end = kFolds ? min(n, s + kFold) : n;
+    for (; s < end; ++s) slice();
+    if constexpr (kFolds) {
+#pragma unroll
+      for (int rb = 0; rb < RB; ++rb) {
+        lead[1][rb] += lead[0][rb];
+        lead[0][rb] = f16v{};
+      }
     }
   }
 
