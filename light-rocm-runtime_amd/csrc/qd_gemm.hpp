@@ -262,17 +262,20 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_split_kernel(Args<W> g, int 
   };
 
   // Sums of many leading products are rounded at their own size, so they are
-  // kept short: where a wave multiplies all of its split's k's, their chain is
-  // added to a total every kFold slices; else (at most 14 slices to a wave) two
-  // chains take every other 16 k's each. The 128-row tile has no registers for
-  // a second accumulator (30 spilt, 13.9 ms for 1,999 rows instead of 11.2).
-  // Errors of the last of two layers' K rows against 64 bits, two chains / folded
-  // / a step per token, 1e-7, BF16: 200 rows 3.22 / 2.92 / 3.11, 512 3.44 / 3.18
-  // / 3.18, 1,000 3.92 / 3.64 / 3.58. Folding costs 0.5 % of a 512-row prompt and
-  // 1.5 % of 200 rows in F16.
-  constexpr bool kFolds = WK == 1 && RB < 4;
-  constexpr int kFold = 4, kLeads = RB < 4 ? 2 : 1;
-  f16v lead[kLeads][RB] = {}, tail[RB] = {};
+  // kept short: where a wave multiplies all of its split's k's, their chain
+  // (lead[0]) is added to a total (lead[1]) every kFold slices; else, at most 14
+  // slices to a wave, two chains take every other 16 k's each.
+  // Errors of the last of two layers' K rows against 64 bits, two chains (beyond
+  // 1,024 rows one) / folded / a step per token, 1e-7, BF16: 200 rows 3.22 / 2.92
+  // / 3.11, 512 3.44 / 3.18 / 3.18, 1,000 3.92 / 3.64 / 3.58; the logits of 1,999
+  // rows 12.6 / 8.5 / 7.1. It costs 0.5 % of a 512-row prompt, 1.5 % of 200 rows
+  // in F16 and 1.6 % of 1,999 rows (folding every 4 slices there: 2.2 %, 8.4).
+  // The 128-row tile has registers for the total only if it holds the operands
+  // of kAtOnce blocks of rows at a time (all four: 30 spilt, 13.9 ms for 1,999
+  // rows instead of 11.3).
+  constexpr bool kFolds = WK == 1;
+  constexpr int kFold = RB < 4 ? 4 : 8, kAtOnce = RB < 4 ? RB : 1;
+  f16v lead[2][RB] = {}, tail[RB] = {};
   if (n > 0) fetch(0);
   int b = 0, s = 0;
   auto slice = [&] {
@@ -286,29 +289,33 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_split_kernel(Args<W> g, int 
     b = b + 1 == kStages ? 0 : b + 1;
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
-      bf8v av[RB][3], wv[Op::kParts];
-#pragma unroll
-      for (int rb = 0; rb < RB; ++rb) {
-        const int row = 32 * (wm * RB + rb) + lr;
-        const int slot = (2 * j + half) ^ narrow_swizzle(row);
-#pragma unroll
-        for (int p = 0; p < 3; ++p)
-          av[rb][p] = *reinterpret_cast<const bf8v *>(st + (wk * 3 + p) * kPlane + row * kSliceK * 2 + 16 * slot);
-      }
+      bf8v wv[Op::kParts];
       const int c = 32 * wn + lr;
       Op::operand(reinterpret_cast<const u4v *>(st + kABytes + (wk * kCols + c) * kWRow), Op::swizzle(c), 2 * j + half,
                   wv);
-      auto mac = [&](f16v (&acc)[RB], int pa, int pw) {
 #pragma unroll
-        for (int rb = 0; rb < RB; ++rb)
-          acc[rb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[rb][pa], wv[pw], acc[rb], 0, 0, 0);
-      };
-      mac(lead[kFolds ? 0 : j % kLeads], 0, 0);
-      if constexpr (Op::kParts > 1) mac(tail, 0, 1);
-      mac(tail, 1, 0);
-      if constexpr (Op::kParts > 1) mac(tail, 1, 1);
-      if constexpr (Op::kParts > 2) mac(tail, 0, 2);
-      mac(tail, 2, 0);
+      for (int r0 = 0; r0 < RB; r0 += kAtOnce) {
+        bf8v av[kAtOnce][3];
+#pragma unroll
+        for (int r = 0; r < kAtOnce; ++r) {
+          const int row = 32 * (wm * RB + r0 + r) + lr;
+          const int slot = (2 * j + half) ^ narrow_swizzle(row);
+#pragma unroll
+          for (int p = 0; p < 3; ++p)
+            av[r][p] = *reinterpret_cast<const bf8v *>(st + (wk * 3 + p) * kPlane + row * kSliceK * 2 + 16 * slot);
+        }
+        auto mac = [&](f16v (&acc)[RB], int pa, int pw) {
+#pragma unroll
+          for (int r = 0; r < kAtOnce; ++r)
+            acc[r0 + r] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[r][pa], wv[pw], acc[r0 + r], 0, 0, 0);
+        };
+        mac(lead[kFolds ? 0 : j], 0, 0);
+        if constexpr (Op::kParts > 1) mac(tail, 0, 1);
+        mac(tail, 1, 0);
+        if constexpr (Op::kParts > 1) mac(tail, 1, 1);
+        if constexpr (Op::kParts > 2) mac(tail, 0, 2);
+        mac(tail, 2, 0);
+      }
     }
   };
   while (s < n) {
@@ -328,9 +335,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_split_kernel(Args<W> g, int 
   constexpr int kRegs = RB * 16 / WK;
   float v[kRegs];
   auto sum = [&](int i) {
-    float s = lead[0][i / 16][i % 16];
-    if constexpr (kLeads == 2) s += lead[1][i / 16][i % 16];
-    return s + tail[i / 16][i % 16];
+    return (lead[0][i / 16][i % 16] + lead[1][i / 16][i % 16]) + tail[i / 16][i % 16];
   };
   if constexpr (WK == 1) {
 #pragma unroll

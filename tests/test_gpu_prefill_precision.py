@@ -1,6 +1,6 @@
-"""The prompt path is no further from 64-bit arithmetic than a step per token:
+"""The prompt path is as near to 64-bit arithmetic as a step per token:
 K and V rows of the last of two layers (through everything of the first) for
-prompts in each tile shape of the GEMMs up to 1,024 rows, per storage type."""
+prompts in each tile shape of the GEMMs, per storage type."""
 import numpy as np
 import pytest
 
@@ -9,7 +9,7 @@ import qwen_oracle as qo
 
 pytestmark = pytest.mark.gpu
 
-LAYERS, VOCAB, ROWS, THETA, EPS = 2, 1024, 1000, 1e6, 1e-6
+LAYERS, VOCAB, ROWS, THETA, EPS = 2, 1024, 1100, 1e6, 1e-6
 H, HEADS, KV, D, I = 896, 14, 2, 64, 4864
 SIZES = [H, H, H * H, KV * D * H, KV * D * H, H, KV * D, KV * D, H * H, I * H, I * H, H * I]
 
@@ -68,7 +68,7 @@ def error(got, want, rows):
     return [float(np.linalg.norm(g[:rows] - w[:rows]) / np.linalg.norm(w[:rows])) for g, w in zip(got, want)]
 
 
-@pytest.mark.parametrize("rows", [20, 60, 128, 200, 300, 512, 640, 1000])
+@pytest.mark.parametrize("rows", [20, 60, 128, 200, 300, 512, 640, 1000, 1100])
 def test_prompt_is_as_exact_as_steps(setup, rows):
     eng, tokens, want, steps = setup
     eng.kv_reset(0, 0)
@@ -79,5 +79,9 @@ def test_prompt_is_as_exact_as_steps(setup, rows):
     assert max(ref) < 1e-6  # the reference is the engine's model
     # Two orders of the same sums: the steps' own error moves by 1 to 2 per cent
     # from one storage type to the next, and beyond 512 rows the attention of the
-    # prompt sums over more keys than a chunk of a step's.
-    assert all(g <= (1.03 if rows <= 512 else 1.05) * r for g, r in zip(got, ref))
+    # prompt sums over more keys than a chunk of a step's. The 128-row tile adds
+    # its chains to the total half as often: by the random walk of the roundings
+    # sqrt((56 / 2 * 16 + 56^2 / 32) / (56 / 2 * 8 + 56^2 / 16)) = 1.14 times the
+    # shorter chain's error in the gate and up products (one chain: 1.9 times).
+    bound = 1.03 if rows <= 512 else 1.05 if rows <= 1024 else 1.12
+    assert all(g <= bound * r for g, r in zip(got, ref))
