@@ -569,9 +569,9 @@ struct qd_engine {
   };
   static const char *prefill_kernel_name(int id) {
     static const char *const names[kPrefillKernels] = {
-        "embed_norm_kernel",    "gemm_nt_kernel:qkv+rope",
-        "attention_prefill_kernel", "gemm_nt_kernel:o+norm",
-        "gemm_nt_kernel:gateup+swiglu", "gemm_nt_kernel:down+norm",
+        "embed_norm_kernel",    "gemm_split_kernel:qkv+rope",
+        "attention_prefill_kernel", "gemm_split_kernel:o+norm",
+        "gemm_split_kernel:gateup+swiglu", "gemm_split_kernel:down+norm",
         "lmhead_kernel+argmax"};
     return id >= 0 && id < kPrefillKernels ? names[id] : "unknown";
   }

@@ -1,8 +1,8 @@
 // Prompt (prefill) kernels for gfx950: the prompt's positions go through a
 // layer together, so its projections are dense FP32 GEMMs on the BF16 matrix
 // cores (operands split exactly into BF16 parts, qd_gemm.hpp) and its
-// attention a causal flash attention (v_mfma_f32_16x16x4f32), instead of one
-// decode step per position.
+// attention a causal flash attention on the same split
+// (v_mfma_f32_16x16x32_bf16), instead of one decode step per position.
 //
 // Semantics follow the decode step per position (the reference's prompt
 // stack, benchmarks/triton_mini_decoder_layer.cpp:811-849, is P sequential
@@ -245,8 +245,9 @@ __global__ __launch_bounds__(kAttnThreads, 4) void attention_prefill_kernel(Attn
   const int lr = lane & 15, lg = lane >> 4;
   const int row = min(r0 + lr, g.rows - 1), pos = g.pos0 + row;
 
-  // The block's K and V^T items of this thread, loaded one block ahead: item
-  // i < 1024 is float4 i % 16 of key i / 16; 1024 + i is keys 4 (i / 64) .. + 3
+  // The block's K and V^T items of this thread (a block's are loaded when the
+  // one before is done: the other workgroup of the CU fills the wait): item i <
+  // 1024 is float4 i % 16 of key i / 16; 1024 + i is keys 4 (i / 64) .. + 3
   // of dim i % 64. Keys past the causal extent are zeros.
   constexpr int kItems = 2 * kKeyBlock * kHeadDim / 4, kPer = (kItems + kAttnThreads - 1) / kAttnThreads;
   float4 item[kPer];

@@ -1,4 +1,6 @@
-"""The prompt path's GEMMs next to the vendor FP32 GEMM at the same shapes.
+"""The prompt path's GEMMs next to the vendor FP32 GEMM at the same shapes, and
+the vendor BF16 GEMM at a large one: a sixth of its rate is what the prompt
+GEMMs' six BF16 products per FP32 one could reach.
 
 Times `A . W^T` in FP32 through torch (hipBLASLt / rocBLAS, TF32 off) for the
 four projection shapes of a 512-token prompt, and the engine's own prompt
@@ -23,18 +25,21 @@ import qwen_decode as qd  # noqa: E402
 
 ROWS = 512
 # (engine kernel name, n, k): the projections of one layer of the prompt path.
-SHAPES = (("gemm_nt_kernel:gateup+swiglu", 2 * 4864, 896),
-          ("gemm_nt_kernel:down+norm", 896, 4864),
-          ("gemm_nt_kernel:qkv+rope", 1152, 896),
-          ("gemm_nt_kernel:o+norm", 896, 896))
+SHAPES = (("gemm_split_kernel:gateup+swiglu", 2 * 4864, 896),
+          ("gemm_split_kernel:down+norm", 896, 4864),
+          ("gemm_split_kernel:qkv+rope", 1152, 896),
+          ("gemm_split_kernel:o+norm", 896, 896))
 
 
-def vendor_us(m: int, n: int, k: int, reps: int = 20) -> float:
+LARGE = 8192
+
+
+def vendor_us(m: int, n: int, k: int, dtype: str = "float32", reps: int = 20) -> float:
     import torch
 
     torch.backends.cuda.matmul.allow_tf32 = False
-    a = torch.randn(m, k, device="cuda")
-    w = torch.randn(n, k, device="cuda")
+    a = torch.randn(m, k, device="cuda").to(getattr(torch, dtype))
+    w = torch.randn(n, k, device="cuda").to(getattr(torch, dtype))
     for _ in range(3):
         a @ w.t()
     torch.cuda.synchronize()
@@ -49,7 +54,7 @@ def vendor_us(m: int, n: int, k: int, reps: int = 20) -> float:
 
 def main() -> int:
     if len(sys.argv) > 1 and sys.argv[1] == "--vendor":
-        print(json.dumps([vendor_us(ROWS, n, k) for _, n, k in SHAPES]))
+        print(json.dumps([vendor_us(ROWS, n, k) for _, n, k in SHAPES] + [vendor_us(LARGE, LARGE, LARGE, "bfloat16")]))
         return 0
     child = subprocess.run([sys.executable, os.path.abspath(__file__), "--vendor"], check=True,
                            capture_output=True, text=True)
@@ -70,6 +75,8 @@ def main() -> int:
         ours = prof[name][1]
         print(f"{name:34s} {f'{ROWS} x {n} x {k}':>20s} {ours:10.1f} {flops / ours / 1e6:8.1f} "
               f"{lib:10.1f} {flops / lib / 1e6:8.1f}")
+    rate = 2.0 * LARGE ** 3 / vendor[-1] / 1e6
+    print(f"vendor BF16 GEMM {LARGE} x {LARGE} x {LARGE}: {rate:.0f} TFLOP/s; a sixth {rate / 6:.0f}")
     return 0
 
 
