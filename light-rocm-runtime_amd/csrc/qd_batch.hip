@@ -13,9 +13,11 @@
 // the operand rows in LDS and streams the vocabulary past them.
 //
 // What bounds a step (16 rows): the weights' 1.98 GB would stream in about
-// 280 us; a layer's five kernels take 8.0 (QKV), 16.8 (attention, contexts to
-// 2,048), 7.4 (O), 12.8 (gate/up) and 10 us (down), of which each kernel's
+// 280 us; a layer's five kernels take 5.1 (QKV), 12.7 (attention, contexts to
+// 2,048), 4.7 (O), 10.3 (gate/up) and 7.3 us (down), of which each kernel's
 // start, first load and split-K hand-over are most of the three small ones.
+// (Kernel trace. The before-and-after figures below are HIP-event spans of
+// qd_profile_batch, which hold the gap between two launches too, 2 to 3 us.)
 //
 // Semantics per sequence are those of the batch-1 step (qd_kernels.hip):
 //   RMSNorm                 benchmarks/qwen_stateful_graph_kernel.cpp:665-701

@@ -494,11 +494,18 @@ constexpr ShapeInfo kSwiGLUShapes[] = {{32, 32, 4}, {32, 64, 2}, {64, 64, 2}, {1
 // Gate/up from 193 to 864 rows: 96 x 128 tiles do less per product outside
 // the matrix cores, but are few, and a round of 256 that they hardly begin
 // costs as much as a full one; so they are taken where they fill more than two
-// fifths of their last round. us with 64 / 96 rows, FP32 (F16): m = 200
-// 42.6 / 40.7 (37.8 / 33.4), 288 46.5 / 41.8 (39.2 / 36.5), 512 66.8 / 65.8
-// (59.1 / 55.4), 860 110.8 / 99.7 (95.9 / 79.6); and where not taken, 300
-// 45.1 / 56.8 (40.6 / 48.9), 640 75.4 / 94.3 (65.0 / 73.0), 960 113.6 / 118.4
-// (97.0 / 101.3).
+// fifths of their last round. us with 64 / 96 rows (event spans), FP32, F16, BF16:
+//   m = 200  43.4 / 40.0    37.6 / 35.2    34.6 / 31.1
+//       288  47.3 / 41.8    39.6 / 36.5    36.7 / 32.9
+//       512  67.4 / 65.0    59.1 / 56.1    60.4 / 42.9
+//       860 110.9 / 99.1    96.5 / 84.9    85.7 / 69.3
+// and where not taken
+//       300  47.2 / 56.7    40.1 / 49.9    38.0 / 38.2
+//       640  78.3 / 95.2    67.4 / 81.5    59.4 / 64.8
+//       960 113.5 / 117.2   97.9 / 101.7   90.3 / 75.7
+//     1,024 123.9 / 120.4  106.7 / 103.7  104.0 / 78.2
+// One rule for the three types: the order of a sum must not depend on the type
+// (a BF16 or F16 engine equals an FP32 one with the rounded weights).
 Shape gemm_shape(int m, int n, bool swiglu) {
   if (m <= 32) return kRows32K4;
   if (m <= (swiglu ? 64 : 128)) return kRows32;
