@@ -837,6 +837,11 @@ struct qd_engine {
       resident_status(err);
     }
   }
+  // Before a call that moves a slot on: an earlier layers-only launch that
+  // failed fails this call while nothing has moved.
+  void settle_layers() {
+    if (layers_pending) sync();
+  }
   // Runs fn, which advances slot seq past decoder layers whose errors surface
   // when it waits. If it fails, the slot is where it was: its position, and its
   // device state if fn has called keep_state.
@@ -1634,6 +1639,7 @@ qd_status step_common(qd_engine *e, uint32_t seq, uint32_t token, float *logits_
     if (e->positions[seq] >= e->CAP)
       fail(QD_ERROR_INVALID_ARGUMENT, "sequence %u is full (capacity %zu)", seq, e->CAP);
     e->set_device();
+    e->settle_layers();
     float *dev_logits = e->logits + seq * e->V;
     // qd_step runs the resident kernel for one token when the engine has it
     // (one cooperative launch instead of the stream kernels' ~150); the graph
@@ -1838,6 +1844,7 @@ void check_batch(qd_engine *e, uint32_t n_seq, const uint32_t *seq_ids, const ui
       fail(QD_ERROR_INVALID_ARGUMENT, "sequence %u is full", seq_ids[i]);
   }
   e->set_device();
+  e->settle_layers();
 }
 
 // Enqueues one batched step of the listed slots (groups of kBatchRows) and
@@ -1918,6 +1925,7 @@ qd_status qd_step_batch_noalloc(qd_engine *e, uint32_t n_seq, const uint32_t *se
     if (!e->batch_scratch)
       fail(QD_ERROR_NOT_SUPPORTED, "static batch workspace unavailable: %s", e->batch_scratch_error.c_str());
     e->set_device();
+    e->settle_layers();
     // One step at a time per GPU on the shared workspace.
     std::lock_guard<std::mutex> lock(qd::batch_scratch_lock(e->cfg.device));
     // Every buffer but the step's inputs and outputs (weights, KV cache,
@@ -1987,6 +1995,7 @@ qd_status qd_generate_resident(qd_engine *e, uint32_t seq, uint32_t first_token,
       fail(QD_ERROR_INVALID_ARGUMENT, "generation of %u tokens from position %u overflows capacity %zu",
            max_tokens, e->positions[seq], e->CAP);
     e->set_device();
+    e->settle_layers();
     float *hist = e->logits + size_t(seq) * e->V;
     int use_hist = 0;
     if (all_logits) {
@@ -2062,6 +2071,7 @@ qd_status qd_profile_kernels(qd_engine *e, uint32_t seq, uint32_t first_token, u
     if (size_t(e->positions[seq]) + tokens > e->CAP)
       fail(QD_ERROR_INVALID_ARGUMENT, "profiling %u tokens overflows capacity", tokens);
     e->set_device();
+    e->settle_layers();
     EventMarker marker(e);
     marker.cost = [&](int k) {
       return std::pair<double, double>{e->kernel_bytes(k, marker.ctx_a), e->kernel_flops(k, marker.ctx_a)};
@@ -2133,6 +2143,7 @@ void profiled_resident_launch(qd_engine *e, uint32_t seq, uint32_t first_token, 
   if (!e->resident_plan(e->positions[seq], tokens, &plan))
     fail(QD_ERROR_NOT_SUPPORTED, "no resident role plan reaches context %zu", size_t(e->positions[seq]) + tokens);
   e->set_device();
+  e->settle_layers();
   const size_t trace_elems =
       trace_out ? size_t(e->roles_grid) * (e->L + 1) * qd::kResidentStages : 0;
   // Temporary buffers of a diagnostic call, released before returning.

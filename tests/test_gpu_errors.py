@@ -112,6 +112,33 @@ def test_failed_layers_leave_the_slot_where_it_was(monkeypatch, call):
         ref.close()
 
 
+@pytest.mark.parametrize("call", ["step_graph", "step_batch", "step_batch_noalloc"])
+def test_failed_layers_of_another_slot_leave_the_slot_where_it_was(monkeypatch, call):
+    say(f"layers-only launch of slot 1 gives up, {call} of slot 0 reports it")
+    config = dict(SMALL, layers=6, max_batch=2)
+    monkeypatch.setenv("QD_RESIDENT_SPIN_LIMIT", "1")
+    eng = qd.Engine(**config)
+    monkeypatch.delenv("QD_RESIDENT_SPIN_LIMIT")
+    try:
+        eng.load_synthetic(5)
+        eng.prefill(0, qo.fill_tokens(5, 5, 0x300000, SMALL["vocab"]), want_logits=False)
+        before = state_of(eng)
+        assert before["token_position"] == 5
+        eng.embed_hidden(1, 3)
+        eng.layer_decode(1, 0, 6, 1)
+        with pytest.raises(qd.QdError) as err:
+            if call.startswith("step_batch"):
+                getattr(eng, call)([0], [7])
+            else:
+                eng.step_graph(0, 7)
+        assert err.value.status == qd.DEVICE_FAULT
+        assert state_of(eng) == before
+        eng.step_graph(0, 7)  # the error was that launch's, and has been reported
+        assert eng.decode_state(0).token_position == 6
+    finally:
+        eng.close()
+
+
 def test_prompt_without_room_for_its_workspace(monkeypatch):
     say("prompt workspace allocations refused by QD_DEVICE_BYTES_LIMIT")
     config = dict(SMALL, capacity=700)
