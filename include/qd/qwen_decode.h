@@ -233,10 +233,11 @@ QD_API qd_status qd_embed_hidden(qd_engine *engine, uint32_t seq,
  * slot's position to valid_keys - 1 (the token in flight; qd_tail
  * completes it). From three layers on (BF16: four below 64 positions) they run
  * as one launch of the resident kernel when the engine has it, else as the
- * stream-ordered kernels; the two compute the same values bit for bit. Asynchronous: errors surface at the next synchronising
- * call. Replaces DecoderLayer::decode_to_hidden_state / decode_to_buffer
- * (examples/triton/mini_decoder_layer.hpp:345-372), whose valid_keys it
- * takes. */
+ * stream-ordered kernels; the two compute the same values bit for bit.
+ * Asynchronous: errors surface at the next synchronising call, which leaves
+ * its slots where they were. Replaces DecoderLayer::decode_to_hidden_state /
+ * decode_to_buffer (examples/triton/mini_decoder_layer.hpp:345-372), whose
+ * valid_keys it takes. */
 QD_API qd_status qd_layer_decode(qd_engine *engine, uint32_t seq,
                                  uint32_t first_layer, uint32_t layer_count,
                                  uint32_t valid_keys);

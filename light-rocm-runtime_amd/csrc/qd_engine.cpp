@@ -1445,6 +1445,7 @@ qd_status qd_kv_reset(qd_engine *e, uint32_t seq, uint32_t position) {
     e->check_seq(seq);
     if (position > e->CAP) fail(QD_ERROR_INVALID_ARGUMENT, "position %u beyond capacity %zu", position, e->CAP);
     e->set_device();
+    e->settle_layers();
     e->positions[seq] = position;
     e->push_state(seq, 0, qd::kModeStep, UINT32_MAX, 0);
     e->sync();

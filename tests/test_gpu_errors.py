@@ -112,7 +112,7 @@ def test_failed_layers_leave_the_slot_where_it_was(monkeypatch, call):
         ref.close()
 
 
-@pytest.mark.parametrize("call", ["step_graph", "step_batch", "step_batch_noalloc"])
+@pytest.mark.parametrize("call", ["step_graph", "step_batch", "step_batch_noalloc", "kv_reset"])
 def test_failed_layers_of_another_slot_leave_the_slot_where_it_was(monkeypatch, call):
     say(f"layers-only launch of slot 1 gives up, {call} of slot 0 reports it")
     config = dict(SMALL, layers=6, max_batch=2)
@@ -129,6 +129,8 @@ def test_failed_layers_of_another_slot_leave_the_slot_where_it_was(monkeypatch, 
         with pytest.raises(qd.QdError) as err:
             if call.startswith("step_batch"):
                 getattr(eng, call)([0], [7])
+            elif call == "kv_reset":
+                eng.kv_reset(0, 3)
             else:
                 eng.step_graph(0, 7)
         assert err.value.status == qd.DEVICE_FAULT
