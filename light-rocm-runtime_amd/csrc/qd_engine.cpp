@@ -191,10 +191,10 @@ struct qd_engine {
   PromptWorkspace pf{};
   // Batched-step workspace (allocated on the first batched step): rows of
   // up to kBatchRows sequences, attention and split-K partials, arrival
-  // counters, the LM-head top-1 partials and each row's greedy result.
-  float *bt_h = nullptr, *bt_hg = nullptr, *bt_sq = nullptr, *bt_q = nullptr, *bt_attn = nullptr, *bt_act = nullptr,
-        *bt_part = nullptr, *bt_split = nullptr, *bt_val = nullptr, *bt_top = nullptr;
-  uint32_t *bt_idx = nullptr, *bt_counters = nullptr, *bt_token = nullptr;
+  // counters, the LM-head top-1 partials and each row's greedy result (the
+  // last two regions hold max_batch rows). One allocation, there as a whole or
+  // not at all.
+  qd::BatchWorkspace bt{};
   uint32_t *h_bt_out = nullptr;  // pinned [max_batch] tokens then [max_batch] top logits
   // The library's static batch workspace on this engine's device
   // (qd_step_batch_noalloc), looked up at creation; null if the lookup failed.
@@ -448,30 +448,25 @@ struct qd_engine {
     return 0;
   }
 
-  // Arguments of one batched launch over rows sequences: slot ids, tokens
-  // and (host-tracked) positions of batch rows first .. first + rows - 1.
-  qd::BatchLaunch batch_args(const uint32_t *slots, const uint32_t *tokens, int rows) {
-    if (!bt_h) {
-      const size_t r = qd::kBatchRows;
-      bt_hg = alloc<float>(r * H);
-      bt_sq = alloc<float>(r * qd::kBatchTiles);
-      bt_q = alloc<float>(r * QD);
-      bt_attn = alloc<float>(r * QD);
-      bt_act = alloc<float>(r * I);
-      bt_part = alloc<float>(r * NQ * qd::kAttnMaxChunks * qd::kPartStride);
-      bt_split = alloc<float>(qd::kBatchSplitFloats);
-      bt_counters = alloc<uint32_t>(qd::kBatchCounters);
-      bt_val = alloc<float>(r * qd::kBatchLmParts);
-      bt_idx = alloc<uint32_t>(r * qd::kBatchLmParts);
-      bt_token = alloc<uint32_t>(B);
-      bt_top = alloc<float>(B);
-      check(hipMemsetAsync(bt_sq, 0, r * qd::kBatchTiles * sizeof(float), stream), "memset");
-      check(hipMemsetAsync(bt_counters, 0, qd::kBatchCounters * sizeof(uint32_t), stream), "memset");
-      check(hipHostMalloc(reinterpret_cast<void **>(&h_bt_out), 2 * B * sizeof(uint32_t),
-                          hipHostMallocDefault),
+  void batch_workspace() {
+    if (bt.hidden) return;
+    if (!h_bt_out)
+      check(hipHostMalloc(reinterpret_cast<void **>(&h_bt_out), 2 * B * sizeof(uint32_t), hipHostMallocDefault),
             "hipHostMalloc");
-      bt_h = alloc<float>(r * H);
-    }
+    const size_t bytes = qd::batch_workspace_bytes(int(NQ));
+    char *block = alloc<char>(bytes + 2 * B * sizeof(uint32_t));
+    qd::BatchWorkspace w = qd::carve_batch_workspace(block, int(NQ));
+    w.out_token = reinterpret_cast<uint32_t *>(block + bytes);
+    w.out_top = reinterpret_cast<float *>(block + bytes) + B;
+    check(hipMemsetAsync(w.squares, 0, qd::kBatchRows * qd::kBatchTiles * sizeof(float), stream), "memset");
+    check(hipMemsetAsync(w.counters, 0, qd::kBatchCounters * sizeof(uint32_t), stream), "memset");
+    bt = w;
+  }
+
+  // Arguments of one batched launch over rows sequences: slot ids, tokens
+  // and (host-tracked) positions of the batch rows.
+  qd::BatchLaunch batch_args(const qd::BatchWorkspace &w, const uint32_t *slots, const uint32_t *tokens,
+                             int rows) const {
     qd::BatchLaunch b{};
     b.rows = rows;
     for (int i = 0; i < rows; ++i) {
@@ -480,15 +475,15 @@ struct qd_engine {
       b.token[i] = tokens[i];
     }
     b.states = states;
-    b.hidden = bt_h;
-    b.gained = bt_hg;
-    b.squares = bt_sq;
-    b.q = bt_q;
-    b.attn = bt_attn;
-    b.act = bt_act;
-    b.part = bt_part;
-    b.split = bt_split;
-    b.counters = bt_counters;
+    b.hidden = w.hidden;
+    b.gained = w.gained;
+    b.squares = w.squares;
+    b.q = w.q;
+    b.attn = w.attn;
+    b.act = w.act;
+    b.part = w.part;
+    b.split = w.split;
+    b.counters = w.counters;
     b.k_cache = k_cache;
     b.v_cache = v_cache;
     b.rope_cos = rope_cos;
@@ -503,24 +498,21 @@ struct qd_engine {
 
   // Tail arguments of the group whose first batch row is `first`: each
   // row's logits go to its slot's row of the logits buffer (where
-  // qd_read_logits finds them), greedy results to bt_token/bt_top.
-  qd::BatchTail batch_tail(size_t first) const {
+  // qd_read_logits finds them), greedy results to w's out_token / out_top.
+  qd::BatchTail batch_tail(const qd::BatchWorkspace &w, size_t first) const {
     qd::BatchTail t{};
     t.head = lm_head;
     t.logits = logits;
-    t.part_val = bt_val;
-    t.part_idx = bt_idx;
-    t.out_token = bt_token + first;
-    t.out_top = bt_top + first;
+    t.part_val = w.part_val;
+    t.part_idx = w.part_idx;
+    t.out_token = w.out_token + first;
+    t.out_top = w.out_top + first;
     t.vocab = static_cast<int>(V);
     return t;
   }
 
   // Embedding + every layer + LM head + argmax of one batch group (states
   // and slot list already on the device).
-  void enqueue_batch(const qd::BatchLaunch &b, size_t first, qd::Marker *m = nullptr) {
-    enqueue_batch(b, batch_tail(first), m);
-  }
   void enqueue_batch(const qd::BatchLaunch &b, const qd::BatchTail &t, qd::Marker *m = nullptr) {
     check(qd::launch_batch_embed(stream, b, embed, layers[0].attn_norm, static_cast<int>(V), m),
           "batch embed launch");
@@ -1849,19 +1841,20 @@ void check_batch(qd_engine *e, uint32_t n_seq, const uint32_t *seq_ids, const ui
 }
 
 // Enqueues one batched step of the listed slots (groups of kBatchRows) and
-// leaves every row's greedy token and logit in bt_token / bt_top; m
+// leaves every row's greedy token and logit in bt.out_token / bt.out_top; m
 // (nullable) times every launch.
 void enqueue_step_batch(qd_engine *e, uint32_t n_seq, const uint32_t *seq_ids, const uint32_t *tokens,
                         EventMarker *m) {
+  e->batch_workspace();
   for (uint32_t first = 0; first < n_seq; first += qd::kBatchRows) {
     const int rows = static_cast<int>(std::min<uint32_t>(qd::kBatchRows, n_seq - first));
-    const qd::BatchLaunch b = e->batch_args(seq_ids + first, tokens + first, rows);
+    const qd::BatchLaunch b = e->batch_args(e->bt, seq_ids + first, tokens + first, rows);
     if (m) {
       m->ctx_a = rows;
       m->ctx_b = 0;
       for (int i = 0; i < rows; ++i) m->ctx_b += b.pos[i] + 1.0;
     }
-    e->enqueue_batch(b, first, m);
+    e->enqueue_batch(b, e->batch_tail(e->bt, first), m);
   }
 }
 
@@ -1892,8 +1885,8 @@ qd_status qd_step_batch(qd_engine *e, uint32_t n_seq, const uint32_t *seq_ids, c
     // kernels take each row's slot, token and position as arguments and
     // leave the slot's state as a batch-1 step would.
     enqueue_step_batch(e, n_seq, seq_ids, tokens, nullptr);
-    check(hipMemcpyAsync(e->h_bt_out, e->bt_token, n_seq * 4, hipMemcpyDeviceToHost, e->stream), "D2H");
-    check(hipMemcpyAsync(e->h_bt_out + e->B, e->bt_top, n_seq * 4, hipMemcpyDeviceToHost, e->stream),
+    check(hipMemcpyAsync(e->h_bt_out, e->bt.out_token, n_seq * 4, hipMemcpyDeviceToHost, e->stream), "D2H");
+    check(hipMemcpyAsync(e->h_bt_out + e->B, e->bt.out_top, n_seq * 4, hipMemcpyDeviceToHost, e->stream),
           "D2H");
     if (logits) e->read_rows(e->logits, seq_ids, n_seq, logits);
     e->sync();
@@ -1932,45 +1925,11 @@ qd_status qd_step_batch_noalloc(qd_engine *e, uint32_t n_seq, const uint32_t *se
     // Every buffer but the step's inputs and outputs (weights, KV cache,
     // slot states, the logits rows) lives in the static workspace.
     const qd::BatchWorkspace w = qd::carve_batch_workspace(e->batch_scratch, int(e->NQ));
-    qd::BatchLaunch b{};
-    b.rows = static_cast<int>(n_seq);
-    for (uint32_t i = 0; i < n_seq; ++i) {
-      b.slot[i] = seq_ids[i];
-      b.pos[i] = e->positions[seq_ids[i]];
-      b.token[i] = tokens[i];
-    }
-    b.states = e->states;
-    b.hidden = w.hidden;
-    b.gained = w.gained;
-    b.squares = w.squares;
-    b.q = w.q;
-    b.attn = w.attn;
-    b.act = w.act;
-    b.part = w.part;
-    b.split = w.split;
-    b.counters = w.counters;
-    b.k_cache = e->k_cache;
-    b.v_cache = e->v_cache;
-    b.rope_cos = e->rope_cos;
-    b.rope_sin = e->rope_sin;
-    b.layers = static_cast<int>(e->L);
-    b.capacity = static_cast<int>(e->CAP);
-    b.nq = static_cast<int>(e->NQ);
-    b.nkv = static_cast<int>(e->NKV);
-    b.eps = e->cfg.rms_eps;
-    qd::BatchTail t{};
-    t.head = e->lm_head;
-    t.logits = e->logits;
-    t.part_val = w.part_val;
-    t.part_idx = w.part_idx;
-    t.out_token = w.out_token;
-    t.out_top = w.out_top;
-    t.vocab = static_cast<int>(e->V);
     // The workspace keeps the last call's contents: the arrival counters
     // start at zero (a fill kernel, no memset node). The places of `squares`
     // past the 56 tiles are never written: zero as the array was.
     check(qd::launch_batch_clear_counters(e->stream, w.counters), "counter clear");
-    e->enqueue_batch(b, t);
+    e->enqueue_batch(e->batch_args(w, seq_ids, tokens, int(n_seq)), e->batch_tail(w, 0));
     if (greedy)
       check(hipMemcpyAsync(greedy, w.out_token, n_seq * 4, hipMemcpyDeviceToHost, e->stream), "D2H");
     if (logits)
@@ -2099,7 +2058,7 @@ qd_status qd_profile_batch(qd_engine *e, uint32_t n_seq, const uint32_t *seq_ids
     std::vector<uint32_t> feed(tokens, tokens + n_seq);
     for (uint32_t step = 0; step < steps; ++step) {
       enqueue_step_batch(e, n_seq, seq_ids, feed.data(), &marker);
-      check(hipMemcpyAsync(e->h_bt_out, e->bt_token, n_seq * 4, hipMemcpyDeviceToHost, e->stream), "D2H");
+      check(hipMemcpyAsync(e->h_bt_out, e->bt.out_token, n_seq * 4, hipMemcpyDeviceToHost, e->stream), "D2H");
       e->sync();
       for (uint32_t i = 0; i < n_seq; ++i) {
         e->positions[seq_ids[i]] += 1;

@@ -5,8 +5,8 @@
   (the call returns) and the engine keeps working. The give-up is forced
   with QD_RESIDENT_SPIN_LIMIT=1 at engine creation: waits then give up after
   a few polls, long before any producer publishes.
-* A prompt whose workspace the device has no room for fails and can be tried
-  again (QD_DEVICE_BYTES_LIMIT refuses the allocation); long prompts make do
+* A prompt or a batched step whose workspace the device has no room for fails
+  and can be tried again (QD_DEVICE_BYTES_LIMIT refuses the allocation); long prompts make do
   with the workspace of a short one.
 * NaN payloads never survive a load: K/V rows written through qd_write_kv,
   hidden vectors of qd_load_hidden and qd_layer_step and weights loaded from a
@@ -189,6 +189,31 @@ def test_prompt_without_room_for_its_workspace(monkeypatch):
     finally:
         for e in engines:
             e.close()
+
+
+def test_batch_without_room_for_its_workspace(monkeypatch):
+    say("batch workspace allocation refused by QD_DEVICE_BYTES_LIMIT")
+    config = dict(SMALL, max_batch=2)
+    ref = qd.Engine(**config)
+    base = ref.device_bytes()
+    monkeypatch.setenv("QD_DEVICE_BYTES_LIMIT", str(base + (1 << 20)))
+    eng = qd.Engine(**config)
+    monkeypatch.delenv("QD_DEVICE_BYTES_LIMIT")
+    try:
+        for e in (ref, eng):
+            e.load_synthetic(5)
+        for _ in range(2):
+            with pytest.raises(qd.QdError) as err:
+                eng.step_batch([0, 1], [3, 4])
+            assert err.value.status == qd.RUNTIME and eng.device_bytes() == base  # nothing kept
+        assert [eng.decode_state(s).token_position for s in range(2)] == [0, 0]
+        got = eng.step_batch_noalloc([0, 1], [3, 4])
+        want = ref.step_batch([0, 1], [3, 4])
+        assert ref.device_bytes() > base + (1 << 20)
+        assert all(np.array_equal(a, b) for a, b in zip(got, want))
+    finally:
+        ref.close()
+        eng.close()
 
 
 def nan_bits(*patterns):
