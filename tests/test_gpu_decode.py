@@ -535,7 +535,8 @@ def test_profile_prefill_matches_prefill(full):
 
 def test_prefill_in_pieces_and_over_chunks_agree(full):
     """A prompt prefilled in two calls (the second continuing at position 300)
-    and one longer than a 512-row chunk give the one-call results."""
+    gives the results of one call, whose 700 rows need the large workspace.
+    (Prompts of more than one chunk: test_gpu_prefill_shapes.py.)"""
     eng, _ = full
     prompt = qo.fill_tokens(700, 4, PROMPT_STREAM + 5, FULL.vocab)
     say("prefill 700 at once / 300 + 400")
